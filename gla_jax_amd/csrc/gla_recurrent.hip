@@ -1,12 +1,13 @@
-// recurrent_gla forward and backward for gfx950: the per-timestep rank-1 state update
+// recurrent_gla for gfx950: entry points of the forward and backward, and the vector kernels of the backward for the
+// per-timestep rank-1 state update
 //   S_t = exp(g_t)[:,None] * S_{t-1} + k_t v_t^T ,   o_t = S_t^T q_t            (gla.py:35-37, 50-96)
-// and its two-sweep gradient (gla.py:271-360, 263).  The [DK,DV] state of one (batch, head) pair
+// with its two-sweep gradient (gla.py:271-360, 263).  The [DK,DV] state of one (batch, head) pair
 // lives in the registers of one workgroup for the whole sequence; nothing but inputs, outputs and
 // the final state touches HBM.  fp32 VALU work throughout (the state is fp32, gla.py:89).
 //
-// Register tiling: a wave owns 16 columns (forward) or 16 rows (backward) of the state; a lane owns
-// a 4-wide strip of that and 1/16 of the other dimension, so per step it needs 4 + R inputs per
-// operand, does 3*4*R FMAs and its partial sums are reduced over 16 lanes by xor-shuffles.
+// Register tiling: a wave owns 16 rows of the state; a lane owns a 4-wide strip of that and 1/16 of the
+// other dimension, so per step it needs 4 + R inputs per operand, does 3*4*R FMAs and its partial
+// sums are reduced over 16 lanes by xor-shuffles.  (The forward's vector kernel: gla_recurrent_steps.hip.)
 #include "gla_common.hpp"
 #include "gla_recurrent_stream.hpp"
 #include "gla_split.hpp"
@@ -61,94 +62,6 @@ __device__ __forceinline__ float reduce_over_c(float x)
     x += dpp_f32<kDppRowHalfMirror>(x);
     x += dpp_f32<kDppRowMirror>(x);
     return x;
-}
-
-// ------------------------------------------------------------------------------------------------
-// forward.  Block = DV/16 waves = one (b,h); wave w owns state columns [16w, 16w+16); lane (a = l>>4,
-// c = l&15) owns rows [c*RK, (c+1)*RK) x columns 16w + [4a, 4a+4).
-// ------------------------------------------------------------------------------------------------
-template <typename T, typename TO, int RK, int U>
-__global__ __launch_bounds__(RK * 64) void recurrent_fwd_kernel(
-    const void *__restrict__ h0, const float *__restrict__ g, const T *__restrict__ v,
-    const T *__restrict__ k, const T *__restrict__ q, void *__restrict__ hT, TO *__restrict__ out,
-    int T_len, int H, int reverse, int hdt)
-{
-    constexpr int DK = RK * 16, DV = DK;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int a = lane >> 4, c = lane & 15;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int dk0 = c * RK, dv0 = wave * 16 + a * 4;
-    const int64_t bh = (int64_t)b * H + h;
-
-    float S[RK][4];
-    {
-        const int64_t ho = bh * DK * DV + (int64_t)dk0 * DV + dv0;
-#pragma unroll
-        for (int i = 0; i < RK; ++i) load_hidden<4>(h0, hdt, ho + (int64_t)i * DV, S[i]);
-    }
-    const int64_t strideK = (int64_t)H * DK, strideV = (int64_t)H * DV;
-    const float *gp = g + ((int64_t)b * T_len * H + h) * DK + dk0;
-    const T *kp = k + ((int64_t)b * T_len * H + h) * DK + dk0;
-    const T *qp = q + ((int64_t)b * T_len * H + h) * DK + dk0;
-    const T *vp = v + ((int64_t)b * T_len * H + h) * DV + dv0;
-    TO *op = out + ((int64_t)b * T_len * H + h) * DV + dv0;
-
-    struct Step {
-        RawVec<float, RK> g;
-        RawVec<T, RK> k, q;
-        RawVec<T, 4> v;
-    };
-    auto load_step = [&](Step &s, int step) {
-        int t = reverse ? T_len - 1 - step : step;
-        s.g.load(gp + t * strideK);
-        s.k.load(kp + t * strideK);
-        s.q.load(qp + t * strideK);
-        s.v.load(vp + t * strideV);
-    };
-    auto compute = [&](const Step &s, int step) {
-        int t = reverse ? T_len - 1 - step : step;
-        float vv[4], o[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vv[j] = s.v.get(j);
-#pragma unroll
-        for (int i = 0; i < RK; ++i) {
-            float f = __expf(s.g.get(i)), ki = s.k.get(i), qi = s.q.get(i);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                S[i][j] = f * S[i][j] + ki * vv[j];
-                o[j] += qi * S[i][j];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = reduce_over_c(o[j]);
-        if (c == 0) store_vec<TO, 4>(op + t * strideV, o);
-    };
-
-    Step cur[U], nxt[U];
-    const int nblk = T_len / U;
-    if (nblk > 0) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) load_step(cur[u], u);
-    }
-    for (int blk = 0; blk < nblk; ++blk) {
-        if (blk + 1 < nblk) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) load_step(nxt[u], (blk + 1) * U + u);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) compute(cur[u], blk * U + u);
-#pragma unroll
-        for (int u = 0; u < U; ++u) cur[u] = nxt[u];
-    }
-    for (int step = nblk * U; step < T_len; ++step) {
-        load_step(cur[0], step);
-        compute(cur[0], step);
-    }
-    {
-        const int64_t ho = bh * DK * DV + (int64_t)dk0 * DV + dv0;
-#pragma unroll
-        for (int i = 0; i < RK; ++i) store_hidden<4>(hT, hdt, ho + (int64_t)i * DV, S[i]);
-    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -398,27 +311,14 @@ __global__ __launch_bounds__(RV * 64) void recurrent_bwd_rev_kernel(
 }
 
 // ------------------------------------------------------------------------------------------------
-template <typename T, typename TO>
-static int launch_fwd(hipStream_t st, int B, int T_len, int H, int DK, int DV, int reverse, int hdt,
-                      const void *h0, const float *g, const void *v, const void *k, const void *q,
-                      void *hT, void *out)
-{
-    dim3 grid(H, B), block(DV / 16 * 64);
-#define GLA_FWD_CASE(RK_, U_)                                                                        \
-    hipLaunchKernelGGL((recurrent_fwd_kernel<T, TO, RK_, U_>), grid, block, 0, st, h0, g,            \
-                       (const T *)v, (const T *)k, (const T *)q, hT, (TO *)out, T_len, H,            \
-                       reverse, hdt)
-    switch (DK / 16) {
-    case 1: GLA_FWD_CASE(1, 4); break;
-    case 2: GLA_FWD_CASE(2, 4); break;
-    case 4: GLA_FWD_CASE(4, 4); break;
-    case 8: GLA_FWD_CASE(8, 2); break;
-    case 16: GLA_FWD_CASE(16, 1); break;
-    default: return GLA_ERR_SHAPE;
-    }
-#undef GLA_FWD_CASE
-    return launch_status();
-}
+// bf16 data at head dimensions 64 and 128 runs on the matrix cores, 64 or 128 steps per iteration, from kFewSteps steps on:
+// an iteration takes 11 to 25 us however few its steps are (B*H = 16 to 256; four times that at 1024), the vector kernel
+// 5 us for one step and 10 to 24 us for 32 (D = 64: 9.8 against 10.8 us at B*H = 16, 11.2 / 11.6 at 256, 28 / 42 at
+// 1024; D = 128: 11.7 / 20.9, 23.8 / 25.1, 70 / 92; at 64 steps the matrix cores win, 18 / 11 and 39 / 26 us).
+constexpr int64_t kFewSteps = 32;
+// Head dimension 256 takes two passes of the 128-feature kernels and the copies around them: 60 us and more, which the vector
+// kernel needs for more than 64 steps (B*H = 16: 30 / 61 us at 64 steps, 125 / 165 at 256, 484 / 711 at 1024).
+constexpr int64_t kFewSteps256 = 64;
 
 template <typename T, typename TO>
 static int launch_bwd(hipStream_t st, int B, int T_len, int H, int DK, int DV, int reverse, int hdt,
@@ -507,23 +407,17 @@ static int recurrent_fwd_run(void *stream, int64_t B, int64_t T, int64_t H, int6
     for (const void *p : ptrs)
         if (!gla::aligned16(p)) return GLA_ERR_ALIGN;
     hipStream_t st = (hipStream_t)stream;
-    // bf16 inputs at head dimension 64 or 128 run on the matrix cores, 64 or 128 steps per iteration; fp32 `out`
-    // (the recurrent_gla_naive flavour, gla.py:37) is the same kernel storing its fp32 accumulators unrounded
-    if (dtype == GLA_BF16 && (DK == 64 || DK == 128)) {
-        if (out_dtype == GLA_F32)
-            return gla::launch_recurrent_stream_fwd<float>(st, B, T, H, DK, reverse, hidden_dtype, hidden_init,
-                                                           log_fgate, value, key, query, hidden_final, out);
-        return gla::launch_recurrent_stream_fwd<__bf16>(st, B, T, H, DK, reverse, hidden_dtype, hidden_init,
-                                                        log_fgate, value, key, query, hidden_final, out);
+    // fp32 `out` beside bf16 data (the recurrent_gla_naive flavour, gla.py:37) is the same kernels storing their fp32 sums
+    // unrounded
+    const bool out_f32 = dtype == GLA_BF16 && out_dtype == GLA_F32;
+    if (dtype == GLA_BF16 && (DK == 64 || DK == 128) && T > gla::kFewSteps) {
+        auto run = out_f32 ? gla::launch_recurrent_stream_fwd<float> : gla::launch_recurrent_stream_fwd<__bf16>;
+        return run(st, B, T, H, DK, reverse, hidden_dtype, hidden_init, log_fgate, value, key, query, hidden_final, out);
     }
-    if (dtype == GLA_BF16 && out_dtype == GLA_BF16)
-        return gla::launch_fwd<__bf16, __bf16>(st, B, T, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value,
-                                               key, query, hidden_final, out);
-    if (dtype == GLA_BF16)
-        return gla::launch_fwd<__bf16, float>(st, B, T, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value,
-                                              key, query, hidden_final, out);
-    return gla::launch_fwd<float, float>(st, B, T, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value, key,
-                                         query, hidden_final, out);
+    auto run = dtype == GLA_F32 ? gla::launch_recurrent_steps<float, float>
+               : out_f32        ? gla::launch_recurrent_steps<__bf16, float>
+                                : gla::launch_recurrent_steps<__bf16, __bf16>;
+    return run(st, B, T, H, DK, reverse, hidden_dtype, hidden_init, log_fgate, value, key, query, hidden_final, out);
 }
 
 extern "C" int gla_recurrent_fwd(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
@@ -593,7 +487,7 @@ struct TimeSplit {
 };
 static size_t inner_fwd_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
 {
-    return DK == 256 ? SplitSizes(B, T, H, dtype).fwd() : 0;
+    return DK == 256 && dtype == GLA_BF16 ? SplitSizes(B, T, H, dtype).fwd() : 0;   // fp32 data needs no passes
 }
 static size_t inner_bwd_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
 {
@@ -605,6 +499,7 @@ extern "C" size_t gla_recurrent_fwd_workspace_bytes(int64_t B, int64_t T, int64_
                                                     gla_dtype dtype)
 {
     if (gla::check_recurrent(B, T, H, DK, DV, dtype, GLA_F32, GLA_F32) || 2 * H > 65535) return 0;
+    if (DK == 256 && T <= gla::kFewSteps256) return 0;
     const gla::TimeSplit ts(B, T, H, DK, dtype);      // the passes run on B*S batch entries of L steps: their state blocks count
     return ts.fwd() + gla::inner_fwd_bytes(B * ts.S * ts.F, ts.Lf, H, DK, dtype);
 }
@@ -635,7 +530,7 @@ static int recurrent_fwd_inner(void *stream, int64_t B, int64_t T, int64_t H, in
     if (lean && (DK == 64 || DK == 128))
         return gla::launch_recurrent_stream_state((hipStream_t)stream, B, T, H, DK, reverse, hidden_dtype, hidden_init,
                                                   log_fgate, value, key, query, hidden_final, g_shift, gate_sums);
-    if (DK != 256 || !workspace)
+    if (DK != 256 || !workspace || dtype == GLA_F32)
         return recurrent_fwd_run(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
                                  log_fgate, value, key, query, hidden_final, out);
     const gla::SplitSizes z(B, T, H, dtype);

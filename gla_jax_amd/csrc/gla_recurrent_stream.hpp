@@ -12,6 +12,11 @@ int launch_recurrent_stream_fwd(hipStream_t st, int B, int T_len, int H, int D, 
                                 const void *h0, const float *g, const void *v, const void *k, const void *q,
                                 void *hT, void *out);
 
+// The forward in fp32 vector arithmetic (gla_recurrent_steps.hip): any element types and head dimension.
+template <typename T, typename TO>
+int launch_recurrent_steps(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt, const void *h0,
+                           const float *g, const void *v, const void *k, const void *q, void *hT, void *out);
+
 // The forward without its outputs: hidden_final alone (what a segment contributes to the state that leaves it).
 // h0 may be null: the state starts from zeros.  g_shift = +1 or -1: every step takes the gate of the next (previous)
 // row of the array instead of its own (the recurrence of the state's cotangent, where the decay between two steps
