@@ -74,15 +74,17 @@ template <typename T, typename TO, int RV, int U>
 __global__ __launch_bounds__(RV * 64) void recurrent_bwd_dq_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const T *__restrict__ v,
     const T *__restrict__ k, const T *__restrict__ q, const void *__restrict__ dhT,
-    const TO *__restrict__ dout, T *__restrict__ dq, float *__restrict__ qdq, int T_len, int H, int reverse,
+    const TO *__restrict__ dout, T *__restrict__ dq, float *__restrict__ qdq, Segments sg, int H, int reverse,
     int hdt)
 {
     constexpr int DV = RV * 16, DK = DV;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int a = lane >> 4, c = lane & 15;
-    const int h = blockIdx.x, b = blockIdx.y;
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x;
     const int dk0 = wave * 16 + a * 4, dv0 = c * RV;
-    const int64_t bh = (int64_t)b * H + h;
+    const int64_t bh = (int64_t)seg.index * H + h;
 
     float S[4][RV];
     {
@@ -91,8 +93,8 @@ __global__ __launch_bounds__(RV * 64) void recurrent_bwd_dq_kernel(
         for (int i = 0; i < 4; ++i) load_hidden<RV>(h0, hdt, ho + (int64_t)i * DV, S[i]);
     }
     const int64_t strideK = (int64_t)H * DK, strideV = (int64_t)H * DV;
-    const int64_t offK = ((int64_t)b * T_len * H + h) * DK + dk0;
-    const int64_t offV = ((int64_t)b * T_len * H + h) * DV + dv0;
+    const int64_t offK = (seg.row0 * H + h) * DK + dk0;
+    const int64_t offV = (seg.row0 * H + h) * DV + dv0;
 
     struct Step {
         RawVec<float, 4> g;
@@ -191,15 +193,17 @@ __global__ __launch_bounds__(RV * 64) void recurrent_bwd_rev_kernel(
     const float *__restrict__ g, const T *__restrict__ v, const T *__restrict__ k,
     const T *__restrict__ q, const void *__restrict__ dhT,
     const TO *__restrict__ dout, void *__restrict__ dh0, float *__restrict__ dg, T *__restrict__ dv,
-    T *__restrict__ dk, int T_len, int H, int reverse, int hdt)
+    T *__restrict__ dk, Segments sg, int H, int reverse, int hdt)
 {
     constexpr int DV = RV * 16, DK = DV, NW = RV;
     __shared__ float part[TB * NW * 4 * DV];   // [slot][wave][a][dv]: partial dv of 4 state rows each
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int a = lane >> 4, c = lane & 15;
-    const int h = blockIdx.x, b = blockIdx.y;
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x;
     const int dk0 = wave * 16 + a * 4, dv0 = c * RV;
-    const int64_t bh = (int64_t)b * H + h;
+    const int64_t bh = (int64_t)seg.index * H + h;
 
     float D[4][RV], run[4];   // run: sum over the later steps of q*dq - k*dk (sweep 1 put sum_v dhT*hT into the last q*dq)
     {
@@ -211,9 +215,9 @@ __global__ __launch_bounds__(RV * 64) void recurrent_bwd_rev_kernel(
         }
     }
     const int64_t strideK = (int64_t)H * DK, strideV = (int64_t)H * DV;
-    const int64_t offK = ((int64_t)b * T_len * H + h) * DK + dk0;
-    const int64_t offV = ((int64_t)b * T_len * H + h) * DV + dv0;
-    const int64_t offVrow = ((int64_t)b * T_len * H + h) * DV;
+    const int64_t offK = (seg.row0 * H + h) * DK + dk0;
+    const int64_t offV = (seg.row0 * H + h) * DV + dv0;
+    const int64_t offVrow = (seg.row0 * H + h) * DV;
 
     struct Step {
         RawVec<float, 4> g, w;
@@ -321,19 +325,19 @@ constexpr int64_t kFewSteps = 32;
 constexpr int64_t kFewSteps256 = 64;
 
 template <typename T, typename TO>
-static int launch_bwd(hipStream_t st, int B, int T_len, int H, int DK, int DV, int reverse, int hdt,
+static int launch_bwd(hipStream_t st, int B, Segments sg, int H, int DK, int DV, int reverse, int hdt,
                       const void *h0, const float *g, const void *v, const void *k, const void *q,
                       const void * /* hidden_final: recomputed in fp32 by sweep 1 */, const void *dhT,
                       const void *dout, void *dh0, float *dg, void *dv, void *dk, void *dq, int wide)
 {
-    dim3 grid(H, B), block(DK / 16 * 64);
+    dim3 grid(H, sg.S, B), block(DK / 16 * 64);
     // bf16 data at head dimensions 64 and 128 runs both sweeps on the matrix cores, whatever the type of dout
     if (sizeof(T) == 2 && (DK == 64 || DK == 128)) {
         const int dout_f32 = sizeof(TO) == 4;
-        int e = launch_recurrent_stream_dq(st, B, T_len, H, DK, reverse, hdt, dout_f32, h0, g, v, k, q, dhT, dout, dq,
+        int e = launch_recurrent_stream_dq(st, B, sg, H, DK, reverse, hdt, dout_f32, h0, g, v, k, q, dhT, dout, dq,
                                            dg, wide);
         if (e) return e;
-        return launch_recurrent_stream_rev(st, B, T_len, H, DK, reverse, hdt, dout_f32, g, v, k, q, dhT, dout, dh0, dg,
+        return launch_recurrent_stream_rev(st, B, sg, H, DK, reverse, hdt, dout_f32, g, v, k, q, dhT, dout, dh0, dg,
                                            dv, dk, wide);
     }
     if (wide && sizeof(T) != 4) return GLA_ERR_UNSUPPORTED;   // float gradients: the matrix-core kernels or float data
@@ -341,10 +345,10 @@ static int launch_bwd(hipStream_t st, int B, int T_len, int H, int DK, int DV, i
     do {                                                                                                \
         hipLaunchKernelGGL((recurrent_bwd_dq_kernel<T, TO, RV_, U_>), grid, block, 0, st,               \
                            h0, g, (const T *)v, (const T *)k, (const T *)q,                             \
-                           dhT, (const TO *)dout, (T *)dq, dg, T_len, H, reverse, hdt);                 \
+                           dhT, (const TO *)dout, (T *)dq, dg, sg, H, reverse, hdt);                 \
         hipLaunchKernelGGL((recurrent_bwd_rev_kernel<T, TO, RV_, TB_>), grid, block, 0, st, g,          \
                            (const T *)v, (const T *)k, (const T *)q, dhT,                               \
-                           (const TO *)dout, dh0, dg, (T *)dv, (T *)dk, T_len, H, reverse, hdt);        \
+                           (const TO *)dout, dh0, dg, (T *)dv, (T *)dk, sg, H, reverse, hdt);        \
     } while (0)
     switch (DV / 16) {
     case 1: GLA_BWD_CASE(1, 4, 4); break;
@@ -376,13 +380,14 @@ static int check_recurrent(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t 
 
 // ---- head dimension 256 as four problems of head dimension 128 (gla_split.hip) ---------------------------------
 // Two passes of the 128-feature kernels over 2H heads, their results left in fp32 and added with one rounding.
-// rows: one [B,T,H,256] array of floats; hid: one [B,2H,128,128] array of states (sized for fp32 states).
+// rows: one [B,T,H,256] array; hid: one [B,2H,128,128] array of states per segment (sized for fp32 states).
 namespace gla {
 struct SplitSizes {
     size_t rows_e, rows_f32, hid;
-    SplitSizes(int64_t B, int64_t T, int64_t H, int dtype)
-        : rows_e(round_up256((size_t)B * T * H * 256 * (dtype == GLA_BF16 ? 2 : 4))),
-          rows_f32(round_up256((size_t)B * T * H * 256 * 4)), hid(round_up256((size_t)B * 2 * H * 128 * 128 * 4))
+    // `rows` time steps in all and `states` states per head
+    SplitSizes(int64_t rows, int64_t states, int64_t H, int dtype)
+        : rows_e(round_up256((size_t)rows * H * 256 * (dtype == GLA_BF16 ? 2 : 4))),
+          rows_f32(round_up256((size_t)rows * H * 256 * 4)), hid(round_up256((size_t)states * 2 * H * 128 * 128 * 4))
     {
     }
     static size_t round_up256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -394,14 +399,16 @@ struct SplitSizes {
 };
 }  // namespace gla
 
-static int recurrent_fwd_run(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
+static gla::Segments whole(int64_t T) { return {(int)T, 1, (int)T}; }
+
+static int recurrent_fwd_run(void *stream, int64_t B, gla::Segments sg, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
                              gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse, const void *hidden_init,
                              const float *log_fgate, const void *value, const void *key, const void *query,
-                             void *hidden_final, void *out)
+                             void *hidden_final, void *out, bool zero_init = false)
 {
-    int rc = gla::check_recurrent(B, T, H, DK, DV, dtype, hidden_dtype, out_dtype);
+    int rc = gla::check_recurrent(B, sg.T, H, DK, DV, dtype, hidden_dtype, out_dtype);
     if (rc) return rc;
-    if (!hidden_init || !log_fgate || !value || !key || !query || !hidden_final || !out)
+    if ((!hidden_init && !zero_init) || !log_fgate || !value || !key || !query || !hidden_final || !out)
         return GLA_ERR_NULL;
     const void *ptrs[] = {hidden_init, log_fgate, value, key, query, hidden_final, out};
     for (const void *p : ptrs)
@@ -410,14 +417,14 @@ static int recurrent_fwd_run(void *stream, int64_t B, int64_t T, int64_t H, int6
     // fp32 `out` beside bf16 data (the recurrent_gla_naive flavour, gla.py:37) is the same kernels storing their fp32 sums
     // unrounded
     const bool out_f32 = dtype == GLA_BF16 && out_dtype == GLA_F32;
-    if (dtype == GLA_BF16 && (DK == 64 || DK == 128) && T > gla::kFewSteps) {
+    if (dtype == GLA_BF16 && (DK == 64 || DK == 128) && sg.L > gla::kFewSteps) {
         auto run = out_f32 ? gla::launch_recurrent_stream_fwd<float> : gla::launch_recurrent_stream_fwd<__bf16>;
-        return run(st, B, T, H, DK, reverse, hidden_dtype, hidden_init, log_fgate, value, key, query, hidden_final, out);
+        return run(st, B, sg, H, DK, reverse, hidden_dtype, hidden_init, log_fgate, value, key, query, hidden_final, out);
     }
     auto run = dtype == GLA_F32 ? gla::launch_recurrent_steps<float, float>
                : out_f32        ? gla::launch_recurrent_steps<__bf16, float>
                                 : gla::launch_recurrent_steps<__bf16, __bf16>;
-    return run(st, B, T, H, DK, reverse, hidden_dtype, hidden_init, log_fgate, value, key, query, hidden_final, out);
+    return run(st, B, sg, H, DK, reverse, hidden_dtype, hidden_init, log_fgate, value, key, query, hidden_final, out);
 }
 
 extern "C" int gla_recurrent_fwd(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
@@ -425,73 +432,90 @@ extern "C" int gla_recurrent_fwd(void *stream, int64_t B, int64_t T, int64_t H, 
                                  const void *hidden_init, const float *log_fgate, const void *value,
                                  const void *key, const void *query, void *hidden_final, void *out)
 {
-    return recurrent_fwd_run(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init, log_fgate,
-                             value, key, query, hidden_final, out);
+    return recurrent_fwd_run(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
+                             log_fgate, value, key, query, hidden_final, out);
 }
 
 // ---- a sequence as S segments side by side (gla_timesplit.hip) -------------------------------------------------
-// With few (batch, head) pairs (at most half of the GPU's compute units for bf16 data at 64 features and more, a
-// quarter otherwise), a call with a workspace runs every sequence as S segments at once: one pass from zero states for the segments' own contributions, a scan over the
-// segments, and the real pass with the states that enter each segment (fp32); the backward does the same for
-// the states' cotangents.  The segments are batch entries of the same kernels: [B,T,H,D] is [B*S,T/S,H,D].
+// With few (batch, head) pairs (at most half of the GPU's compute units), a call with a workspace runs every sequence as S segments at once: one pass from zero states for
+// the segments' own contributions, a scan over the segments, and the real pass with the states that enter each segment
+// (fp32); the backward does the same for the states' cotangents.
 namespace gla {
 constexpr int64_t kComputeUnits = 256;       // MI355X
-constexpr int64_t kMinSegment = 128;         // steps: one or two iterations of the kernels (with 256 the small shapes left
-                                             // compute units idle: B1 T2048 H4 D128 0.31 -> 0.20 ms, B1 T1024 H8 D64 0.11 -> 0.08)
+constexpr int64_t kMinSegment = 128;         // steps
 constexpr int64_t kMinLeanPiece = 256;       // steps of a piece where the lean passes take a segment in two
 // bf16 data at head dimensions 64, 128 (and 256 as two passes of 128): the forward kernel has a form that leaves out
 // everything but the state
 static inline bool has_lean_pass(int dtype, int64_t DK) { return dtype == GLA_BF16 && DK >= 64; }
+static inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 struct TimeSplit {
-    int64_t S = 1, L = 0;
-    int64_t F = 1, Lf = 0;       // the lean passes run every segment as F pieces of Lf steps
+    Segments sg, pieces;         // `pieces`: what the lean passes run, every segment as F of them
+    int F = 1;
+    int64_t nseg = 0, npiece = 0;               // segments and pieces of the whole batch
     size_t hid = 0, hidf = 0, sums = 0;
-    TimeSplit(int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
+    TimeSplit(int64_t B, int64_t T, int64_t H, int64_t DK, int dtype) : sg{(int)T, 1, (int)T}, pieces(sg)
     {
+        const bool lean = has_lean_pass(dtype, DK), heavy = lean && DK >= 128;
         const int64_t seqs = B * H * (DK == 256 ? 2 : 1);    // head dimension 256 runs as 2H heads of 128
-        // the most segments that divide T into pieces of kMinSegment steps or more without asking for more
-        // workgroups than there are compute units
-        for (int64_t s = kComputeUnits / (seqs > 0 ? seqs : 1); s > 1; --s)
-            if (T % s == 0 && T / s >= kMinSegment && B * s <= 65535) {
-                S = s;
+        const int64_t most = kComputeUnits / seqs;           // no more workgroups than compute units
+        // where the first pass is a full kernel, two or three segments save too little
+        if (most < (lean ? 2 : 4)) return;
+        // whole iterations of the matrix-core kernels (64 steps), of both pieces where the lean passes run in two; two
+        // iterations at least (with four the small shapes left compute units idle: B1 T2048 H4 D128 0.31 -> 0.20 ms)
+        const int64_t unit = !lean ? 1 : (heavy && ceil_div(T, most) >= 2 * kMinLeanPiece ? 128 : 64);
+        auto rounded = [&](int64_t steps) { return ceil_div(steps, unit) * unit; };
+        int64_t L = rounded(ceil_div(T, most));
+        if (L < kMinSegment) L = kMinSegment;
+        // segments of one length, if that is hardly longer
+        for (int64_t s = most; s > 1; --s)
+            if (T % s == 0 && T / s >= L) {
+                if (rounded(T / s) * 4 <= L * 5) L = T / s;
                 break;
             }
-        // At 128 features an iteration of the kernels is 64 steps, and segments of one iteration still pay while they
-        // leave half of the compute units idle or more (B1 T2048 H4 D128 0.20 -> 0.17 ms); beyond that a segment's
-        // own state, read and written once per pass, outweighs its 64 rows (B1 T8192 H2 D128 0.27 -> 0.29 ms).
-        if (DK >= 128 && S > 1 && seqs * S * 2 <= kComputeUnits / 2 && (T / S) % 2 == 0 && T / S / 2 >= 64 &&
-            B * S * 2 <= 65535)
-            S *= 2;
-        // Two segments mean two passes over half the steps each: that pays where the first pass is the lean one (bf16
-        // data at 64 features and more: B16 T2048 H8 1.47 -> 1.08 ms at 128 features, 0.44 -> 0.39 ms at 64); where it
-        // is a full kernel, from four segments on.
-        const bool heavy = dtype == GLA_BF16 && DK >= 128;
-        if (S < (has_lean_pass(dtype, DK) ? 2 : 4)) S = 1;
-        L = T / S;
+        // At 128 features segments of one iteration still pay while they leave half of the compute units idle or more
+        // (B1 T2048 H4 D128 0.20 -> 0.17 ms); beyond that a segment's own state, read and written once per pass,
+        // outweighs its 64 rows (B1 T8192 H2 D128 0.27 -> 0.29 ms).
+        if (heavy && L == kMinSegment && seqs * ceil_div(T, 64) <= kComputeUnits / 2) L = 64;
+        const int64_t S = ceil_div(T, L);
+        // From which length on the passes over shorter segments outweigh the pass they add (forward + backward, whole /
+        // in segments, us).  64 features: 61 / 68 at T = 256 and 76 / 69 at 288 with 8 sequences, 63 / 75 and 78 / 79 with
+        // 64; two segments per sequence 190 / 192 at 896 and 215 / 203 at 1024.  128 features: 206 / 200 at 193 (161 / 200
+        // at 129), and less where segments of 64 steps fit (156 / 120 at 129); two segments 251 / 283 at 288 and 297 / 286
+        // at 384.  Full first pass (fp32, 64 features, 8 sequences): 350 / 360 at 300, 593 / 278 at 512.
+        const int64_t from = heavy ? (most == 2 ? 384 : 201) : lean ? (most == 2 ? 1024 : (most == 3 ? 384 : 256)) : 256;
+        if (T < from || S < 2 || S * 2 > 65535) return;
+        sg.S = (int)S;
+        sg.L = (int)L;
         // The lean kernel of 128 features fits a compute unit twice (256 registers, 52 KB of LDS) where the full
         // kernels fit once: its passes take every segment in two pieces (512 workgroups: 100 -> 70 us at 1024 steps
         // per segment), and the scan puts the pieces together.  Pieces of 128 steps are two iterations of the kernel
         // and lose what the second workgroup gains.
-        if (S > 1 && heavy && L % 2 == 0 && L / 2 >= kMinLeanPiece && B * S * 2 <= 65535) F = 2;
-        Lf = L / F;
-        hid = SplitSizes::round_up256((size_t)B * S * H * DK * DK * 4);
-        hidf = SplitSizes::round_up256((size_t)B * S * F * H * DK * DK * 4);
-        sums = SplitSizes::round_up256((size_t)B * S * F * H * DK * 4);
+        if (heavy && L % 2 == 0 && L / 2 >= kMinLeanPiece) F = 2;
+        pieces.L = (int)(L / F);
+        pieces.S = (int)ceil_div(T, pieces.L);
+        nseg = B * S;
+        npiece = B * pieces.S;
+        hid = SplitSizes::round_up256((size_t)nseg * H * DK * DK * 4);
+        hidf = SplitSizes::round_up256((size_t)npiece * H * DK * DK * 4);
+        sums = SplitSizes::round_up256((size_t)npiece * H * DK * 4);
     }
-    bool on() const { return S > 1; }
+    bool on() const { return sg.S > 1; }
     // forward: entering states, the pieces' own contributions, gate sums
     size_t fwd() const { return on() ? hid + hidf + sums : 0; }
     // backward: the same, the cotangents that leave the segments, and a second array of contributions for an fp32
     // dout beside bf16 data (two passes)
     size_t bwd() const { return on() ? 2 * hid + 2 * hidf + sums : 0; }
 };
-static size_t inner_fwd_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
+// what head dimension 256 needs for its own passes, over the segments or pieces there are
+static size_t inner_fwd_bytes(const TimeSplit &ts, int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
 {
-    return DK == 256 && dtype == GLA_BF16 ? SplitSizes(B, T, H, dtype).fwd() : 0;   // fp32 data needs no passes
+    if (DK != 256 || dtype == GLA_F32) return 0;                 // (the forward of fp32 data takes no passes)
+    if (T <= kFewSteps256) return 256;                           // nor do few steps: the argument stays required, at no cost
+    return SplitSizes(B * T, ts.on() ? ts.npiece : B, H, dtype).fwd();
 }
-static size_t inner_bwd_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
+static size_t inner_bwd_bytes(const TimeSplit &ts, int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
 {
-    return DK == 256 ? SplitSizes(B, T, H, dtype).bwd() : 0;
+    return DK == 256 ? SplitSizes(B * T, ts.on() ? ts.npiece : B, H, dtype).bwd() : 0;
 }
 }  // namespace gla
 
@@ -499,9 +523,8 @@ extern "C" size_t gla_recurrent_fwd_workspace_bytes(int64_t B, int64_t T, int64_
                                                     gla_dtype dtype)
 {
     if (gla::check_recurrent(B, T, H, DK, DV, dtype, GLA_F32, GLA_F32) || 2 * H > 65535) return 0;
-    if (DK == 256 && T <= gla::kFewSteps256) return 0;
-    const gla::TimeSplit ts(B, T, H, DK, dtype);      // the passes run on B*S batch entries of L steps: their state blocks count
-    return ts.fwd() + gla::inner_fwd_bytes(B * ts.S * ts.F, ts.Lf, H, DK, dtype);
+    const gla::TimeSplit ts(B, T, H, DK, dtype);
+    return ts.fwd() + gla::inner_fwd_bytes(ts, B, T, H, DK, dtype);
 }
 
 extern "C" size_t gla_recurrent_bwd_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
@@ -509,63 +532,64 @@ extern "C" size_t gla_recurrent_bwd_workspace_bytes(int64_t B, int64_t T, int64_
 {
     if (gla::check_recurrent(B, T, H, DK, DV, dtype, GLA_F32, GLA_F32) || 2 * H > 65535) return 0;
     const gla::TimeSplit ts(B, T, H, DK, dtype);
-    return ts.bwd() + gla::inner_bwd_bytes(B * ts.S * ts.F, ts.Lf, H, DK, dtype);
+    return ts.bwd() + gla::inner_bwd_bytes(ts, B, T, H, DK, dtype);
 }
 
-// One pass over whole sequences; arguments checked by the caller.  Head dimension 256 with a workspace: two passes
+// One pass over the segments of `sg`; arguments checked by the caller.  Head dimension 256 with a workspace: two passes
 // of the 128-feature kernels; everything else: the kernels directly.
-static int recurrent_fwd_inner(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
+static int recurrent_fwd_inner(void *stream, int64_t B, gla::Segments sg, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
                                gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse, const void *hidden_init,
                                const float *log_fgate, const void *value, const void *key, const void *query,
                                void *hidden_final, void *out, void *workspace, bool state_only = false,
                                int g_shift = 0, float *gate_sums = nullptr)
 {
-    // state_only: the caller wants hidden_final alone and `out` is a buffer it will overwrite.  The matrix-core
-    // kernels have a form without the output products (hidden_init may be null there: zeros); the other kernels
-    // write the unused `out`.
+    // state_only: the caller wants hidden_final alone, from zero states (hidden_init is null), and `out` is a buffer it
+    // will overwrite.  The matrix-core kernels have a form without the output products; the vector kernel writes the
+    // unused `out`.
     // g_shift (lean passes only): the gates are taken one row further on (+1) or back (-1), see the launcher.
     const bool lean = state_only && dtype == GLA_BF16;
     // gate_sums (lean passes only): the pass also leaves the sum of every sequence's gates there, [B][H][DK].
     if ((g_shift || gate_sums) && !(lean && DK >= 64)) return GLA_ERR_UNSUPPORTED;
     if (lean && (DK == 64 || DK == 128))
-        return gla::launch_recurrent_stream_state((hipStream_t)stream, B, T, H, DK, reverse, hidden_dtype, hidden_init,
+        return gla::launch_recurrent_stream_state((hipStream_t)stream, B, sg, H, DK, reverse, hidden_dtype, hidden_init,
                                                   log_fgate, value, key, query, hidden_final, g_shift, gate_sums);
-    if (DK != 256 || !workspace || dtype == GLA_F32)
-        return recurrent_fwd_run(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
-                                 log_fgate, value, key, query, hidden_final, out);
-    const gla::SplitSizes z(B, T, H, dtype);
+    if (DK != 256 || !workspace || dtype == GLA_F32 || (sg.S == 1 && sg.T <= gla::kFewSteps256))
+        return recurrent_fwd_run(stream, B, sg, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
+                                 log_fgate, value, key, query, hidden_final, out, state_only);
+    const int64_t states = B * sg.S, rows = B * sg.T;
+    const gla::SplitSizes z(rows, states, H, dtype);
     hipStream_t st = (hipStream_t)stream;
     unsigned char *ws = (unsigned char *)workspace;
     unsigned char *v_sw = ws, *out1 = v_sw + z.rows_e, *out2 = out1 + z.rows_f32, *h0_same = out2 + z.rows_f32,
                   *h0_cross = h0_same + z.hid, *hT_same = h0_cross + z.hid, *hT_cross = hT_same + z.hid;
     int e = 0;
     if (hidden_init) {      // (a lean pass may start from zeros: no initial state given)
-        e = gla::launch_hidden_blocks(st, hidden_dtype, B * H, const_cast<void *>(hidden_init), h0_same, h0_cross, 1);
+        e = gla::launch_hidden_blocks(st, hidden_dtype, states * H, const_cast<void *>(hidden_init), h0_same, h0_cross, 1);
         if (e) return e;
     }
-    e = gla::launch_swap_halves(st, dtype, B * T * H, v_sw, value);
+    e = gla::launch_swap_halves(st, dtype, rows * H, v_sw, value);
     if (e) return e;
     // key half a with value half a on the arrays as they lie, then key half a with the other value half; `out` of
     // both in fp32 (the recurrent_gla_naive flavour of the 128-feature kernels)
     if (lean) {
-        e = gla::launch_recurrent_stream_state(st, B, T, 2 * H, 128, reverse, hidden_dtype, hidden_init ? h0_same : nullptr,
+        e = gla::launch_recurrent_stream_state(st, B, sg, 2 * H, 128, reverse, hidden_dtype, hidden_init ? h0_same : nullptr,
                                                log_fgate, value, key, query, hT_same, g_shift, gate_sums);
         if (e) return e;
-        e = gla::launch_recurrent_stream_state(st, B, T, 2 * H, 128, reverse, hidden_dtype,
+        e = gla::launch_recurrent_stream_state(st, B, sg, 2 * H, 128, reverse, hidden_dtype,
                                                hidden_init ? h0_cross : nullptr, log_fgate, v_sw, key, query, hT_cross,
                                                g_shift);
         if (e) return e;
-        return gla::launch_hidden_blocks(st, hidden_dtype, B * H, hidden_final, hT_same, hT_cross, 0);
+        return gla::launch_hidden_blocks(st, hidden_dtype, states * H, hidden_final, hT_same, hT_cross, 0);
     }
-    e = recurrent_fwd_run(stream, B, T, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_same, log_fgate,
+    e = recurrent_fwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_same, log_fgate,
                           value, key, query, hT_same, out1);
     if (e) return e;
-    e = recurrent_fwd_run(stream, B, T, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_cross, log_fgate, v_sw,
+    e = recurrent_fwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_cross, log_fgate, v_sw,
                           key, query, hT_cross, out2);
     if (e) return e;
-    e = gla::launch_sum_rows(st, out_dtype, B * T * H, out, (const float *)out1, (const float *)out2, 1);
+    e = gla::launch_sum_rows(st, out_dtype, rows * H, out, (const float *)out1, (const float *)out2, 1);
     if (e) return e;
-    return gla::launch_hidden_blocks(st, hidden_dtype, B * H, hidden_final, hT_same, hT_cross, 0);
+    return gla::launch_hidden_blocks(st, hidden_dtype, states * H, hidden_final, hT_same, hT_cross, 0);
 }
 
 extern "C" int gla_recurrent_fwd_ws(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
@@ -576,7 +600,7 @@ extern "C" int gla_recurrent_fwd_ws(void *stream, int64_t B, int64_t T, int64_t 
 {
     const size_t need = gla_recurrent_fwd_workspace_bytes(B, T, H, DK, DV, dtype);
     if (!need)      // nothing to gain from a workspace at this shape
-        return recurrent_fwd_run(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
+        return recurrent_fwd_run(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
                                  log_fgate, value, key, query, hidden_final, out);
     int rc = gla::check_recurrent(B, T, H, DK, DV, dtype, hidden_dtype, out_dtype);
     if (rc) return rc;
@@ -589,41 +613,38 @@ extern "C" int gla_recurrent_fwd_ws(void *stream, int64_t B, int64_t T, int64_t 
     if (!gla::aligned16(workspace)) return GLA_ERR_ALIGN;
     const gla::TimeSplit ts(B, T, H, DK, dtype);
     if (!ts.on())
-        return recurrent_fwd_inner(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
+        return recurrent_fwd_inner(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
                                    log_fgate, value, key, query, hidden_final, out, workspace);
     hipStream_t st = (hipStream_t)stream;
     unsigned char *ws = (unsigned char *)workspace;
     float *entering = (float *)ws, *loc = (float *)(ws + ts.hid), *sums = (float *)(ws + ts.hid + ts.hidf);
     void *inner_ws = DK == 256 ? ws + ts.fwd() : nullptr;
     const bool lean = gla::has_lean_pass(dtype, DK);
-    const int64_t pieces = B * ts.S * ts.F;
     int e = 0;
-    if (!lean) {            // (F = 1 then) the full kernels want an initial state, zeros, and leave the gate sums to a kernel
-        e = gla::launch_segment_gate_sums(st, B, ts.S * ts.F, ts.Lf, H, (int)DK, log_fgate, sums);
-        if (e) return e;
-        e = gla::launch_zero_fill(st, entering, ts.hid);
+    if (!lean) {            // (F = 1 then) the vector kernel leaves the gate sums to one of their own
+        e = gla::launch_segment_gate_sums(st, B, ts.sg, H, (int)DK, log_fgate, sums);
         if (e) return e;
     }
     // every piece from a zero state: its own contribution to the state that leaves it, and its gate sums (where this
     // is a full pass, it writes an `out` that the pass below writes again)
-    e = recurrent_fwd_inner(stream, pieces, ts.Lf, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, lean ? nullptr : entering,
-                            log_fgate, value, key, query, loc, out, inner_ws, true, 0, lean ? sums : nullptr);
+    e = recurrent_fwd_inner(stream, B, ts.pieces, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, nullptr, log_fgate, value,
+                            key, query, loc, out, inner_ws, true, 0, lean ? sums : nullptr);
     if (e) return e;
-    e = gla::launch_segment_scan(st, B, ts.S, ts.F, ts.Lf, H, (int)DK, hidden_dtype, hidden_init, loc, nullptr, sums,
+    e = gla::launch_segment_scan(st, B, ts.pieces, ts.F, H, (int)DK, hidden_dtype, hidden_init, loc, nullptr, sums,
                                  nullptr, 0, reverse, entering, hidden_final);
     if (e) return e;
-    return recurrent_fwd_inner(stream, B * ts.S, ts.L, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, entering,
-                               log_fgate, value, key, query, loc, out, inner_ws);
+    return recurrent_fwd_inner(stream, B, ts.sg, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, entering, log_fgate, value,
+                               key, query, loc, out, inner_ws);
 }
 
 // wide != 0: dvalue, dkey, dquery are float arrays whatever `dtype` is
-static int recurrent_bwd_run(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
+static int recurrent_bwd_run(void *stream, int64_t B, gla::Segments sg, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
                              gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse, const void *hidden_init,
                              const float *log_fgate, const void *value, const void *key, const void *query,
                              const void *hidden_final, const void *dhidden_final, const void *dout,
                              void *dhidden_init, float *dlog_fgate, void *dvalue, void *dkey, void *dquery, int wide)
 {
-    int rc = gla::check_recurrent(B, T, H, DK, DV, dtype, hidden_dtype, out_dtype);
+    int rc = gla::check_recurrent(B, sg.T, H, DK, DV, dtype, hidden_dtype, out_dtype);
     if (rc) return rc;
     const void *ptrs[] = {hidden_init, log_fgate, value, key, query, hidden_final, dhidden_final,
                           dout, dhidden_init, dlog_fgate, dvalue, dkey, dquery};
@@ -633,14 +654,14 @@ static int recurrent_bwd_run(void *stream, int64_t B, int64_t T, int64_t H, int6
     }
     hipStream_t st = (hipStream_t)stream;
     if (dtype == GLA_BF16 && out_dtype == GLA_BF16)
-        return gla::launch_bwd<__bf16, __bf16>(st, B, T, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value,
+        return gla::launch_bwd<__bf16, __bf16>(st, B, sg, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value,
                                                key, query, hidden_final, dhidden_final, dout, dhidden_init,
                                                dlog_fgate, dvalue, dkey, dquery, wide);
     if (dtype == GLA_BF16)
-        return gla::launch_bwd<__bf16, float>(st, B, T, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value,
+        return gla::launch_bwd<__bf16, float>(st, B, sg, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value,
                                               key, query, hidden_final, dhidden_final, dout, dhidden_init,
                                               dlog_fgate, dvalue, dkey, dquery, wide);
-    return gla::launch_bwd<float, float>(st, B, T, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value, key,
+    return gla::launch_bwd<float, float>(st, B, sg, H, DK, DV, reverse, hidden_dtype, hidden_init, log_fgate, value, key,
                                          query, hidden_final, dhidden_final, dout, dhidden_init, dlog_fgate,
                                          dvalue, dkey, dquery, wide);
 }
@@ -652,13 +673,13 @@ extern "C" int gla_recurrent_bwd(void *stream, int64_t B, int64_t T, int64_t H, 
                                  const void *dhidden_final, const void *dout, void *dhidden_init,
                                  float *dlog_fgate, void *dvalue, void *dkey, void *dquery)
 {
-    return recurrent_bwd_run(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init, log_fgate,
+    return recurrent_bwd_run(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init, log_fgate,
                              value, key, query, hidden_final, dhidden_final, dout, dhidden_init, dlog_fgate, dvalue,
                              dkey, dquery, 0);
 }
 
-// One backward over whole sequences; arguments checked by the caller (see recurrent_fwd_inner).
-static int recurrent_bwd_inner(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
+// One backward over the segments of `sg`; arguments checked by the caller (see recurrent_fwd_inner).
+static int recurrent_bwd_inner(void *stream, int64_t B, gla::Segments sg, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype,
                                gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse, const void *hidden_init,
                                const float *log_fgate, const void *value, const void *key, const void *query,
                                const void *hidden_final, const void *dhidden_final, const void *dout,
@@ -666,10 +687,11 @@ static int recurrent_bwd_inner(void *stream, int64_t B, int64_t T, int64_t H, in
                                void *workspace)
 {
     if (DK != 256 || !workspace)
-        return recurrent_bwd_run(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
+        return recurrent_bwd_run(stream, B, sg, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
                                  log_fgate, value, key, query, hidden_final, dhidden_final, dout, dhidden_init,
                                  dlog_fgate, dvalue, dkey, dquery, 0);
-    const gla::SplitSizes z(B, T, H, dtype);
+    const int64_t states = B * sg.S, rows = B * sg.T * H;
+    const gla::SplitSizes z(B * sg.T, states, H, dtype);
     hipStream_t st = (hipStream_t)stream;
     unsigned char *ws = (unsigned char *)workspace;
     unsigned char *v_sw = ws, *do_sw = v_sw + z.rows_e, *dg2 = do_sw + z.rows_f32, *dq1 = dg2 + z.rows_f32,
@@ -677,20 +699,19 @@ static int recurrent_bwd_inner(void *stream, int64_t B, int64_t T, int64_t H, in
                   *dv2 = dv1 + z.rows_f32, *h0_same = dv2 + z.rows_f32, *h0_cross = h0_same + z.hid,
                   *dhT_same = h0_cross + z.hid, *dhT_cross = dhT_same + z.hid, *dh0_same = dhT_cross + z.hid,
                   *dh0_cross = dh0_same + z.hid;
-    const int64_t rows = B * T * H;
-    int e = gla::launch_hidden_blocks(st, hidden_dtype, B * H, const_cast<void *>(hidden_init), h0_same, h0_cross, 1);
+    int e = gla::launch_hidden_blocks(st, hidden_dtype, states * H, const_cast<void *>(hidden_init), h0_same, h0_cross, 1);
     if (e) return e;
-    e = gla::launch_hidden_blocks(st, hidden_dtype, B * H, const_cast<void *>(dhidden_final), dhT_same, dhT_cross, 1);
+    e = gla::launch_hidden_blocks(st, hidden_dtype, states * H, const_cast<void *>(dhidden_final), dhT_same, dhT_cross, 1);
     if (e) return e;
     e = gla::launch_swap_halves(st, dtype, rows, v_sw, value);
     if (e) return e;
     e = gla::launch_swap_halves(st, out_dtype, rows, do_sw, dout);
     if (e) return e;
     // hidden_final is not read by the kernels (sweep 1 forms the final state again in fp32); it is handed on as it is
-    e = recurrent_bwd_run(stream, B, T, 2 * H, 128, 128, dtype, hidden_dtype, out_dtype, reverse, h0_same, log_fgate,
+    e = recurrent_bwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, out_dtype, reverse, h0_same, log_fgate,
                           value, key, query, hidden_final, dhT_same, dout, dh0_same, dlog_fgate, dv1, dk1, dq1, 1);
     if (e) return e;
-    e = recurrent_bwd_run(stream, B, T, 2 * H, 128, 128, dtype, hidden_dtype, out_dtype, reverse, h0_cross, log_fgate,
+    e = recurrent_bwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, out_dtype, reverse, h0_cross, log_fgate,
                           v_sw, key, query, hidden_final, dhT_cross, do_sw, dh0_cross, (float *)dg2, dv2, dk2, dq2, 1);
     if (e) return e;
     e = gla::launch_sum_rows(st, dtype, rows, dquery, (const float *)dq1, (const float *)dq2, 0);
@@ -701,7 +722,7 @@ static int recurrent_bwd_inner(void *stream, int64_t B, int64_t T, int64_t H, in
     if (e) return e;
     e = gla::launch_add_rows(st, GLA_F32, rows, dlog_fgate, dg2, 0);
     if (e) return e;
-    return gla::launch_hidden_blocks(st, hidden_dtype, B * H, dhidden_init, dh0_same, dh0_cross, 0);
+    return gla::launch_hidden_blocks(st, hidden_dtype, states * H, dhidden_init, dh0_same, dh0_cross, 0);
 }
 
 extern "C" int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
@@ -714,7 +735,7 @@ extern "C" int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t 
 {
     const size_t need = gla_recurrent_bwd_workspace_bytes(B, T, H, DK, DV, dtype);
     if (!need)
-        return recurrent_bwd_run(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
+        return recurrent_bwd_run(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
                                  log_fgate, value, key, query, hidden_final, dhidden_final, dout, dhidden_init,
                                  dlog_fgate, dvalue, dkey, dquery, 0);
     int rc = gla::check_recurrent(B, T, H, DK, DV, dtype, hidden_dtype, out_dtype);
@@ -734,7 +755,7 @@ extern "C" int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t 
     // `out`: where there are none (D = 16, 32) such a call runs the sequences whole.
     const bool split_dout = out_dtype != dtype;
     if (!ts.on() || (split_dout && DK < 64))
-        return recurrent_bwd_inner(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
+        return recurrent_bwd_inner(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
                                    log_fgate, value, key, query, hidden_final, dhidden_final, dout, dhidden_init,
                                    dlog_fgate, dvalue, dkey, dquery, DK == 256 ? (unsigned char *)workspace + ts.bwd() : nullptr);
     hipStream_t st = (hipStream_t)stream;
@@ -742,23 +763,18 @@ extern "C" int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t 
     float *entering = (float *)ws, *dleaving = (float *)(ws + ts.hid), *loc = (float *)(ws + 2 * ts.hid),
           *loc_rem = (float *)(ws + 2 * ts.hid + ts.hidf), *sums = (float *)(ws + 2 * ts.hid + 2 * ts.hidf);
     void *inner_ws = DK == 256 ? ws + ts.bwd() : nullptr;      // sized for the backward, which needs more
-    const int64_t BS = B * ts.S, pieces = BS * ts.F;
     const bool lean = gla::has_lean_pass(dtype, DK);
     // 1. the states that enter the segments, as the forward formed them (where the pass is a full one, its `out` lands
     //    in dquery, which the backward proper overwrites)
     int e = 0;
     if (!lean) {
-        e = gla::launch_segment_gate_sums(st, B, ts.S * ts.F, ts.Lf, H, (int)DK, log_fgate, sums);
-        if (e) return e;
-        e = gla::launch_zero_fill(st, entering, ts.hid);
-        if (e) return e;
-        e = gla::launch_zero_fill(st, dleaving, ts.hid);
+        e = gla::launch_segment_gate_sums(st, B, ts.sg, H, (int)DK, log_fgate, sums);
         if (e) return e;
     }
-    e = recurrent_fwd_inner(stream, pieces, ts.Lf, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, lean ? nullptr : entering,
-                            log_fgate, value, key, query, loc, dquery, inner_ws, true, 0, lean ? sums : nullptr);
+    e = recurrent_fwd_inner(stream, B, ts.pieces, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, nullptr, log_fgate, value,
+                            key, query, loc, dquery, inner_ws, true, 0, lean ? sums : nullptr);
     if (e) return e;
-    e = gla::launch_segment_scan(st, B, ts.S, ts.F, ts.Lf, H, (int)DK, hidden_dtype, hidden_init, loc, nullptr, sums,
+    e = gla::launch_segment_scan(st, B, ts.pieces, ts.F, H, (int)DK, hidden_dtype, hidden_init, loc, nullptr, sums,
                                  nullptr, 0, reverse, entering, nullptr);
     if (e) return e;
     // 2. the cotangents of the states that leave the segments.  d(state) obeys the state's recurrence against time
@@ -779,27 +795,27 @@ extern "C" int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t 
         // dkey and dvalue hold the two halves of dout until the backward proper writes its results there
         e = gla::launch_head_remainder(st, B * T * H * DV, (const float *)dout, dkey, dvalue);
         if (e) return e;
-        e = recurrent_fwd_inner(stream, pieces, ts.Lf, H, DK, DV, dtype, GLA_F32, dtype, !reverse, nullptr, gates, dkey,
+        e = recurrent_fwd_inner(stream, B, ts.pieces, H, DK, DV, dtype, GLA_F32, dtype, !reverse, nullptr, gates, dkey,
                                 query, key, loc, nullptr, inner_ws, true, gs);
         if (e) return e;
-        e = recurrent_fwd_inner(stream, pieces, ts.Lf, H, DK, DV, dtype, GLA_F32, dtype, !reverse, nullptr, gates, dvalue,
+        e = recurrent_fwd_inner(stream, B, ts.pieces, H, DK, DV, dtype, GLA_F32, dtype, !reverse, nullptr, gates, dvalue,
                                 query, key, loc_rem, nullptr, inner_ws, true, gs);
         if (e) return e;
         loc2 = loc_rem;
     } else {
-        e = recurrent_fwd_inner(stream, pieces, ts.Lf, H, DK, DV, dtype, GLA_F32, out_dtype, !reverse,
-                                lean ? nullptr : dleaving, gates, dout, query, key, loc, dkey, inner_ws, true, gs);
+        e = recurrent_fwd_inner(stream, B, ts.pieces, H, DK, DV, dtype, GLA_F32, out_dtype, !reverse, nullptr,
+                                gates, dout, query, key, loc, dkey, inner_ws, true, gs);
         if (e) return e;
     }
     // what enters segment p from the steps behind it: per piece, the gate of its first step (in the order of the
     // recurrence) times its own contribution, plus its whole decay times what entered from further behind; after
     // the last piece that is dhidden_init
-    e = gla::launch_segment_scan(st, B, ts.S, ts.F, ts.Lf, H, (int)DK, hidden_dtype, dhidden_final, loc, loc2, sums,
-                                 log_fgate, reverse ? (int)ts.Lf - 1 : 0, !reverse, dleaving, dhidden_init);
+    e = gla::launch_segment_scan(st, B, ts.pieces, ts.F, H, (int)DK, hidden_dtype, dhidden_final, loc, loc2, sums,
+                                 log_fgate, reverse, !reverse, dleaving, dhidden_init);
     if (e) return e;
     // 3. the backward proper, every segment with its entering state and its leaving cotangent: the gate gradient's
     //    running sum starts from sum_v d(state) * state at the segment's end, which is what the steps behind it add
-    return recurrent_bwd_inner(stream, BS, ts.L, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, entering, log_fgate,
+    return recurrent_bwd_inner(stream, B, ts.sg, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, entering, log_fgate,
                                value, key, query, hidden_final, dleaving, dout, loc, dlog_fgate, dvalue, dkey, dquery,
                                inner_ws);
 }

@@ -31,24 +31,30 @@ constexpr int kStepsBatch = 8;           // steps whose inputs and partial outpu
 template <typename T, typename TO, int D>
 __global__ __launch_bounds__(StepsGeom<D>::NT) void recurrent_steps_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const T *__restrict__ v, const T *__restrict__ k,
-    const T *__restrict__ q, void *hT, TO *__restrict__ out, int T_len, int H, int reverse, int hdt)
+    const T *__restrict__ q, void *hT, TO *__restrict__ out, Segments sg, int H, int reverse, int hdt)
 {
     typedef StepsGeom<D> G;
     constexpr int W = G::W, CL = G::CL, NT = G::NT, RPT = G::RPT, NP = G::NP, TB = kStepsBatch;
     constexpr int kItems = (TB * D / 4 + NT - 1) / NT;           // groups of 4 features a thread brings in per batch
     extern __shared__ __align__(16) float smem[];
     const int tid = threadIdx.x, cl = tid % CL, rg = tid / CL;
-    const int h = blockIdx.x / (D / W), slab = blockIdx.x % (D / W), b = blockIdx.y;
-    const int64_t bh = (int64_t)b * H + h;
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x / (D / W), slab = blockIdx.x % (D / W);
+    const int64_t bh = (int64_t)seg.index * H + h;
     const int64_t ho = (bh * D + rg * RPT) * D + slab * W + 4 * cl;
-    const int64_t seq = ((int64_t)b * T_len * H + h) * D, rowstride = (int64_t)H * D;
+    const int64_t seq = (seg.row0 * H + h) * D, rowstride = (int64_t)H * D;
     const int tb = T_len < TB ? T_len : TB;                      // the launcher's LDS holds this many steps
     float *sf = smem, *sk = sf + tb * D, *sq = sk + tb * D;      // [tb][D] e^g, key, query
     float *sv = sq + tb * D, *part = sv + tb * W;                // [tb][W] value; [tb][NP][W] partial outputs
 
     float S[RPT][4];
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) load_hidden<4>(h0, hdt, ho + (int64_t)i * D, S[i]);
+    for (int i = 0; i < RPT; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[i][j] = 0.f;
+        if (h0) load_hidden<4>(h0, hdt, ho + (int64_t)i * D, S[i]);
+    }
 
     auto row = [&](int step) { return seq + (int64_t)(reverse ? T_len - 1 - step : step) * rowstride; };
     float gN[kItems][4], kN[kItems][4], qN[kItems][4], vN[4];
@@ -126,15 +132,15 @@ __global__ __launch_bounds__(StepsGeom<D>::NT) void recurrent_steps_kernel(
 }
 
 template <typename T, typename TO>
-int launch_recurrent_steps(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt, const void *h0,
+int launch_recurrent_steps(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, const void *h0,
                            const float *g, const void *v, const void *k, const void *q, void *hT, void *out)
 {
-    const size_t tb = T_len < kStepsBatch ? T_len : kStepsBatch;
+    const size_t tb = sg.L < kStepsBatch ? sg.L : kStepsBatch;
 #define GLA_STEPS_CASE(D_)                                                                                          \
     case D_:                                                                                                        \
-        hipLaunchKernelGGL((recurrent_steps_kernel<T, TO, D_>), dim3(H * (D_ / StepsGeom<D_>::W), B),               \
+        hipLaunchKernelGGL((recurrent_steps_kernel<T, TO, D_>), dim3(H * (D_ / StepsGeom<D_>::W), sg.S, B),               \
                            dim3(StepsGeom<D_>::NT), tb * StepsGeom<D_>::kStepFloats * sizeof(float), st, h0, g, (const T *)v, (const T *)k, (const T *)q, hT,     \
-                           (TO *)out, T_len, H, reverse, hdt);                                                      \
+                           (TO *)out, sg, H, reverse, hdt);                                                      \
         break
     switch (D) {
     GLA_STEPS_CASE(16);
@@ -148,11 +154,11 @@ int launch_recurrent_steps(hipStream_t st, int B, int T_len, int H, int D, int r
     return launch_status();
 }
 
-template int launch_recurrent_steps<__bf16, __bf16>(hipStream_t, int, int, int, int, int, int, const void *, const float *,
+template int launch_recurrent_steps<__bf16, __bf16>(hipStream_t, int, Segments, int, int, int, int, const void *, const float *,
                                                     const void *, const void *, const void *, void *, void *);
-template int launch_recurrent_steps<__bf16, float>(hipStream_t, int, int, int, int, int, int, const void *, const float *,
+template int launch_recurrent_steps<__bf16, float>(hipStream_t, int, Segments, int, int, int, int, const void *, const float *,
                                                    const void *, const void *, const void *, void *, void *);
-template int launch_recurrent_steps<float, float>(hipStream_t, int, int, int, int, int, int, const void *, const float *,
+template int launch_recurrent_steps<float, float>(hipStream_t, int, Segments, int, int, int, int, const void *, const float *,
                                                   const void *, const void *, const void *, void *, void *);
 
 }  // namespace gla

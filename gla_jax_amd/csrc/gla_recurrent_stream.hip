@@ -37,7 +37,7 @@ template <typename TO, int C, int D, bool STATE = false>
 __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const __bf16 *__restrict__ v,
     const __bf16 *__restrict__ k, const __bf16 *__restrict__ q, void *__restrict__ hT,
-    TO *__restrict__ out, int T_len, int H, int reverse, int hdt, int g_shift, float *__restrict__ gate_sums)
+    TO *__restrict__ out, Segments sg, int H, int reverse, int hdt, int g_shift, float *__restrict__ gate_sums)
 {
     typedef __bf16 T;
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4, NT = D / 16;
@@ -60,10 +60,12 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, c = lane >> 4;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int64_t seq = ((int64_t)b * T_len * H + h) * D;      // element offset of (b, t = 0, h)
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x;
+    const int64_t seq = (seg.row0 * H + h) * D;      // element offset of (b, t = 0, h)
     const int64_t rowstride = (int64_t)H * D;
-    const int64_t bh = (int64_t)b * H + h;
+    const int64_t bh = (int64_t)seg.index * H + h;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const int ptl = plain_tr_lane<T>(LS);
     const int wrow = 16 * w * LS + L.nat;          // this lane's row of a [token][feature] tile
@@ -131,8 +133,8 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
             // g_shift: a step takes the gate of the row g_shift rows further on in the array (the sequences of a
             // launch lie one behind the other).  Where the array ends the nearest row stands in: that step is the
             // first of its sequence, and its gate scales the zeros, or the initial state, it starts from.
-            int64_t gr = (int64_t)b * T_len + at + g_shift;
-            const int64_t last = (int64_t)gridDim.y * T_len - 1;
+            int64_t gr = seg.row0 + at + g_shift;
+            const int64_t last = (int64_t)gridDim.z * sg.T - 1;
             gr = gr < 0 ? 0 : (gr > last ? last : gr);
             growN = (gr * H + h) * D;
         }
@@ -312,7 +314,7 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
 }
 
 template <typename TO, int C, int D, bool STATE = false>
-static int launch_one(hipStream_t st, int B, int T_len, int H, int reverse, int hdt, const void *h0, const float *g,
+static int launch_one(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
                       const void *v, const void *k, const void *q, void *hT, void *out, int g_shift = 0,
                       float *gate_sums = nullptr)
 {
@@ -324,40 +326,40 @@ static int launch_one(hipStream_t st, int B, int T_len, int H, int reverse, int 
     auto kern = recurrent_stream_fwd_kernel<TO, C, D, STATE>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
-    dim3 grid(H, B), block(C * 4);
+    dim3 grid(H, sg.S, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, hT, (TO *)out,
-                       T_len, H, reverse, hdt, g_shift, gate_sums);
+                       sg, H, reverse, hdt, g_shift, gate_sums);
     return launch_status();
 }
 
 template <typename TO>
-int launch_recurrent_stream_fwd(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt,
+int launch_recurrent_stream_fwd(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt,
                                 const void *h0, const float *g, const void *v, const void *k, const void *q,
                                 void *hT, void *out)
 {
-    if (D == 64) return launch_one<TO, 128, 64>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, hT, out);
-    if (D == 128) return launch_one<TO, 64, 128>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, hT, out);
+    if (D == 64) return launch_one<TO, 128, 64>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, out);
+    if (D == 128) return launch_one<TO, 64, 128>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, out);
     return GLA_ERR_UNSUPPORTED;
 }
 
-int launch_recurrent_stream_state(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt, const void *h0,
+int launch_recurrent_stream_state(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, const void *h0,
                                  const float *g, const void *v, const void *k, const void *q, void *hT, int g_shift,
                                  float *gate_sums)
 {
     if (g_shift < -1 || g_shift > 1 || (g_shift && gate_sums)) return GLA_ERR_SHAPE;
     if (D == 64)
-        return launch_one<__bf16, 128, 64, true>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, hT, nullptr, g_shift,
+        return launch_one<__bf16, 128, 64, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, nullptr, g_shift,
                                                  gate_sums);
     if (D == 128)
-        return launch_one<__bf16, 64, 128, true>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, hT, nullptr, g_shift,
+        return launch_one<__bf16, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, nullptr, g_shift,
                                                  gate_sums);
     return GLA_ERR_UNSUPPORTED;
 }
 
-template int launch_recurrent_stream_fwd<__bf16>(hipStream_t, int, int, int, int, int, int, const void *,
+template int launch_recurrent_stream_fwd<__bf16>(hipStream_t, int, Segments, int, int, int, int, const void *,
                                                  const float *, const void *, const void *, const void *,
                                                  void *, void *);
-template int launch_recurrent_stream_fwd<float>(hipStream_t, int, int, int, int, int, int, const void *,
+template int launch_recurrent_stream_fwd<float>(hipStream_t, int, Segments, int, int, int, int, const void *,
                                                 const float *, const void *, const void *, const void *,
                                                 void *, void *);
 

@@ -29,7 +29,7 @@ template <typename TO, int C, int D, bool WIDE>
 __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k,
     const BT *__restrict__ q, const void *__restrict__ dhT, const TO *__restrict__ dout,
-    std::conditional_t<WIDE, float, BT> *__restrict__ dq, float *__restrict__ qdq, int T_len, int H, int reverse,
+    std::conditional_t<WIDE, float, BT> *__restrict__ dq, float *__restrict__ qdq, Segments sg, int H, int reverse,
     int hdt)
 {
     typedef BT T;
@@ -53,10 +53,12 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, c = lane >> 4;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int64_t seq = ((int64_t)b * T_len * H + h) * D;
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x;
+    const int64_t seq = (seg.row0 * H + h) * D;
     const int64_t rowstride = (int64_t)H * D;
-    const int64_t bh = (int64_t)b * H + h;
+    const int64_t bh = (int64_t)seg.index * H + h;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
     const int ptl = plain_tr_lane<T>(LS);
@@ -364,7 +366,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
     const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k, const BT *__restrict__ q,
     const void *__restrict__ dhT, const TO *__restrict__ dout, void *__restrict__ dh0,
     float *__restrict__ dg, std::conditional_t<WIDE, float, BT> *__restrict__ dv,
-    std::conditional_t<WIDE, float, BT> *__restrict__ dk, int T_len, int H, int reverse, int hdt)
+    std::conditional_t<WIDE, float, BT> *__restrict__ dk, Segments sg, int H, int reverse, int hdt)
 {
     typedef BT T;
     typedef std::conditional_t<WIDE, float, BT> TG;
@@ -392,10 +394,12 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, c = lane >> 4;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int64_t seq = ((int64_t)b * T_len * H + h) * D;
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x;
+    const int64_t seq = (seg.row0 * H + h) * D;
     const int64_t rowstride = (int64_t)H * D;
-    const int64_t bh = (int64_t)b * H + h;
+    const int64_t bh = (int64_t)seg.index * H + h;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
     const int ptl = plain_tr_lane<T>(LS);
@@ -791,7 +795,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
 }
 
 template <typename TO, int C, int D, bool WIDE>
-static int launch_dq(hipStream_t st, int B, int T_len, int H, int reverse, int hdt, const void *h0, const float *g,
+static int launch_dq(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
                      const void *v, const void *k, const void *q, const void *dhT, const void *dout, void *dq,
                      float *qdq)
 {
@@ -803,14 +807,14 @@ static int launch_dq(hipStream_t st, int B, int T_len, int H, int reverse, int h
     auto kern = recurrent_stream_dq_kernel<TO, C, D, WIDE>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
-    dim3 grid(H, B), block(C * 4);
+    dim3 grid(H, sg.S, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q,
-                       dhT, (const TO *)dout, (std::conditional_t<WIDE, float, T> *)dq, qdq, T_len, H, reverse, hdt);
+                       dhT, (const TO *)dout, (std::conditional_t<WIDE, float, T> *)dq, qdq, sg, H, reverse, hdt);
     return launch_status();
 }
 
 template <typename TO, int C, int D, bool WIDE>
-static int launch_rev(hipStream_t st, int B, int T_len, int H, int reverse, int hdt, const float *g, const void *v,
+static int launch_rev(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const float *g, const void *v,
                       const void *k, const void *q, const void *dhT, const void *dout, void *dh0,
                       float *dg, void *dv, void *dk)
 {
@@ -823,43 +827,43 @@ static int launch_rev(hipStream_t st, int B, int T_len, int H, int reverse, int 
     auto kern = recurrent_stream_rev_kernel<TO, C, D, WIDE>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
-    dim3 grid(H, B), block(C * 4);
+    dim3 grid(H, sg.S, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q,
                        dhT, (const TO *)dout, dh0, dg, (std::conditional_t<WIDE, float, T> *)dv,
-                       (std::conditional_t<WIDE, float, T> *)dk, T_len, H, reverse, hdt);
+                       (std::conditional_t<WIDE, float, T> *)dk, sg, H, reverse, hdt);
     return launch_status();
 }
 
-int launch_recurrent_stream_rev(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt, int dout_f32,
+int launch_recurrent_stream_rev(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, int dout_f32,
                                 const float *g, const void *v, const void *k, const void *q, const void *dhT,
                                 const void *dout, void *dh0, float *dg, void *dv, void *dk, int wide)
 {
     if (D == 64 && !wide)
-        return launch_recurrent_stream_rev2(st, B, T_len, H, D, reverse, hdt, dout_f32, g, v, k, q, dhT, dout, dh0, dg,
+        return launch_recurrent_stream_rev2(st, B, sg, H, D, reverse, hdt, dout_f32, g, v, k, q, dhT, dout, dh0, dg,
                                             dv, dk);
     if (D != 128) return GLA_ERR_UNSUPPORTED;
     if (wide)
         return dout_f32
-                   ? launch_rev<float, 64, 128, true>(st, B, T_len, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
-                   : launch_rev<BT, 64, 128, true>(st, B, T_len, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
-    return dout_f32 ? launch_rev<float, 64, 128, false>(st, B, T_len, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
-                    : launch_rev<BT, 64, 128, false>(st, B, T_len, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
+                   ? launch_rev<float, 64, 128, true>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
+                   : launch_rev<BT, 64, 128, true>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
+    return dout_f32 ? launch_rev<float, 64, 128, false>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
+                    : launch_rev<BT, 64, 128, false>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
 }
 
-int launch_recurrent_stream_dq(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt, int dout_f32,
+int launch_recurrent_stream_dq(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, int dout_f32,
                                const void *h0, const float *g, const void *v, const void *k, const void *q,
                                const void *dhT, const void *dout, void *dq, float *qdq, int wide)
 {
     if (D == 64 && !wide)
-        return launch_recurrent_stream_dq2(st, B, T_len, H, D, reverse, hdt, dout_f32, h0, g, v, k, q, dhT, dout, dq,
+        return launch_recurrent_stream_dq2(st, B, sg, H, D, reverse, hdt, dout_f32, h0, g, v, k, q, dhT, dout, dq,
                                            qdq);
     if (D != 128) return GLA_ERR_UNSUPPORTED;
     if (wide)
         return dout_f32
-                   ? launch_dq<float, 64, 128, true>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
-                   : launch_dq<BT, 64, 128, true>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
-    return dout_f32 ? launch_dq<float, 64, 128, false>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
-                    : launch_dq<BT, 64, 128, false>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
+                   ? launch_dq<float, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
+                   : launch_dq<BT, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
+    return dout_f32 ? launch_dq<float, 64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
+                    : launch_dq<BT, 64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
 }
 
 }  // namespace gla

@@ -25,7 +25,7 @@ template <typename TO, int C, int D>
 __global__ __launch_bounds__(C * 8) void recurrent_stream_dq2_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k,
     const BT *__restrict__ q, const void *__restrict__ dhT, const TO *__restrict__ dout, BT *__restrict__ dq,
-    float *__restrict__ qdq, int T_len, int H, int reverse, int hdt)
+    float *__restrict__ qdq, Segments sg, int H, int reverse, int hdt)
 {
     typedef BT T;
     constexpr int NB = C / 16, NW = 2 * NB, KS = D / 32, NT = D / 16;
@@ -52,10 +52,12 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_dq2_kernel(
     const int I = W < NB ? W : NW - 1 - W;         // the wave's sub-block
     const int fo = W < NB ? 0 : 32;                // ... and its first feature
     const int r = lane & 15, c = lane >> 4;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int64_t seq = ((int64_t)b * T_len * H + h) * D;
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x;
+    const int64_t seq = (seg.row0 * H + h) * D;
     const int64_t rowstride = (int64_t)H * D;
-    const int64_t bh = (int64_t)b * H + h;
+    const int64_t bh = (int64_t)seg.index * H + h;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
     const int ptl = plain_tr_lane<T>(LS);
@@ -399,7 +401,7 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_dq2_kernel(
 }
 
 template <typename TO, int C, int D>
-static int launch_dq2(hipStream_t st, int B, int T_len, int H, int reverse, int hdt, const void *h0, const float *g,
+static int launch_dq2(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
                       const void *v, const void *k, const void *q, const void *dhT, const void *dout, void *dq,
                       float *qdq)
 {
@@ -412,9 +414,9 @@ static int launch_dq2(hipStream_t st, int B, int T_len, int H, int reverse, int 
     auto kern = recurrent_stream_dq2_kernel<TO, C, D>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
-    dim3 grid(H, B), block(C * 8);
+    dim3 grid(H, sg.S, B), block(C * 8);
     hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q,
-                       dhT, (const TO *)dout, (T *)dq, qdq, T_len, H, reverse, hdt);
+                       dhT, (const TO *)dout, (T *)dq, qdq, sg, H, reverse, hdt);
     return launch_status();
 }
 
@@ -428,7 +430,7 @@ template <typename TO, int C, int D>
 __global__ __launch_bounds__(C * 8) void recurrent_stream_rev2_kernel(
     const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k, const BT *__restrict__ q,
     const void *__restrict__ dhT, const TO *__restrict__ dout, void *__restrict__ dh0,
-    float *__restrict__ dg, BT *__restrict__ dv, BT *__restrict__ dk, int T_len, int H, int reverse, int hdt)
+    float *__restrict__ dg, BT *__restrict__ dv, BT *__restrict__ dk, Segments sg, int H, int reverse, int hdt)
 {
     typedef BT T;
     constexpr int NB = C / 16, NW = 2 * NB, KS = D / 32, NT = D / 16;
@@ -461,10 +463,12 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev2_kernel(
     const int fo = W < NB ? 0 : 32;                // ... and its first feature
     const int PW = NW - 1 - W;                     // the wave with the other half of the sub-block
     const int r = lane & 15, c = lane >> 4;
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int64_t seq = ((int64_t)b * T_len * H + h) * D;
+    const SegmentRows seg(sg, blockIdx.z, blockIdx.y);
+    const int T_len = seg.len;
+    const int h = blockIdx.x;
+    const int64_t seq = (seg.row0 * H + h) * D;
     const int64_t rowstride = (int64_t)H * D;
-    const int64_t bh = (int64_t)b * H + h;
+    const int64_t bh = (int64_t)seg.index * H + h;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
     const int ptl = plain_tr_lane<T>(LS);
@@ -877,7 +881,7 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev2_kernel(
 }
 
 template <typename TO, int C, int D>
-static int launch_rev2(hipStream_t st, int B, int T_len, int H, int reverse, int hdt, const float *g, const void *v,
+static int launch_rev2(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const float *g, const void *v,
                        const void *k, const void *q, const void *dhT, const void *dout, void *dh0, float *dg,
                        void *dv, void *dk)
 {
@@ -890,29 +894,29 @@ static int launch_rev2(hipStream_t st, int B, int T_len, int H, int reverse, int
     auto kern = recurrent_stream_rev2_kernel<TO, C, D>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
-    dim3 grid(H, B), block(C * 8);
+    dim3 grid(H, sg.S, B), block(C * 8);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q, dhT,
-                       (const TO *)dout, dh0, dg, (T *)dv, (T *)dk, T_len, H, reverse, hdt);
+                       (const TO *)dout, dh0, dg, (T *)dv, (T *)dk, sg, H, reverse, hdt);
     return launch_status();
 }
 
-int launch_recurrent_stream_rev2(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt, int dout_f32,
+int launch_recurrent_stream_rev2(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, int dout_f32,
                                  const float *g, const void *v, const void *k, const void *q, const void *dhT,
                                  const void *dout, void *dh0, float *dg, void *dv, void *dk)
 {
     if (D == 64 && dout_f32)
-        return launch_rev2<float, 64, 64>(st, B, T_len, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
-    if (D == 64) return launch_rev2<BT, 64, 64>(st, B, T_len, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
+        return launch_rev2<float, 64, 64>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
+    if (D == 64) return launch_rev2<BT, 64, 64>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
     return GLA_ERR_UNSUPPORTED;
 }
 
-int launch_recurrent_stream_dq2(hipStream_t st, int B, int T_len, int H, int D, int reverse, int hdt, int dout_f32,
+int launch_recurrent_stream_dq2(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, int dout_f32,
                                 const void *h0, const float *g, const void *v, const void *k, const void *q,
                                 const void *dhT, const void *dout, void *dq, float *qdq)
 {
     if (D == 64 && dout_f32)
-        return launch_dq2<float, 64, 64>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
-    if (D == 64) return launch_dq2<BT, 64, 64>(st, B, T_len, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
+        return launch_dq2<float, 64, 64>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
+    if (D == 64) return launch_dq2<BT, 64, 64>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
     return GLA_ERR_UNSUPPORTED;
 }
 
