@@ -5,6 +5,7 @@ wrapper raises on a non-zero status."""
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -66,6 +67,22 @@ def load():
                           "(`python -m gla_jax_amd.build`)")
     _lib = lib
     return lib
+
+
+_binding = None
+
+
+def binding():
+    """The native host side of the torch entry points (csrc/gla_torch.cpp), loaded once, behind the library."""
+    global _binding
+    if _binding is None:
+        load()
+        try:
+            _binding = importlib.import_module("gla_jax_amd._gla_torch")
+        except ImportError as e:
+            raise ImportError("the torch binding is missing or does not fit this torch: build it with "
+                              "`python -m gla_jax_amd.build`.  There is no fallback path.") from e
+    return _binding
 
 
 def status_string(status: int) -> str:

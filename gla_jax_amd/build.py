@@ -1,6 +1,6 @@
-"""Builds libgla_hip.so (hand-written HIP for gfx950) in-tree with hipcc.
+"""Builds libgla_hip.so (hand-written HIP for gfx950) and the torch binding in-tree, with hipcc and g++.
 
-    python -m gla_jax_amd.build            # compile every csrc/*.hip and link
+    python -m gla_jax_amd.build            # compile every csrc/*.hip and link, then csrc/gla_torch.cpp
 """
 from __future__ import annotations
 
@@ -13,6 +13,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgla_hip.so")
+BINDING = os.path.join(HERE, "_gla_torch.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # packed fp32 VALU ops are switched off for all device code (some of their forms have produced
@@ -48,6 +49,26 @@ def build(verbose: bool = True) -> str:
     return LIB
 
 
+def build_torch_binding(verbose: bool = True) -> str:
+    """Compiles the native host side of the Python entry points (csrc/gla_torch.cpp) against the installed torch and
+    links it with libgla_hip.so, which has to be built."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    inc = cpp_extension.include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-I{i}" for i in inc], os.path.join(CSRC, "gla_torch.cpp"), "-o", BINDING, "-L", HERE, "-lgla_hip", "-L", lib,
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("the torch binding failed to build:\n" + r.stderr)
+    if verbose:
+        print(f"built {BINDING}")
+    return BINDING
+
+
 def jaxlib_include():
     """Directory holding xla/ffi/api/ffi.h (shipped inside jaxlib), or None."""
     try:
@@ -81,4 +102,5 @@ def build_xla_ffi(verbose: bool = True):
 
 if __name__ == "__main__":
     build()
+    build_torch_binding()
     build_xla_ffi()

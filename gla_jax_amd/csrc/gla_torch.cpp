@@ -1,0 +1,335 @@
+// The host side of the Python entry points for arrays that are already as the kernels take them (on the GPU, dense, one
+// element type): argument checks, buffers, launches and the autograd rules in one native call.  The same path in Python
+// took 23 us for a forward and 105 to 210 us for a forward and backward, more than the kernels of a small call; here it
+// is about a third of that.  Everything else (other layouts and types, function transforms, error messages) stays in
+// gla.py, which calls this again once the arrays are converted.
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_like.h>
+#include <ATen/ops/zeros.h>
+#include <ATen/ops/zeros_like.h>
+#include <c10/core/DeviceGuard.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <optional>
+
+#include "../../include/gla_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// A status of the library, raised as gla_jax_amd._lib.GlaError where Python can see it.
+struct GlaFailure : std::runtime_error {
+    const char *fn;
+    int status;
+    GlaFailure(const char *f, int s)
+        : std::runtime_error(std::string(f) + " failed with status " + std::to_string(s) + ": " + gla_status_string(s)),
+          fn(f), status(s)
+    {
+    }
+};
+void check(const char *fn, int status)
+{
+    if (status != 0) throw GlaFailure(fn, status);
+}
+
+void *stream_of(const Tensor &t)
+{
+    return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
+}
+
+bool known(at::ScalarType s) { return s == at::kFloat || s == at::kBFloat16; }
+gla_dtype code(const Tensor &t) { return t.scalar_type() == at::kFloat ? GLA_F32 : GLA_BF16; }
+bool dense_on_gpu(const Tensor &t) { return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.is_contiguous(); }
+
+struct Dims {
+    int64_t B, T, H, D;
+};
+Dims dims_of(const Tensor &k)
+{
+    const auto s = k.sizes();
+    const size_t n = s.size();
+    int64_t B = 1;
+    for (size_t i = 0; i + 3 < n; ++i) B *= s[i];
+    return {B, s[n - 3], s[n - 2], s[n - 1]};
+}
+
+// The arrays can go to the kernels as they are: see gla.py's _prep for the contract.
+bool canonical(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q)
+{
+    for (const Tensor *t : {&h0, &g, &v, &k, &q})
+        if (!dense_on_gpu(*t) || t->device() != k.device()) return false;
+    const auto s = k.sizes();
+    const size_t n = s.size();
+    if (n < 3 || q.sizes() != s || g.sizes() != s || v.sizes() != s) return false;
+    if (g.scalar_type() != at::kFloat || !known(h0.scalar_type()) || !known(v.scalar_type())) return false;
+    if (k.scalar_type() != v.scalar_type() || q.scalar_type() != v.scalar_type()) return false;
+    const auto hs = h0.sizes();
+    if (hs.size() != n || hs[n - 1] != s[n - 1] || hs[n - 2] != s[n - 1] || hs[n - 3] != s[n - 2]) return false;
+    for (size_t i = 0; i + 3 < n; ++i)
+        if (hs[i] != s[i]) return false;
+    return true;
+}
+
+Tensor bytes_like(size_t n, const Tensor &t) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
+
+[[noreturn]] void no_double_backward(const char *name)
+{
+    TORCH_CHECK_NOT_IMPLEMENTED(false, name, ": second-order gradients are not provided (the reference defines first-order "
+                                             "custom_vjp rules only)");
+    std::abort();
+}
+
+bool wants_grad(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q)
+{
+    return at::GradMode::is_enabled() && (h0.requires_grad() || g.requires_grad() || v.requires_grad() ||
+                                          k.requires_grad() || q.requires_grad());
+}
+
+// ---- chunk_gla ----------------------------------------------------------------------------------
+struct ChunkOut {
+    Tensor hT, out, states;
+};
+ChunkOut chunk_forward(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q, int64_t chunk,
+                       bool residual)
+{
+    const c10::DeviceGuard guard(k.device());
+    const Dims d = dims_of(k);
+    const gla_dtype dt = code(v);
+    const size_t nws = gla_chunk_fwd_workspace_bytes(d.B, d.T, d.H, d.D, d.D, chunk, dt);
+    const size_t nst = residual ? gla_chunk_states_bytes(d.B, d.T, d.H, d.D, d.D, chunk, dt) : 0;
+    if (nws == 0) check("gla_chunk_fwd", GLA_ERR_UNSUPPORTED);
+    ChunkOut r{at::empty_like(h0), at::empty_like(v), residual ? bytes_like(nst, v) : Tensor()};
+    const Tensor ws = bytes_like(nws, v);
+    check("gla_chunk_fwd",
+          gla_chunk_fwd(stream_of(k), d.B, d.T, d.H, d.D, d.D, chunk, dt, code(h0), h0.data_ptr(), (const float *)g.data_ptr(),
+                        v.data_ptr(), k.data_ptr(), q.data_ptr(), r.hT.data_ptr(), r.out.data_ptr(),
+                        residual ? r.states.data_ptr() : nullptr, ws.data_ptr(), nws));
+    return r;
+}
+
+variable_list chunk_backward(const Tensor &states, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q,
+                             const Tensor &dhT, const Tensor &dout, int64_t chunk)
+{
+    const c10::DeviceGuard guard(k.device());
+    const Dims d = dims_of(k);
+    const gla_dtype dt = code(v);
+    const size_t nws = gla_chunk_bwd_workspace_bytes(d.B, d.T, d.H, d.D, d.D, chunk, dt);
+    const Tensor ws = bytes_like(nws, v);
+    Tensor dh0 = at::empty_like(dhT), dg = at::empty_like(g), dv = at::empty_like(v), dk = at::empty_like(k),
+           dq = at::empty_like(q);
+    check("gla_chunk_bwd",
+          gla_chunk_bwd(stream_of(k), d.B, d.T, d.H, d.D, d.D, chunk, dt, code(dhT), (const float *)g.data_ptr(), v.data_ptr(),
+                        k.data_ptr(), q.data_ptr(), states.data_ptr(), dhT.data_ptr(), dout.data_ptr(), dh0.data_ptr(),
+                        (float *)dg.data_ptr(), dv.data_ptr(), dk.data_ptr(), dq.data_ptr(), ws.data_ptr(), nws));
+    return {dh0, dg, dv, dk, dq};
+}
+
+// a cotangent as the kernels take it: zeros where autograd has none, dense, in the type of what it belongs to
+Tensor cotangent(const Tensor &d, at::IntArrayRef sizes, at::ScalarType type, const Tensor &like)
+{
+    if (!d.defined()) return at::zeros(sizes, like.options().dtype(type));
+    return d.to(type).contiguous();
+}
+std::vector<int64_t> state_sizes(const Tensor &k)
+{
+    std::vector<int64_t> s = k.sizes().vec();
+    const size_t n = s.size();
+    s[n - 3] = s[n - 2];
+    s[n - 2] = s[n - 1];
+    return s;
+}
+
+// The backward rules as functions of their own, used where a graph of the gradients is asked for: what they return can
+// be differentiated no further, and says so.
+struct ChunkBackward : torch::autograd::Function<ChunkBackward> {
+    static variable_list forward(AutogradContext *, const Tensor &states, const Tensor &g, const Tensor &v, const Tensor &k,
+                                 const Tensor &q, const Tensor &dhT, const Tensor &dout, int64_t chunk)
+    {
+        return chunk_backward(states, g, v, k, q, dhT, dout, chunk);
+    }
+    static variable_list backward(AutogradContext *, variable_list) { no_double_backward("chunk_gla"); }
+};
+
+struct Chunk : torch::autograd::Function<Chunk> {      // gla.py:483-550, 552-625
+    static variable_list forward(AutogradContext *ctx, const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k,
+                                 const Tensor &q, int64_t chunk)
+    {
+        ChunkOut r = chunk_forward(h0, g, v, k, q, chunk, true);
+        ctx->save_for_backward({r.states, g, v, k, q});      // residuals of gla.py:542-549
+        ctx->saved_data["chunk"] = chunk;
+        ctx->saved_data["hidden"] = (int64_t)h0.scalar_type();
+        ctx->set_materialize_grads(false);
+        return {r.hT, r.out};
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list d)
+    {
+        const auto s = ctx->get_saved_variables();
+        const int64_t chunk = ctx->saved_data["chunk"].toInt();
+        const Tensor dhT = cotangent(d[0], state_sizes(s[3]), (at::ScalarType)ctx->saved_data["hidden"].toInt(), s[3]);
+        const Tensor dout = cotangent(d[1], s[2].sizes(), s[2].scalar_type(), s[2]);
+        variable_list r = at::GradMode::is_enabled() ? ChunkBackward::apply(s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk)
+                                                     : chunk_backward(s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk);
+        r.emplace_back();
+        return r;
+    }
+};
+
+// ---- recurrent_gla ------------------------------------------------------------------------------
+std::pair<Tensor, Tensor> recurrent_forward(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k,
+                                            const Tensor &q, bool reverse, bool out_fp32)
+{
+    const c10::DeviceGuard guard(k.device());
+    const Dims d = dims_of(k);
+    const gla_dtype dt = code(v);
+    Tensor hT = at::empty_like(h0), out = out_fp32 ? at::empty_like(v, v.options().dtype(at::kFloat)) : at::empty_like(v), ws;
+    // a workspace where the library can use one (head dimension 256, few sequences)
+    const size_t nws = gla_recurrent_fwd_workspace_bytes(d.B, d.T, d.H, d.D, d.D, dt);
+    if (nws) ws = bytes_like(nws, v);
+    check("gla_recurrent_fwd_ws",
+          gla_recurrent_fwd_ws(stream_of(k), d.B, d.T, d.H, d.D, d.D, dt, code(h0), out_fp32 ? GLA_F32 : dt, reverse,
+                               h0.data_ptr(), (const float *)g.data_ptr(), v.data_ptr(), k.data_ptr(), q.data_ptr(),
+                               hT.data_ptr(), out.data_ptr(), nws ? ws.data_ptr() : nullptr, nws));
+    return {hT, out};
+}
+
+variable_list recurrent_backward(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q,
+                                 const Tensor &hT, const Tensor &dhT, const Tensor &dout, bool reverse, bool out_fp32)
+{
+    const c10::DeviceGuard guard(k.device());
+    const Dims d = dims_of(k);
+    const gla_dtype dt = code(v);
+    Tensor dh0 = at::empty_like(h0), dg = at::empty_like(g), dv = at::empty_like(v), dk = at::empty_like(k),
+           dq = at::empty_like(q), ws;
+    const size_t nws = gla_recurrent_bwd_workspace_bytes(d.B, d.T, d.H, d.D, d.D, dt);
+    if (nws) ws = bytes_like(nws, v);
+    check("gla_recurrent_bwd_ws",
+          gla_recurrent_bwd_ws(stream_of(k), d.B, d.T, d.H, d.D, d.D, dt, code(h0), out_fp32 ? GLA_F32 : dt, reverse,
+                               h0.data_ptr(), (const float *)g.data_ptr(), v.data_ptr(), k.data_ptr(), q.data_ptr(),
+                               hT.data_ptr(), dhT.data_ptr(), dout.data_ptr(), dh0.data_ptr(), (float *)dg.data_ptr(),
+                               dv.data_ptr(), dk.data_ptr(), dq.data_ptr(), nws ? ws.data_ptr() : nullptr, nws));
+    return {dh0, dg, dv, dk, dq};
+}
+
+struct RecurrentBackward : torch::autograd::Function<RecurrentBackward> {
+    static variable_list forward(AutogradContext *, const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k,
+                                 const Tensor &q, const Tensor &hT, const Tensor &dhT, const Tensor &dout, bool reverse,
+                                 bool out_fp32)
+    {
+        return recurrent_backward(h0, g, v, k, q, hT, dhT, dout, reverse, out_fp32);
+    }
+    static variable_list backward(AutogradContext *, variable_list) { no_double_backward("recurrent_gla"); }
+};
+
+struct Recurrent : torch::autograd::Function<Recurrent> {      // gla.py:99-170, 172-269
+    static variable_list forward(AutogradContext *ctx, const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k,
+                                 const Tensor &q, bool reverse, bool out_fp32)
+    {
+        auto [hT, out] = recurrent_forward(h0, g, v, k, q, reverse, out_fp32);
+        ctx->save_for_backward({h0, g, v, k, q, hT});          // residuals of gla.py:169
+        ctx->saved_data["reverse"] = reverse;
+        ctx->saved_data["out_fp32"] = out_fp32;
+        ctx->set_materialize_grads(false);
+        return {hT, out};
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list d)
+    {
+        const auto s = ctx->get_saved_variables();
+        const bool reverse = ctx->saved_data["reverse"].toBool(), out_fp32 = ctx->saved_data["out_fp32"].toBool();
+        const Tensor dhT = cotangent(d[0], s[0].sizes(), s[0].scalar_type(), s[0]);
+        const Tensor dout = cotangent(d[1], s[2].sizes(), out_fp32 ? at::kFloat : s[2].scalar_type(), s[2]);
+        variable_list r = at::GradMode::is_enabled()
+                              ? RecurrentBackward::apply(s[0], s[1], s[2], s[3], s[4], s[5], dhT, dout, reverse, out_fp32)
+                              : recurrent_backward(s[0], s[1], s[2], s[3], s[4], s[5], dhT, dout, reverse, out_fp32);
+        r.resize(7);
+        return r;
+    }
+};
+
+// ---- module -------------------------------------------------------------------------------------
+typedef std::optional<std::vector<Tensor>> Result;       // none: not for this path
+
+Result chunk(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q, int64_t size)
+{
+    if (!canonical(h0, g, v, k, q) || size <= 0 || (size & (size - 1)) || dims_of(k).T % size) return std::nullopt;
+    if (wants_grad(h0, g, v, k, q)) return Chunk::apply(h0, g, v, k, q, size);
+    ChunkOut r = chunk_forward(h0, g, v, k, q, size, false);
+    return std::vector<Tensor>{r.hT, r.out};
+}
+
+Result recurrent(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q, bool reverse,
+                 bool out_fp32)
+{
+    if (!canonical(h0, g, v, k, q) || k.size(-1) < 16) return std::nullopt;
+    if (wants_grad(h0, g, v, k, q)) return Recurrent::apply(h0, g, v, k, q, reverse, out_fp32);
+    auto [hT, out] = recurrent_forward(h0, g, v, k, q, reverse, out_fp32);
+    return std::vector<Tensor>{hT, out};
+}
+
+bool plain_f32(const Tensor &t) { return dense_on_gpu(t) && t.scalar_type() == at::kFloat; }
+
+std::optional<Tensor> cumsum(const Tensor &src, int64_t axis, const std::optional<Tensor> &init, bool reverse)
+{
+    const int64_t n = src.dim();
+    if (!plain_f32(src) || axis < 0 || axis >= n) return std::nullopt;
+    int64_t outer = 1, inner = 1;
+    for (int64_t i = 0; i < axis; ++i) outer *= src.size(i);
+    for (int64_t i = axis + 1; i < n; ++i) inner *= src.size(i);
+    if (outer > 65535) return std::nullopt;
+    if (init) {
+        if (!plain_f32(*init) || init->dim() != n - 1 || init->device() != src.device()) return std::nullopt;
+        for (int64_t i = 0; i < n - 1; ++i)
+            if (init->size(i) != src.size(i < axis ? i : i + 1)) return std::nullopt;
+    }
+    const c10::DeviceGuard guard(src.device());
+    Tensor dst = at::empty_like(src);
+    check("gla_cumsum_f32", gla_cumsum_f32(stream_of(src), (const float *)src.data_ptr(),
+                                           init ? (const float *)init->data_ptr() : nullptr, (float *)dst.data_ptr(), outer,
+                                           src.size(axis), inner, reverse));
+    return dst;
+}
+
+std::optional<std::pair<Tensor, Tensor>> rnn(const Tensor &a, const Tensor &b, const std::optional<Tensor> &ia,
+                                             const std::optional<Tensor> &ib, bool reverse)
+{
+    const int64_t n = b.dim();
+    if (!plain_f32(a) || !plain_f32(b) || (n != 3 && n != 4) || a.dim() != n - 1 || a.device() != b.device()) return std::nullopt;
+    for (int64_t i = 0; i < n - 1; ++i)
+        if (a.size(i) != b.size(i)) return std::nullopt;
+    if ((bool)ia != (bool)ib) return std::nullopt;
+    const int64_t B = n == 4 ? b.size(0) : 1, T = b.size(n - 3), K = b.size(n - 2), V = b.size(n - 1);
+    // the initial pair is read as B rows of K (and K x V) whatever its shape: the number of values is what has to fit
+    if (ia && (!plain_f32(*ia) || !plain_f32(*ib) || ia->numel() != B * K || ib->numel() != B * K * V ||
+               ia->device() != b.device() || ib->device() != b.device()))
+        return std::nullopt;
+    const c10::DeviceGuard guard(b.device());
+    Tensor oa = at::empty_like(a), ox = at::empty_like(b);
+    check("gla_rnn_scan_f32",
+          gla_rnn_scan_f32(stream_of(b), (const float *)a.data_ptr(), (const float *)b.data_ptr(),
+                           ia ? (const float *)ia->data_ptr() : nullptr, ib ? (const float *)ib->data_ptr() : nullptr,
+                           (float *)oa.data_ptr(), (float *)ox.data_ptr(), B, T, K, V, reverse));
+    return std::make_pair(oa, ox);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_gla_torch, m)
+{
+    static py::handle error = py::object(py::module_::import("gla_jax_amd._lib").attr("GlaError")).release();
+    py::register_exception_translator([](std::exception_ptr p) {
+        try {
+            if (p) std::rethrow_exception(p);
+        } catch (const GlaFailure &e) {
+            PyErr_SetObject(error.ptr(), py::object(error(e.fn, e.status, gla_status_string(e.status))).ptr());
+        }
+    });
+    typedef py::call_guard<py::gil_scoped_release> NoGil;
+    m.def("chunk", &chunk, NoGil());
+    m.def("recurrent", &recurrent, NoGil());
+    m.def("cumsum", &cumsum, NoGil());
+    m.def("rnn", &rnn, NoGil());
+}

@@ -4,7 +4,8 @@
 (hidden_init, log_fgate, value, key, query, ...), shapes and dtype rules of gla.py:657-692,
 405-439 and 26-47 of zhixuan-lin/gla-jax.  Arrays are torch tensors on the GPU; the forward and
 backward rules of the reference's `jax.custom_vjp` (gla.py:628-655, 362-388, 441) are
-`torch.autograd.Function`s whose bodies are single calls into libgla_hip.so.  Batching: the
+autograd functions whose bodies are single calls into libgla_hip.so: native ones (csrc/gla_torch.cpp) where no function
+transform is active, the Python ones below where one is.  Batching: the
 reference uses `jax.vmap` over a leading axis of all five arrays (gla.py:1335); here any number of
 leading axes may simply be present, and `torch.func.vmap` works through the functions' vmap rule.
 
@@ -78,7 +79,7 @@ def _as(t, shape, dtype):
     return t.reshape(shape).to(dtype).contiguous()
 
 
-_transforms_active = getattr(torch._C, "_are_functorch_transforms_active", None)
+_transforms_active = getattr(torch._C, "_are_functorch_transforms_active", None) or (lambda: True)
 
 
 def _twin(cls):
@@ -99,9 +100,15 @@ def _twin(cls):
 
 
 def _apply(cls, *args):
-    if _transforms_active is None or _transforms_active():
-        return cls.apply(*args)
-    return cls._twin.apply(*args)
+    return (cls if _transforms_active() else cls._twin).apply(*args)
+
+
+def _native(entry, arrays, *args):
+    """One call of the native host side (csrc/gla_torch.cpp), which allocates, launches and keeps the autograd rule.
+    None: the arrays are not as the kernels take them (`_prep` makes them so, or says what is wrong)."""
+    if not all(isinstance(t, torch.Tensor) for t in arrays):
+        return None
+    return getattr(_lib.binding(), entry)(*arrays, *args)
 
 
 def _merge_mapped(info, in_dims, tensors):
@@ -241,6 +248,11 @@ def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_
     if interpret:
         raise ValueError("interpret=True asks for the reference's CPU interpreter; this build has no CPU path")
     chunk_size = int(chunk_size)
+    native = not _transforms_active()
+    if native:
+        done = _native("chunk", (hidden_init, log_fgate, value, key, query), chunk_size)
+        if done is not None:
+            return tuple(done)
     (h0, g, v, k, q), lead, (B, T, H, DK, DV) = _prep(hidden_init, log_fgate, value, key, query)
     if DK != DV:
         raise AssertionError("chunk_gla needs key and value head dims to be equal")   # gla.py:499
@@ -248,11 +260,8 @@ def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_
         raise AssertionError(f"Chunk length must be power of 2, but got {chunk_size}")  # gla.py:500
     if T % chunk_size:
         raise AssertionError(f"sequence length {T} is not a multiple of chunk_size {chunk_size}")
-    if _transforms_active is not None and not _transforms_active() and not (
-            torch.is_grad_enabled() and any(t.requires_grad for t in (h0, g, v, k, q))):
-        hT, out, _ = _chunk_forward(h0, g, v, k, q, chunk_size, False)
-    else:
-        hT, out = _apply(_ChunkGLA, h0, g, v, k, q, chunk_size)[:2]
+    hT, out = (_native("chunk", (h0, g, v, k, q), chunk_size) if native
+               else _ChunkGLA.apply(h0, g, v, k, q, chunk_size)[:2])
     return _as(hT, lead + (H, DK, DV), hidden_init.dtype), _as(out, lead + (T, H, DV), out.dtype)
 
 
@@ -346,6 +355,12 @@ class _RecurrentGLABwd(torch.autograd.Function):
 
 
 def _recurrent(hidden_init, log_fgate, value, key, query, reverse, out_fp32):
+    reverse = bool(reverse)
+    native = not _transforms_active()
+    if native:
+        done = _native("recurrent", (hidden_init, log_fgate, value, key, query), reverse, out_fp32)
+        if done is not None:
+            return tuple(done)
     (h0, g, v, k, q), lead, (B, T, H, DK, DV) = _prep(hidden_init, log_fgate, value, key, query)
     if DK != DV:
         raise AssertionError("Not supported yet: key and value head dims differ")      # gla.py:120, 391
@@ -357,7 +372,8 @@ def _recurrent(hidden_init, log_fgate, value, key, query, reverse, out_fp32):
         F = torch.nn.functional
         h0 = F.pad(h0, (0, pad, 0, pad))
         g, v, k, q = (F.pad(x, (0, pad)) for x in (g, v, k, q))
-    hT, out = _apply(_RecurrentGLA, h0, g, v, k, q, bool(reverse), bool(out_fp32))
+    hT, out = (_native("recurrent", (h0, g, v, k, q), reverse, out_fp32) if native
+               else _RecurrentGLA.apply(h0, g, v, k, q, reverse, out_fp32))
     if pad:
         hT, out = hT[..., :DK, :DV], out[..., :DV]
     return _as(hT, lead + (H, DK, DV), hidden_init.dtype), _as(out, lead + (T, H, DV), out.dtype)

@@ -28,8 +28,11 @@ def cumsum_recursive(src: torch.Tensor, axis: int, init: Optional[torch.Tensor] 
                      reverse: bool = False, block_size_t: int = 2048) -> torch.Tensor:
     """Inclusive cumulative sum of `src` along `axis` plus `init` (shape = src.shape without `axis`),
     from the far end when `reverse` (ops.py:234-284).  Computed in float32, returned in src.dtype."""
-    _require_cuda(src, init)
     axis = axis % src.ndim
+    done = _lib.binding().cumsum(src, axis, init, bool(reverse))      # float32, dense, on the GPU: the usual case
+    if done is not None:
+        return done
+    _require_cuda(src, init)
     pre, T, post = src.shape[:axis], src.shape[axis], src.shape[axis + 1:]
     if init is not None and tuple(init.shape) != tuple(pre + post):
         raise AssertionError(f"init shape {tuple(init.shape)} != {tuple(pre + post)}")   # ops.py:254
@@ -62,6 +65,9 @@ def rnn_recursive(log_fgate: torch.Tensor, kv: torch.Tensor,
     log_fgate [T,K] / kv [T,K,V] with optional initial pair, backwards in n when `reverse`
     (ops.py:396-456).  Returns (running sum of a, states), states in kv.dtype (ops.py:373-374).
     A leading batch axis on all arguments is accepted."""
+    done = _lib.binding().rnn(log_fgate, kv, init_log_fgate, init_kv, bool(reverse))
+    if done is not None:
+        return done
     _require_cuda(log_fgate, kv, init_log_fgate, init_kv)
     if (init_log_fgate is None) != (init_kv is None):
         raise AssertionError("init_log_fgate and init_kv go together")                   # ops.py:407
