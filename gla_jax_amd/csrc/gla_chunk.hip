@@ -10,12 +10,12 @@
 namespace gla {
 
 struct ChunkPlan {
-    int C = 0;       // tokens per workgroup actually used (a divisor of chunk_size)
+    int C = 0;       // tokens per workgroup (choose_tile)
     int D = 0;       // head dimension the kernels work on: DK, or 32 for DK = 16 (rows padded by zeros on the way in)
     size_t prod = 0, decay = 0, states = 0;   // byte sizes, each rounded up to 256
     size_t scale_off = 0;                     // where the products' exponents start inside the decay region
     int bwd_states = 2;                       // arrays of d(chunk-end state): one (tiled) for 16-bit data, both orientations for fp32
-    size_t resid = 0;                         // the forward residual: N + 1 states per (b,h), the last one final
+    size_t resid = 0;                         // the forward residual: N + 1 states per (b,h), the last one final, or more room
     // Head dimension 256 runs as two passes of the 128-feature kernels over 2H heads (gla_split.hip); the
     // sizes above are then those of one such pass, and:
     bool split = false;
@@ -36,11 +36,30 @@ struct ChunkPlan {
 
 static size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// The result does not depend on the chunk length (only its rounding does): chunk_size is checked as the
-// reference checks it, and the kernels then run with the largest compiled tile that divides T, whatever
-// size was asked for (at the headline shape a 64-token tile takes 1.5x, a 32-token tile 2.5x the time of
-// the 128-token one: twice or four times the chunk states).  Sizes below 32 tokens are refused: the leaf
-// of the reference needs 32 rows as well (gla.py:975-977).
+// The tile: tokens per workgroup, 128, 64 or 32 (fp32 data: 64 or 32 up to 64 features, 32 at 128).  The result does not
+// depend on it (only its rounding does), so whatever chunk_size asks for, the lengths and the number of sequences decide; a
+// tile need not divide T, the last one is filled up with zeros.  Wide tiles mean fewer chunk states to write, scan
+// and read; narrow ones more workgroups with less to do each while there are not enough for the 256 compute units.
+// Forward + backward, bf16, us per tile 128 / 64 / 32 (wg: workgroups of 64-token tiles):
+//   128 features  B4 T4096 H6 213 / 298 / 680    B4 T1056 H6 (408 wg) 81 / 101 / 130    B16 T160 H8 (384 wg) 87 / 99 / 121
+//                 B4 T512 H6 (192 wg) 76 / 62 / 73    B16 T96 H8 (256 wg) 80 / 69 / 75    B1 T160 H1 69 / 52 / 50
+//   64 features   B16 T2048 H8 242 / 269 / 385   B16 T1056 H8 (1152 against 1088 rows) 154 / 143 / 183
+//                 B4 T2048 H6 69 / 67 / 91   B1 T16384 H2 75 / 107 (a scan of 256 chunks)   B1 T2048 H1 43 / 37 / 43
+// and fp32, 64 features, 64 / 32: B4 T1056 H6 84 / 93, B1 T512 H2 45 / 39, B1 T2048 H2 51 / 52.
+static int64_t choose_tile(int64_t seqs, int64_t T, int64_t D, int dtype)
+{
+    auto tiles = [&](int64_t c) { return (T + c - 1) / c; };
+    constexpr int64_t kUnits = 256;                          // compute units
+    if (dtype == GLA_F32) return D > 64 || (T < 2048 && seqs * tiles(32) <= kUnits) ? 32 : 64;
+    if (T <= (D > 64 ? 256 : 576) && seqs * tiles(32) <= kUnits) return 32;
+    if (seqs * tiles(64) <= kUnits && tiles(64) <= (D >= 64 ? 64 : 32)) return 64;
+    // 64 features: where a 128-token tile would carry over 5 % more zeros
+    if (D == 64 && T <= 4096 && tiles(128) * 128 * 20 > tiles(64) * 64 * 21) return 64;
+    return 128;
+}
+
+// chunk_size is checked as the reference checks it.  Sizes below 32 tokens are refused: the leaf of the reference needs
+// 32 rows as well (gla.py:975-977).
 static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, int64_t chunk, int dtype,
                       ChunkPlan *plan, int hidden_dtype = GLA_BF16)
 {
@@ -61,9 +80,7 @@ static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, i
         plan->hid = round256((size_t)B * 2 * H * 128 * 128 * sizeof(float));
         return GLA_OK;
     }
-    // largest tile built: 128 tokens for bf16, for fp32 (tiles twice as wide) 64 at D<=64 and 32 at D=128
-    int64_t C = dtype == GLA_BF16 ? 128 : (DK > 64 ? 32 : 64);
-    while (T % C != 0) C /= 2;                               // chunk >= 32 divides T, so this stops at 32 or above
+    const int64_t C = choose_tile(B * H, T, DK, dtype);
     int Dk = 0;
 #define GLA_PLAN_CASE(T_, C_, D_, DM_) \
     if (((dtype == GLA_BF16) == (sizeof(T_) == 2)) && C == C_ && DK == DM_) Dk = D_;
@@ -72,7 +89,7 @@ static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, i
     if (!Dk) return GLA_ERR_UNSUPPORTED;
     plan->D = Dk;
     DK = DV = Dk;                                            // the library's own buffers are sized for the kernels' D
-    const size_t N = (size_t)(T / C);
+    const size_t N = (size_t)((T + C - 1) / C);
     if ((int64_t)N * H > 0x7fffffffLL) return GLA_ERR_SHAPE;   // chunks x heads is the grid's x extent
     const size_t esz = dtype == GLA_BF16 ? 2 : 4;
     plan->C = (int)C;
@@ -83,7 +100,11 @@ static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, i
     plan->decay = round256(plan->scale_off + (size_t)B * H * N * (DK * DV / 16));
     plan->states = round256((size_t)B * H * N * DK * DV * esz);
     plan->bwd_states = dtype == GLA_BF16 ? 1 : 2;
-    plan->resid = round256((size_t)B * H * (N + 1) * DK * DV * esz);
+    // the residual is handed out with room for the states of the largest tile that divides T, which callers may count on
+    int64_t Cd = dtype == GLA_BF16 ? 128 : (DK > 64 ? 32 : 64);
+    while (T % Cd != 0) Cd /= 2;
+    const size_t slots = 1 + (N > (size_t)(T / Cd) ? N : (size_t)(T / Cd));
+    plan->resid = round256((size_t)B * H * slots * DK * DV * esz);
     return GLA_OK;
 }
 
@@ -203,7 +224,7 @@ static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
     unsigned char *pexp = ws + p.prod + p.scale_off;
     void *ws_states = (void *)(ws + p.prod + p.decay);
     hipStream_t st = (hipStream_t)stream;
-    const int N = (int)(T / p.C);
+    const int N = (int)((T + p.C - 1) / p.C);
     // 16-bit data: ONE array of chunk-start states, tiled, read by the output kernel and (as the residual) by the
     // gradient kernel; without a residual to write it goes to the workspace.  fp32 data: the [dv][dk] copy for the
     // output kernel in the workspace beside the residual.
@@ -351,7 +372,7 @@ static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
     void *dstatesT = dtype == GLA_BF16 ? nullptr : (void *)(ws + p.prod + p.decay);
     void *dstatesN = (void *)(ws + p.prod + p.decay + (dtype == GLA_BF16 ? 0 : p.states));
     hipStream_t st = (hipStream_t)stream;
-    const int N = (int)(T / p.C);
+    const int N = (int)((T + p.C - 1) / p.C);
     return dispatch(dtype, p.C, (int)DK, [&](auto t, auto c, auto d, auto dm) -> int {
         typedef decltype(t) E;
         constexpr int C_ = decltype(c)::value, D_ = decltype(d)::value, DM_ = decltype(dm)::value;

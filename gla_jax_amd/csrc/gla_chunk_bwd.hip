@@ -68,9 +68,19 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
     // heads vary fastest over the grid: workgroups that run together touch the same DRAM pages of the
     // [B, T, H, D] arrays (a token's H rows are contiguous)
     const int h = blockIdx.x % H, n = blockIdx.x / H, b = blockIdx.y;
-    const int N = T_len / C;
+    const int N = (T_len + C - 1) / C;
+    const bool live = n * C + 16 * w < T_len;      // the wave has tokens (see rows_or_zeros)
     const int64_t tok = (int64_t)b * T_len + (int64_t)n * C + 16 * w + r;
-    const int64_t rowoff = (tok * H + h) * DM;     // DM features per row in memory (DM < D: see RowMap)
+    const int64_t rowoff = live ? (tok * H + h) * DM : 0;     // DM features per row in memory (DM < D: see RowMap)
+    g = rows_or_zeros(live, g);
+    v = rows_or_zeros(live, v);
+    k = rows_or_zeros(live, k);
+    q = rows_or_zeros(live, q);
+    dout = rows_or_zeros(live, dout);
+    dg = rows_or_spare(live, dg);
+    dv = rows_or_spare(live, dv);
+    dk = rows_or_spare(live, dk);
+    dq = rows_or_spare(live, dq);
     const int64_t bhn = ((int64_t)b * H + h) * N + n;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
@@ -546,7 +556,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                 o[e] = fast_exp2(p8[e]) * hacc + dq8[e];
                 dl8[e] += qr[e] * hacc;
             }
-            st8_row_once<D, DM>(dq + rowoff + fo, c, pack8<TG>(o));
+            st8_row_once<D, DM>(dq + rowoff + fo, c, pack8<TG>(o), live);
         }
         // -- dk: state term V dS'^T first, then the later sub-blocks in descending order
         {
@@ -591,7 +601,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                 o[e] = fast_exp2(s8[e]) * hacc + dk8[e];
                 dl8[e] -= krt[e] * hacc;
             }
-            st8_row_once<D, DM>(dk + rowoff + fo, c, pack8<TG>(o));
+            st8_row_once<D, DM>(dk + rowoff + fo, c, pack8<TG>(o), live);
         }
         // -- dv: state term K~ dS' first, then the own and the later sub-blocks
         {
@@ -619,7 +629,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
             float o[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = acc[e >> 2][e & 3];
-            st8_row_once<D, DM>(dv + rowoff + fo, c, pack8<TG>(o));
+            st8_row_once<D, DM>(dv + rowoff + fo, c, pack8<TG>(o), live);
         }
         // -- dL of the slice is complete: reverse cumsum inside the sub-block (gla.py:616-617), then, once
         // every wave has published its sub-block total, over the whole chunk + the chunk-level term (gla.py:782)
@@ -651,7 +661,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o.v[e] += t.v[e];
             }
-            st8_row_once<D, DM>(dg + rowoff + fo, c, o);
+            st8_row_once<D, DM>(dg + rowoff + fo, c, o, live);
         }
         if (ks + 1 < KS) {
             stage_store(ks + 1);
@@ -676,7 +686,7 @@ int launch_chunk_grad(hipStream_t st, int B, int T_len, int H, const float *g, c
     typedef std::conditional_t<WIDE, float, T> TG;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
-    dim3 grid(T_len / C * H, B), block(C * 4);
+    dim3 grid((T_len + C - 1) / C * H, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q,
                        (const T *)dout, (const T *)statesN, (const T *)dstatesT, (const T *)dstatesN, dg,
                        (TG *)dv, (TG *)dk, (TG *)dq, T_len, H);

@@ -50,9 +50,14 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
     // heads vary fastest over the grid: workgroups that run together touch the same DRAM pages of the
     // [B, T, H, D] arrays (a token's H rows are contiguous)
     const int h = blockIdx.x % H, n = blockIdx.x / H, b = blockIdx.y;
-    const int N = T_len / C;
+    const bool live = n * C + 16 * w < T_len;      // the wave has tokens (see rows_or_zeros)
     const int64_t tok = (int64_t)b * T_len + (int64_t)n * C + 16 * w + r;
-    const int64_t rowoff = (tok * H + h) * DM;     // DM features per row in memory (DM < D: see RowMap)
+    const int64_t rowoff = live ? (tok * H + h) * DM : 0;     // DM features per row in memory (DM < D: see RowMap)
+    g = rows_or_zeros(live, g);
+    v = rows_or_zeros(live, v);
+    k = rows_or_zeros(live, k);
+    q = rows_or_zeros(live, q);
+    out = rows_or_spare(live, out);
     const TrLane<T> L = make_tr_lane<T>(LS);
     const int wrow = 16 * w * LS + L.nat;          // this lane's row of a [token][feature] tile
 
@@ -198,7 +203,7 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = acc[e >> 2][e & 3];
-        st8_row_once<D, DM>(out + rowoff + fo, c, pack8<std::conditional_t<WIDE, float, T>>(o));
+        st8_row_once<D, DM>(out + rowoff + fo, c, pack8<std::conditional_t<WIDE, float, T>>(o), live);
         if (ks + 1 < KS) {
             __syncthreads();             // every wave is done with the staged rows
             stage_store();
@@ -217,7 +222,7 @@ int launch_chunk_out(hipStream_t st, int B, int T_len, int H, const float *g, co
     auto kern = chunk_out_kernel<T, C, D, DM, WIDE>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
-    dim3 grid(T_len / C * H, B), block(C * 4);
+    dim3 grid((T_len + C - 1) / C * H, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q,
                        (const T *)states, slots, (std::conditional_t<WIDE, float, T> *)out, T_len, H);
     return launch_status();

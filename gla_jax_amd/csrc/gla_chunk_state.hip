@@ -61,9 +61,13 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
     // heads vary fastest over the grid: workgroups that run together touch the same DRAM pages of the
     // [B, T, H, D] arrays (a token's H rows are contiguous)
     const int h = blockIdx.x % H, n = blockIdx.x / H, b = blockIdx.y;
-    const int N = T_len / C;
+    const int N = (T_len + C - 1) / C;
+    const bool live = n * C + 16 * w < T_len;      // the wave has tokens (see rows_or_zeros)
     const int64_t tok = (int64_t)b * T_len + (int64_t)n * C + 16 * w + r;
-    const int64_t rowoff = (tok * H + h) * DM;     // DM features per row in memory (DM < D: see RowMap)
+    const int64_t rowoff = live ? (tok * H + h) * DM : 0;     // DM features per row in memory (DM < D: see RowMap)
+    g = rows_or_zeros(live, g);
+    x = rows_or_zeros(live, x);
+    y = rows_or_zeros(live, y);
 
     float p[NV];
     typename FragTypes<T>::d8 yf[KS], xf[KS];
@@ -300,12 +304,19 @@ __global__ __launch_bounds__(64) void chunk_scan_kernel(const void *__restrict__
         batch(b, std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
         if (b + 1 < nb) batch(b + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{});
     }
-    for (int step = nb * U; step < N; ++step) {
-        const int n = chunk_of(step);
-        Raw x;
-        request(n, x);
-        emit(n);
-        advance(x);
+    // what is left, all requested at once (one chunk per round trip to memory took 8 us for 7 chunks)
+    const int first = nb * U;
+    if (first < N) {
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+            if (first + u < N) request(chunk_of(first + u), buf[0][u]);
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u) {
+            if (first + u < N) {
+                emit(chunk_of(first + u));
+                advance(buf[0][u]);
+            }
+        }
     }
     if (tail && statesN) emit_n(N);
     if (in_mem) store_hidden<4>(hout, hdt, (int64_t)bh * DM * DM + dk * DM + dv0, X);
@@ -318,7 +329,7 @@ int launch_chunk_outer(hipStream_t st, int mode, int B, int T_len, int H, const 
     typedef typename Prod<T>::type P;
     constexpr int LS = TileGeom<T, D>::kStride;
     const size_t lds = (size_t)2 * C * LS * sizeof(T) + (size_t)(C / 16) * D * sizeof(float);
-    dim3 grid(T_len / C * H, B), block(C * 4);
+    dim3 grid((T_len + C - 1) / C * H, B), block(C * 4);
     if (mode == 0) {
         auto kern = chunk_outer_kernel<T, C, D, DM, 0>;
         static LdsGrant grant;

@@ -242,7 +242,7 @@ def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_
 
     Same result as `recurrent_gla_naive` up to rounding.  `chunk_size` must be a power of two that
     divides T (gla.py:500, 674), at least 32; since the result does not depend on it, the kernels run
-    with the largest tile built that divides T, whatever size is given.  `block_size_t`, `block_size_d`, `interpret`, `num_warps`,
+    with the tile that suits T, the head dimension and the number of sequences.  `block_size_t`, `block_size_d`, `interpret`, `num_warps`,
     `num_stages` tune the reference's Triton kernels; they are accepted for signature compatibility
     and have no effect here.  Differentiable in all five array arguments (gla.py:625)."""
     if interpret:
