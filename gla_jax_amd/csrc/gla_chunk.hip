@@ -31,12 +31,14 @@ struct ChunkPlan {
     {
         return prod + decay + bwd_states * states + (split ? 2 * rows + (wide ? 7 : 4) * rows_f32 + 4 * hid : 0);
     }
+    // fp32 data at 128 features ran on 32-token tiles only: callers may count on a forward workspace of that size
+    size_t fwd_least = 0;
     size_t resid_bytes() const { return split ? 2 * resid : resid; }
 };
 
 static size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// The tile: tokens per workgroup, 128, 64 or 32 (fp32 data: 64 or 32 up to 64 features, 32 at 128).  The result does not
+// The tile: tokens per workgroup, 128, 64 or 32 (fp32 data: 64 or 32).  The result does not
 // depend on it (only its rounding does), so whatever chunk_size asks for, the lengths and the number of sequences decide; a
 // tile need not divide T, the last one is filled up with zeros.  Wide tiles mean fewer chunk states to write, scan
 // and read; narrow ones more workgroups with less to do each while there are not enough for the 256 compute units.
@@ -45,12 +47,13 @@ static size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 //                 B4 T512 H6 (192 wg) 76 / 62 / 73    B16 T96 H8 (256 wg) 80 / 69 / 75    B1 T160 H1 69 / 52 / 50
 //   64 features   B16 T2048 H8 242 / 269 / 385   B16 T1056 H8 (1152 against 1088 rows) 154 / 143 / 183
 //                 B4 T2048 H6 69 / 67 / 91   B1 T16384 H2 75 / 107 (a scan of 256 chunks)   B1 T2048 H1 43 / 37 / 43
-// and fp32, 64 features, 64 / 32: B4 T1056 H6 84 / 93, B1 T512 H2 45 / 39, B1 T2048 H2 51 / 52.
+// and fp32, 64 / 32: 64 features B4 T1056 H6 84 / 93, B1 T512 H2 45 / 39, B1 T2048 H2 51 / 52; 128 features B4 T4096 H6
+// 671 / 1030, B4 T512 H6 110 / 140, B4 T288 H6 103 / 91, B1 T512 H2 94 / 75.
 static int64_t choose_tile(int64_t seqs, int64_t T, int64_t D, int dtype)
 {
     auto tiles = [&](int64_t c) { return (T + c - 1) / c; };
     constexpr int64_t kUnits = 256;                          // compute units
-    if (dtype == GLA_F32) return D > 64 || (T < 2048 && seqs * tiles(32) <= kUnits) ? 32 : 64;
+    if (dtype == GLA_F32) return T < 2048 && seqs * tiles(32) <= kUnits ? 32 : 64;
     if (T <= (D > 64 ? 256 : 576) && seqs * tiles(32) <= kUnits) return 32;
     if (seqs * tiles(64) <= kUnits && tiles(64) <= (D >= 64 ? 64 : 32)) return 64;
     // 64 features: where a 128-token tile would carry over 5 % more zeros
@@ -99,6 +102,8 @@ static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, i
     plan->scale_off = (size_t)B * H * N * DK * sizeof(float);
     plan->decay = round256(plan->scale_off + (size_t)B * H * N * (DK * DV / 16));
     plan->states = round256((size_t)B * H * N * DK * DV * esz);
+    if (dtype == GLA_F32 && Dk == 128)
+        plan->fwd_least = round256((size_t)B * H * (size_t)(T / 32) * (2 * DK * DV + DK) * sizeof(float));
     plan->bwd_states = dtype == GLA_BF16 ? 1 : 2;
     // the residual is handed out with room for the states of the largest tile that divides T, which callers may count on
     int64_t Cd = dtype == GLA_BF16 ? 128 : (DK > 64 ? 32 : 64);
@@ -163,7 +168,8 @@ extern "C" size_t gla_chunk_fwd_workspace_bytes(int64_t B, int64_t T, int64_t H,
 {
     ChunkPlan p;
     // per-chunk products, decays, and the chunk-start states in [dv][dk] orientation for the output kernel
-    return plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p) == GLA_OK ? p.fwd_bytes() : 0;
+    if (plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p) != GLA_OK) return 0;
+    return p.fwd_bytes() < p.fwd_least && !p.split ? p.fwd_least : p.fwd_bytes();
 }
 
 extern "C" size_t gla_chunk_bwd_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,

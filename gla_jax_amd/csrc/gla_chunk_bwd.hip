@@ -47,7 +47,9 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4;
     constexpr int LS = TileGeom<T, D>::kStride;
     constexpr int XS = 32 + 16 / (int)sizeof(T);   // row stride of the per-wave slice scratch
-    constexpr int VR = C > 96 ? C : 96;            // the value tile is recycled for 3 x 32 staged state rows
+    // fp32 data at 128 features and 64 tokens: one of the three state operands does not fit and is read where it lies
+    constexpr bool kDirectT = sizeof(T) == 4 && C == 64 && D == 128;
+    constexpr int VR = C > 96 ? C : (kDirectT ? 64 : 96);   // the value tile is recycled for 3 (2) x 32 staged state rows
     typedef typename FragTypes<T>::d8 D8;
     typedef typename FragTypes<T>::t4 T4;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                     pfDt[u] = ld8(dSn + (((idx >> 7) * (D / 32) + slice) << 10) + (idx & 127) * 8);   // tiles (i, slice)
                 } else {
                     pfDn[u] = ld8_once(dSn + off);
-                    pfDt[u] = ld8_once(dSt + off);
+                    if constexpr (!kDirectT) pfDt[u] = ld8_once(dSt + off);
                 }
             }
         }
@@ -149,7 +151,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                     const int dkk = 32 * (idx >> 7) + ((idx & 127) >> 2), dvv = 8 * (idx & 3);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) sDt[(dvv + e) * LS + dkk] = pfDt[u][e];
-                } else {
+                } else if constexpr (!kDirectT) {
                     st8(sDt + row * LS + c8, pfDt[u]);
                 }
                 // chunk-level gate gradient (gla.py:782), first term: e^{L_end} sum_v S_n * dS' per key feature.
@@ -398,6 +400,14 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
         for (int e = 0; e < 8; ++e) { p8[e] = gN.v[e] * kLog2e; s8[e] = 0.f; }
         unpack8(qN, a);
         unpack8(kN, bq);
+        [[maybe_unused]] D8 dirT[KS][2];            // the rows of dS' [dv][dk] that are not staged, needed last
+        if constexpr (kDirectT) {
+            const T *rows = dstatesT + bhn * D * D + (fo + 8 * (r >> 2) + (r & 3)) * D + 8 * c;
+#pragma unroll
+            for (int k2 = 0; k2 < KS; ++k2)
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt) dirT[k2][tt] = ld8(rows + 4 * tt * D + 32 * k2);
+        }
         if (ks + 1 < KS) {
             row_fetch(ks + 1);
             stage_fetch(ks + 1);
@@ -571,11 +581,23 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                 // second term of the chunk-level gate gradient: sum over the chunk's rows of k e^{L_end - L_j} times
                 // the state term (v_j dS'^T) just formed (the reference's -sum_c dLambda_k, gla.py:776-782); summed
                 // over the wave's 16 rows here, over the sub-blocks after the barrier
-                D8 kts = Kt[0];
-#pragma unroll
-                for (int i = 1; i < KS; ++i) kts = ks == i ? Kt[i] : kts;
                 float kte[8];
-                unpack8(kts, kte);
+                if constexpr (sizeof(T) == 2) {
+                    D8 kts = Kt[0];
+#pragma unroll
+                    for (int i = 1; i < KS; ++i) kts = ks == i ? Kt[i] : kts;
+                    unpack8(kts, kte);
+                } else {
+                    // value by value: a choice between two of these structs is one between their addresses, in scratch memory
+                    unpack8(Kt[0], kte);
+#pragma unroll
+                    for (int i = 1; i < KS; ++i) {
+                        float t[8];
+                        unpack8(Kt[i], t);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) kte[e] = ks == i ? t[e] : kte[e];
+                    }
+                }
                 f32x8 tb;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) tb.v[e] = suffix_sum_rows(kte[e] * acc[e >> 2][e & 3]);
@@ -609,8 +631,10 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
 #pragma unroll
             for (int k2 = 0; k2 < KS; ++k2) {
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt)
-                    acc[tt] = mma_d(ld8(sDt + L.own + 4 * tt * LS + 32 * k2), Kt[k2], acc[tt]);
+                for (int tt = 0; tt < 2; ++tt) {
+                    if constexpr (kDirectT) acc[tt] = mma_d(dirT[k2][tt], Kt[k2], acc[tt]);
+                    else acc[tt] = mma_d(ld8(sDt + L.own + 4 * tt * LS + 32 * k2), Kt[k2], acc[tt]);
+                }
             }
 #pragma unroll
             for (int I = 0; I < NB; ++I) {
@@ -678,7 +702,7 @@ int launch_chunk_grad(hipStream_t st, int B, int T_len, int H, const float *g, c
     constexpr int LS = TileGeom<T, D>::kStride;
     constexpr int XS = 32 + 16 / (int)sizeof(T);
     constexpr int NB = C / 16;
-    constexpr int VR = C > 96 ? C : 96;
+    constexpr int VR = C > 96 ? C : (sizeof(T) == 4 && C == 64 && D == 128 ? 64 : 96);
     const size_t lds = ((size_t)(3 * C + VR) * LS + (size_t)NB * 16 * XS) * sizeof(T) +
                        ((size_t)(3 * NB + 1) * D + NB * 32) * sizeof(float) +
                        ((C - 96) * LS >= NB * 16 * 32 || sizeof(T) != 2 ? 0 : (size_t)NB * 16 * 32 * sizeof(T));

@@ -24,7 +24,7 @@ namespace gla {
 // that one loads while the other computes.
 // WIDE: `out` is a float array (the sum of two such runs is rounded once: head dimension 256, gla_split.hip).
 template <typename T, int C, int D, int DM, bool WIDE>
-__global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C / 32))) void chunk_out_kernel(
+__global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C < 128 && D < 128 ? 8 : C / 32))) void chunk_out_kernel(
     const float *__restrict__ g, const T *__restrict__ v, const T *__restrict__ k, const T *__restrict__ q,
     const T *__restrict__ states, int slots, std::conditional_t<WIDE, float, T> *__restrict__ out, int T_len, int H)
 {

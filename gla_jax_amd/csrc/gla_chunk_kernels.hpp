@@ -32,6 +32,7 @@ namespace gla {
     M(float, 32, 32, 32)             \
     M(float, 64, 32, 16)             \
     M(float, 32, 32, 16)             \
+    M(float, 64, 128, 128)           \
     M(float, 32, 128, 128)
 
 template <typename T, int C, int D, int DM>

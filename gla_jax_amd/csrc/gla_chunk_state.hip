@@ -41,7 +41,7 @@ constexpr int kProdNotFinite = 255;      // the exponent byte of a group with a 
 // Two tiles and a table fit twice into a CU's LDS; the register budget is held to what lets two
 // workgroups share a CU, so that one loads while the other computes.
 template <typename T, int C, int D, int DM, int MODE>
-__global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C / 32))) void chunk_outer_kernel(const float *__restrict__ g,
+__global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C < 128 && D < 128 ? 8 : C / 32))) void chunk_outer_kernel(const float *__restrict__ g,
                                                             const T *__restrict__ x,
                                                             const T *__restrict__ y,
                                                             typename Prod<T>::type *__restrict__ prodT,

@@ -44,3 +44,15 @@ def test_scan_over_chunks_with_a_last_batch_that_is_not_full(BH, T):
     assert torch.allclose(hT.double(), h0.double() * L[:, -1].exp()[..., None], rtol=1e-5, atol=1e-5)
     want = (q.double() * L.exp()).permute(0, 2, 1, 3) @ h0.double()
     assert torch.allclose(out.double().permute(0, 2, 1, 3), want, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("T,shift", [(2048, 3.0), (2080, -2.0)])
+def test_float_data_at_128_features_on_64_token_tiles(T, shift):
+    from gla_jax_amd import chunk_gla
+    dtype = torch.float32
+    arrs, dev = gpu_inputs(1, T, 1, 128, shift, seed=T, dtype=dtype)
+    dhT, dout = cotangents(arrs[0], arrs[2], 4, dtype)
+    dev = [t.clone().requires_grad_(True) for t in dev]
+    hT, out = chunk_gla(*dev, 32)
+    grads = torch.autograd.grad((hT, out), dev, (to_dev(dhT, dtype), to_dev(dout, dtype)))
+    check_chunk_outputs(dtype, arrs, 32, hT, out, grads, dhT, dout)
