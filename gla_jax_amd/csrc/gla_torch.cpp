@@ -84,10 +84,13 @@ Tensor bytes_like(size_t n, const Tensor &t) { return at::empty({(int64_t)n}, t.
     std::abort();
 }
 
+// The call goes through the autograd function: a gradient may be asked for, or an array carries a forward-mode tangent,
+// which the function refuses (a call past it would drop the tangent without a word).
 bool wants_grad(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q)
 {
-    return at::GradMode::is_enabled() && (h0.requires_grad() || g.requires_grad() || v.requires_grad() ||
-                                          k.requires_grad() || q.requires_grad());
+    for (const Tensor *t : {&h0, &g, &v, &k, &q})
+        if ((at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(/*level=*/0).defined()) return true;
+    return false;
 }
 
 // ---- chunk_gla ----------------------------------------------------------------------------------
@@ -279,7 +282,7 @@ std::optional<Tensor> cumsum(const Tensor &src, int64_t axis, const std::optiona
     int64_t outer = 1, inner = 1;
     for (int64_t i = 0; i < axis; ++i) outer *= src.size(i);
     for (int64_t i = axis + 1; i < n; ++i) inner *= src.size(i);
-    if (outer > 65535) return std::nullopt;
+    if (outer < 1 || outer > 65535) return std::nullopt;
     if (init) {
         if (!plain_f32(*init) || init->dim() != n - 1 || init->device() != src.device()) return std::nullopt;
         for (int64_t i = 0; i < n - 1; ++i)

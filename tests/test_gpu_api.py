@@ -129,3 +129,23 @@ def test_chunk_values_that_are_not_finite_reach_the_state(bad):
     assert not torch.isfinite(hT.float()[0, 0, :, 5]).any()          # that value feature of the final state
     assert torch.isfinite(hT.float()[0, 0, :, 40:]).all()            # value features of other product tiles are untouched
     assert not torch.isfinite(out.float()[0, 130, 0, 5])
+
+
+@pytest.mark.parametrize("name", ["chunk_gla", "recurrent_gla", "recurrent_gla_naive"])
+def test_forward_mode_tangents_are_refused(name):
+    """There is no forward-mode rule: a call on an array with a tangent raises, also where no gradient is asked for,
+    instead of returning results without one."""
+    import torch.autograd.forward_ad as fwAD
+    fn = _bind(name)
+    _, dev = gpu_inputs(1, 64, 1, 64, 3.0, seed=18, dtype=torch.float32)
+    with fwAD.dual_level():
+        query = fwAD.make_dual(dev[4], torch.ones_like(dev[4]))
+        with pytest.raises(RuntimeError):
+            fn(*dev[:4], query)
+        with torch.no_grad(), pytest.raises(RuntimeError):
+            fn(*dev[:4], query)
+
+
+def test_cumsum_of_no_rows_is_empty():
+    from gla_jax_amd import cumsum_recursive
+    assert cumsum_recursive(torch.empty(0, 5, 3, device="cuda"), 1).shape == (0, 5, 3)
