@@ -56,6 +56,22 @@ __device__ __forceinline__ f32x4 mma_t(f32x4 a, f32x4 b, f32x4 c)
     for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
     return c;
 }
+// mma_t2: two such products in one instruction, c += A0 B0 + A1 B1.  The matrix cores take 16 cycles for 16 as for 32
+// contracted values, and a lane's k-slots may hold any 8 of them as long as A and B agree, so the operands of two
+// 16-token contractions side by side fill the instruction of twice the depth: a third to a half of the matrix instructions of
+// recurrent_gla's kernels (B4 T4096 H16 D128: the two backward sweeps 238 -> 226 and 349 -> 325 us).
+// Never add a mma_t to the result of a mma_d or mma_t2 right behind it: the compiler leaves no wait between the two
+// instructions, and the shallower one then takes the sum too early (seen: the low half of the accumulators without the last
+// product).  recurrent_gla's kernels use the deeper instruction alone; elsewhere LDS reads or arithmetic lie between.
+__device__ __forceinline__ f32x4 mma_t2(bf16x4 a0, bf16x4 a1, bf16x4 b0, bf16x4 b1, f32x4 c)
+{
+    return mma_d(__builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7),
+                 __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7), c);
+}
+__device__ __forceinline__ f32x4 mma_t2(f32x4 a0, f32x4 a1, f32x4 b0, f32x4 b1, f32x4 c)
+{
+    return mma_t(a1, b1, mma_t(a0, b0, c));
+}
 
 // ---- packing ----------------------------------------------------------------------------------
 template <typename T> __device__ __forceinline__ typename FragTypes<T>::d8 pack8(const float *x);
@@ -247,6 +263,12 @@ __device__ __forceinline__ f32x4 lds_tr4(const float *p, int stride)
 {
     f32x4 r = {p[0], p[stride], p[2 * stride], p[3 * stride]};
     return r;
+}
+
+// Two such reads, `further` elements apart: the operand of a contraction over 32 rows.
+__device__ __forceinline__ bf16x8 lds_tr4x2(const __bf16 *p, int further)
+{
+    return __builtin_shufflevector(lds_tr4(p, 0), lds_tr4(p + further, 0), 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
 // Plain mapping: tile t covers features 16t .. 16t+15, lane i gets feature 16t + i.

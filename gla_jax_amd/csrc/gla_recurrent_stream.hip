@@ -72,40 +72,38 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
     const int N = (T_len + C - 1) / C;
     const int wv = w % NDV, nt0 = (w / NDV) * NTW;   // the wave's tile rows are wv + i NDV, its tile columns nt0 + j
 
-    // state: S[i][j][e] = state[dk = 16(nt0 + j) + r][dv = 16(wv + i NDV) + 4c + e]  (accumulator layout of a
-    // (dv x dk) product tile)
+    // state: S[i][j][e] = state[dk = 16(nt0 + j) + 4c + e][dv = 16(wv + i NDV) + r]  (accumulator layout of a
+    // (dk x dv) product tile): a lane's four values of a tile are neighbours in the [dv][dk] copy below, one 8-byte
+    // store per tile and precision.  (dv x dk) tiles needed an exchange inside the quads of lanes first, 16 vector
+    // instructions per tile; with the products of mma_t2 B4 T4096 H16 D128 went from 234 to 222 us.  The lean form
+    // writes no copy and keeps (dv x dk) tiles, dk = 16(nt0 + j) + r and dv = 16(wv + i NDV) + 4c + e, whose decay is
+    // one value per lane and tile (four take registers that it does not have: 71.6 -> 75 us).
     f32x4 S[RT][NTW];
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
-            float t4[4] = {0.f, 0.f, 0.f, 0.f};     // no initial state given: zeros (the lean pass of a segment)
-            if (h0) load_hidden<4>(h0, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + r) * D + 16 * (wv + i * NDV) + 4 * c, t4);
-            S[i][nt] = f32x4{t4[0], t4[1], t4[2], t4[3]};
+            S[i][nt] = f32x4{0.f, 0.f, 0.f, 0.f};   // no initial state given: zeros (the lean pass of a segment)
+            if (h0) {
+                if constexpr (STATE) {
+                    float t4[4];
+                    load_hidden<4>(h0, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + r) * D + 16 * (wv + i * NDV) + 4 * c, t4);
+                    S[i][nt] = f32x4{t4[0], t4[1], t4[2], t4[3]};
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        S[i][nt][e] = load_hidden1(h0, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + 4 * c + e) * D + 16 * (wv + i * NDV) + r);
+                }
+            }
         }
-    // A lane's four values of a tile lie in four rows of the [dv][dk] copy.  The four lanes of a quad exchange them
-    // (a 4 x 4 transpose in two steps across lanes 1 and 2 apart), after which lane 4a + j holds the key features
-    // 4a..4a+3 of row 4c + j: one 8-byte store per tile and precision instead of four 2-byte ones.
     auto publish_state = [&]() {
-        const int j = r & 3;
 #pragma unroll
         for (int i = 0; i < RT; ++i)
 #pragma unroll
             for (int nt = 0; nt < NTW; ++nt) {
-                f32x4 x = S[i][nt], y;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float other = dpp_f32<kDppQuadXor1>(x[e ^ 1]);
-                    y[e] = ((j ^ e) & 1) ? other : x[e];
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float other = dpp_f32<kDppQuadXor2>(y[e ^ 2]);
-                    x[e] = ((j ^ e) & 2) ? other : y[e];
-                }
                 T4 hi, lo;
-                split4<T>(x, hi, lo);
-                const int off = (16 * (wv + i * NDV) + 4 * c + j) * LS + 16 * (nt0 + nt) + (r & 12);
+                split4<T>(S[i][nt], hi, lo);
+                const int off = (16 * (wv + i * NDV) + r) * LS + 16 * (nt0 + nt) + 4 * c;
                 *reinterpret_cast<T4 *>(St + off) = hi;
                 *reinterpret_cast<T4 *>(Sl + off) = lo;
             }
@@ -231,10 +229,7 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
         }
 
         // ---- out^T[dv][i] in slices of 32 output features: state term, then the score blocks --------
-        // (a real loop at D = 128: one slice's temporaries live at a time.  The fully unrolled form was also
-        // WRONG there: the slices at features 32 and 64 lost the key features 96..127 of the state term,
-        // with the published state intact and every immediate offset of the reads in range; the cause was
-        // not found, so the unrolled form stays out for D = 128.)
+        // (a real loop at D = 128: one slice's temporaries live at a time)
         constexpr int kSliceUnroll = KS > 2 ? 1 : KS;
 #pragma unroll kSliceUnroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -257,8 +252,7 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
 #pragma unroll
                     for (int tt = 0; tt < 2; ++tt) {
                         const T4 va = lds_tr4(Vn + L.k4 + fo + 4 * tt + 16 * J * LS, LS);
-                        acc[tt] = mma_t(va, l4, acc[tt]);
-                        acc[tt] = mma_t(va, b4, acc[tt]);
+                        acc[tt] = mma_t2(va, va, l4, b4, acc[tt]);
                     }
                 }
             }
@@ -276,18 +270,21 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
         // ---- state update: S <- S e^{tau_J} + V_J^T (k e^{tau_J - l})_J over the sub-blocks in order ------
 #pragma unroll
         for (int J = 0; J < NB; ++J) {
-            float rr[NTW];
+            std::conditional_t<STATE, float, f32x4> rr[NTW];
 #pragma unroll
-            for (int nt = 0; nt < NTW; ++nt) rr[nt] = rtab[J * D + 16 * (nt0 + nt) + r];
+            for (int nt = 0; nt < NTW; ++nt) {
+                if constexpr (STATE) rr[nt] = rtab[J * D + 16 * (nt0 + nt) + r];
+                else rr[nt] = *reinterpret_cast<const f32x4 *>(rtab + J * D + 16 * (nt0 + nt) + 4 * c);
+            }
 #pragma unroll
             for (int i = 0; i < RT; ++i) {
                 auto va = lds_tr4(Vn + ptl + 16 * J * LS + 16 * (wv + i * NDV), LS);
 #pragma unroll
                 for (int nt = 0; nt < NTW; ++nt) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) S[i][nt][e] *= rr[nt];
-                    S[i][nt] = mma_t(va, lds_tr4(Kl + ptl + 16 * J * LS + 16 * (nt0 + nt), LS), S[i][nt]);
-                    S[i][nt] = mma_t(va, lds_tr4(Kh + ptl + 16 * J * LS + 16 * (nt0 + nt), LS), S[i][nt]);
+                    S[i][nt] *= rr[nt];
+                    const T4 kl = lds_tr4(Kl + ptl + 16 * J * LS + 16 * (nt0 + nt), LS);
+                    const T4 kh = lds_tr4(Kh + ptl + 16 * J * LS + 16 * (nt0 + nt), LS);
+                    S[i][nt] = STATE ? mma_t2(va, va, kl, kh, S[i][nt]) : mma_t2(kl, kh, va, va, S[i][nt]);
                 }
             }
         }
@@ -308,8 +305,14 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
     for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
-            float t4[4] = {S[i][nt][0], S[i][nt][1], S[i][nt][2], S[i][nt][3]};
-            store_hidden<4>(hT, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + r) * D + 16 * (wv + i * NDV) + 4 * c, t4);
+            if constexpr (STATE) {
+                float t4[4] = {S[i][nt][0], S[i][nt][1], S[i][nt][2], S[i][nt][3]};
+                store_hidden<4>(hT, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + r) * D + 16 * (wv + i * NDV) + 4 * c, t4);
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                store_hidden1(hT, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + 4 * c + e) * D + 16 * (wv + i * NDV) + r, S[i][nt][e]);
         }
 }
 

@@ -314,8 +314,8 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
                 for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) S[i][nt][e] *= rr[nt];
-                    S[i][nt] = mma_t(va, lds_tr4(Kl + ptl + 16 * J * LS + 16 * nt, LS), S[i][nt]);
-                    S[i][nt] = mma_t(va, lds_tr4(Kh + ptl + 16 * J * LS + 16 * nt, LS), S[i][nt]);
+                    S[i][nt] = mma_t2(va, va, lds_tr4(Kl + ptl + 16 * J * LS + 16 * nt, LS),
+                                      lds_tr4(Kh + ptl + 16 * J * LS + 16 * nt, LS), S[i][nt]);
                 }
             }
         }
@@ -681,10 +681,10 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
 #pragma unroll
                         for (int tt = 0; tt < 2; ++tt) {
                             const T4 oa = lds_tr4(tO + L.k4 + fo + 4 * tt + 16 * I * LS, LS);
-                            acc[tt] = mma_t(oa, bl4, acc[tt]);
                             if constexpr (kSplitDout)
-                                acc[tt] = mma_t(lds_tr4(tOl + L.k4 + fo + 4 * tt + 16 * I * LS, LS), bh4, acc[tt]);
-                            acc[tt] = mma_t(oa, bh4, acc[tt]);
+                                acc[tt] = mma_t_split(oa, lds_tr4(tOl + L.k4 + fo + 4 * tt + 16 * I * LS, LS), bh4, bl4, acc[tt]);
+                            else
+                                acc[tt] = mma_t2(oa, oa, bl4, bh4, acc[tt]);
                         }
                     }
                 }
@@ -696,21 +696,15 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
             // -- dk slice: dS' v first, then the later sub-blocks in descending order
             {
                 f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-                // (dS' v)[dk][j] = sum_dv dS'[dk][dv] v_j[dv]: 16 dv rows per step, read transposed.  Step (k2,
-                // half) contracts over dv = 32 k2 + 8 c + 4 half + m, which is what lane (j, c) holds of v_j.
+                // (dS' v)[dk][j] = sum_dv dS'[dk][dv] v_j[dv]: 32 dv rows per step, read transposed, 16 per read.  Read
+                // (k2, half) holds dv = 32 k2 + 8 c + 4 half + m, which is what lane (j, c) holds of v_j.
 #pragma unroll
-                for (int k2 = 0; k2 < KS; ++k2) {
+                for (int k2 = 0; k2 < KS; ++k2)
 #pragma unroll
-                    for (int half = 0; half < 2; ++half) {
-                        const T4 vb = half ? __builtin_shufflevector(vf[k2], vf[k2], 4, 5, 6, 7)
-                                           : __builtin_shufflevector(vf[k2], vf[k2], 0, 1, 2, 3);
-#pragma unroll
-                        for (int tt = 0; tt < 2; ++tt) {
-                            acc[tt] = mma_t(lds_tr4(DTl + L.k8 + (32 * k2 + 4 * half) * LS + fo + 4 * tt, LS), vb, acc[tt]);
-                            acc[tt] = mma_t(lds_tr4(DTh + L.k8 + (32 * k2 + 4 * half) * LS + fo + 4 * tt, LS), vb, acc[tt]);
-                        }
+                    for (int tt = 0; tt < 2; ++tt) {
+                        acc[tt] = mma_d(lds_tr4x2(DTl + L.k8 + 32 * k2 * LS + fo + 4 * tt, 4 * LS), vf[k2], acc[tt]);
+                        acc[tt] = mma_d(lds_tr4x2(DTh + L.k8 + 32 * k2 * LS + fo + 4 * tt, 4 * LS), vf[k2], acc[tt]);
                     }
-                }
 #pragma unroll
                 for (int I = NB - 1; I >= 1; --I) {
                     if (I > w) {
@@ -757,10 +751,10 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
 #pragma unroll
                     for (int e = 0; e < 4; ++e) DS[i][nt][e] *= rr[e];
                     const T4 ob = lds_tr4(tO + ptl + 16 * I * LS + 16 * nt, LS);
-                    DS[i][nt] = mma_t(qal, ob, DS[i][nt]);
                     if constexpr (kSplitDout)
-                        DS[i][nt] = mma_t(qah, lds_tr4(tOl + ptl + 16 * I * LS + 16 * nt, LS), DS[i][nt]);
-                    DS[i][nt] = mma_t(qah, ob, DS[i][nt]);
+                        DS[i][nt] = mma_t_split(qah, qal, ob, lds_tr4(tOl + ptl + 16 * I * LS + 16 * nt, LS), DS[i][nt]);
+                    else
+                        DS[i][nt] = mma_t2(qah, qal, ob, ob, DS[i][nt]);
                 }
             }
         }

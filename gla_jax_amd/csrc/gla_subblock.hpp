@@ -44,11 +44,10 @@ __device__ __forceinline__ void split4(f32x4 x, typename FragTypes<T>::t4 &hi, t
     for (int e = 0; e < 4; ++e) x[e] -= (float)hi[e];
     lo = pack4<T>(x);
 }
+// (the remainder x remainder term comes with the second product; A's registers serve both)
 template <typename T4> __device__ __forceinline__ f32x4 mma_t_split(T4 ah, T4 al, T4 bh, T4 bl, f32x4 acc)
 {
-    acc = mma_t(al, bh, acc);
-    acc = mma_t(ah, bl, acc);
-    return mma_t(ah, bh, acc);
+    return mma_t2(ah, al, bh, bh, mma_t2(ah, al, bl, bl, acc));
 }
 
 // Hard gates (a sub-block whose gate sums span 48 powers of two or more) are rare, and the dyadic levels need
