@@ -29,6 +29,9 @@ SIGNATURES = {
     "gla_recurrent_bwd_workspace_bytes": (_sz, [_i64] * 5 + [_int]),
     "gla_recurrent_fwd_ws": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int] + [_vp] * 8 + [_sz]),
     "gla_recurrent_bwd_ws": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int] + [_vp] * 14 + [_sz]),
+    "gla_recurrent_residual_bytes": (_sz, [_i64] * 5 + [_int]),
+    "gla_recurrent_fwd_res": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int] + [_vp] * 9 + [_sz]),
+    "gla_recurrent_bwd_res": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int] + [_vp] * 15 + [_sz]),
     "gla_chunk_states_bytes": (_sz, [_i64] * 6 + [_int]),
     "gla_chunk_fwd_workspace_bytes": (_sz, [_i64] * 6 + [_int]),
     "gla_chunk_bwd_workspace_bytes": (_sz, [_i64] * 6 + [_int]),

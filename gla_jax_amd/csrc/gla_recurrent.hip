@@ -505,6 +505,9 @@ struct TimeSplit {
     // backward: the same, the cotangents that leave the segments, and a second array of contributions for an fp32
     // dout beside bf16 data (two passes)
     size_t bwd() const { return on() ? 2 * hid + 2 * hidf + sums : 0; }
+    // what a forward can hand to the backward, which forms it again otherwise (a lean pass and a scan, 88 of 1000 us at
+    // B4 T4096 H16 D128): the entering states and the pieces' gate sums
+    size_t residual() const { return on() ? hid + sums : 0; }
 };
 // what head dimension 256 needs for its own passes, over the segments or pieces there are
 static size_t inner_fwd_bytes(const TimeSplit &ts, int64_t B, int64_t T, int64_t H, int64_t DK, int dtype)
@@ -533,6 +536,12 @@ extern "C" size_t gla_recurrent_bwd_workspace_bytes(int64_t B, int64_t T, int64_
     if (gla::check_recurrent(B, T, H, DK, DV, dtype, GLA_F32, GLA_F32) || 2 * H > 65535) return 0;
     const gla::TimeSplit ts(B, T, H, DK, dtype);
     return ts.bwd() + gla::inner_bwd_bytes(ts, B, T, H, DK, dtype);
+}
+
+extern "C" size_t gla_recurrent_residual_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype)
+{
+    if (gla::check_recurrent(B, T, H, DK, DV, dtype, GLA_F32, GLA_F32) || 2 * H > 65535) return 0;
+    return gla::TimeSplit(B, T, H, DK, dtype).residual();
 }
 
 // One pass over the segments of `sg`; arguments checked by the caller.  Head dimension 256 with a workspace: two passes
@@ -598,6 +607,16 @@ extern "C" int gla_recurrent_fwd_ws(void *stream, int64_t B, int64_t T, int64_t 
                                     const void *key, const void *query, void *hidden_final, void *out,
                                     void *workspace, size_t workspace_bytes)
 {
+    return gla_recurrent_fwd_res(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init, log_fgate, value,
+                                 key, query, hidden_final, out, nullptr, workspace, workspace_bytes);
+}
+
+extern "C" int gla_recurrent_fwd_res(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
+                                     gla_dtype dtype, gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse,
+                                     const void *hidden_init, const float *log_fgate, const void *value,
+                                     const void *key, const void *query, void *hidden_final, void *out, void *residual,
+                                     void *workspace, size_t workspace_bytes)
+{
     const size_t need = gla_recurrent_fwd_workspace_bytes(B, T, H, DK, DV, dtype);
     if (!need)      // nothing to gain from a workspace at this shape
         return recurrent_fwd_run(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
@@ -618,6 +637,11 @@ extern "C" int gla_recurrent_fwd_ws(void *stream, int64_t B, int64_t T, int64_t 
     hipStream_t st = (hipStream_t)stream;
     unsigned char *ws = (unsigned char *)workspace;
     float *entering = (float *)ws, *loc = (float *)(ws + ts.hid), *sums = (float *)(ws + ts.hid + ts.hidf);
+    if (residual) {
+        if (!gla::aligned16(residual)) return GLA_ERR_ALIGN;
+        entering = (float *)residual;
+        sums = (float *)((unsigned char *)residual + ts.hid);
+    }
     void *inner_ws = DK == 256 ? ws + ts.fwd() : nullptr;
     const bool lean = gla::has_lean_pass(dtype, DK);
     int e = 0;
@@ -733,6 +757,19 @@ extern "C" int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t 
                                     float *dlog_fgate, void *dvalue, void *dkey, void *dquery, void *workspace,
                                     size_t workspace_bytes)
 {
+    return gla_recurrent_bwd_res(stream, B, T, H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init, log_fgate, value,
+                                 key, query, hidden_final, dhidden_final, dout, dhidden_init, dlog_fgate, dvalue, dkey, dquery,
+                                 nullptr, workspace, workspace_bytes);
+}
+
+extern "C" int gla_recurrent_bwd_res(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
+                                     gla_dtype dtype, gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse,
+                                     const void *hidden_init, const float *log_fgate, const void *value,
+                                     const void *key, const void *query, const void *hidden_final,
+                                     const void *dhidden_final, const void *dout, void *dhidden_init,
+                                     float *dlog_fgate, void *dvalue, void *dkey, void *dquery, const void *residual,
+                                     void *workspace, size_t workspace_bytes)
+{
     const size_t need = gla_recurrent_bwd_workspace_bytes(B, T, H, DK, DV, dtype);
     if (!need)
         return recurrent_bwd_run(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
@@ -760,23 +797,30 @@ extern "C" int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t 
                                    dlog_fgate, dvalue, dkey, dquery, DK == 256 ? (unsigned char *)workspace + ts.bwd() : nullptr);
     hipStream_t st = (hipStream_t)stream;
     unsigned char *ws = (unsigned char *)workspace;
-    float *entering = (float *)ws, *dleaving = (float *)(ws + ts.hid), *loc = (float *)(ws + 2 * ts.hid),
-          *loc_rem = (float *)(ws + 2 * ts.hid + ts.hidf), *sums = (float *)(ws + 2 * ts.hid + 2 * ts.hidf);
+    if (residual && !gla::aligned16(residual)) return GLA_ERR_ALIGN;
+    float *dleaving = (float *)(ws + ts.hid), *loc = (float *)(ws + 2 * ts.hid),
+          *loc_rem = (float *)(ws + 2 * ts.hid + ts.hidf);
+    const float *entering = residual ? (const float *)residual : (const float *)ws;
+    const float *sums = residual ? (const float *)((const unsigned char *)residual + ts.hid)
+                                 : (const float *)(ws + 2 * ts.hid + 2 * ts.hidf);
     void *inner_ws = DK == 256 ? ws + ts.bwd() : nullptr;      // sized for the backward, which needs more
     const bool lean = gla::has_lean_pass(dtype, DK);
-    // 1. the states that enter the segments, as the forward formed them (where the pass is a full one, its `out` lands
-    //    in dquery, which the backward proper overwrites)
+    // 1. the states that enter the segments, as the forward formed them, unless it has handed them over (where the pass
+    //    is a full one, its `out` lands in dquery, which the backward proper overwrites)
     int e = 0;
-    if (!lean) {
-        e = gla::launch_segment_gate_sums(st, B, ts.sg, H, (int)DK, log_fgate, sums);
+    if (!residual) {
+        float *own = (float *)ws, *own_sums = (float *)(ws + 2 * ts.hid + 2 * ts.hidf);
+        if (!lean) {
+            e = gla::launch_segment_gate_sums(st, B, ts.sg, H, (int)DK, log_fgate, own_sums);
+            if (e) return e;
+        }
+        e = recurrent_fwd_inner(stream, B, ts.pieces, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, nullptr, log_fgate,
+                                value, key, query, loc, dquery, inner_ws, true, 0, lean ? own_sums : nullptr);
+        if (e) return e;
+        e = gla::launch_segment_scan(st, B, ts.pieces, ts.F, H, (int)DK, hidden_dtype, hidden_init, loc, nullptr, own_sums,
+                                     nullptr, 0, reverse, own, nullptr);
         if (e) return e;
     }
-    e = recurrent_fwd_inner(stream, B, ts.pieces, H, DK, DV, dtype, GLA_F32, out_dtype, reverse, nullptr, log_fgate, value,
-                            key, query, loc, dquery, inner_ws, true, 0, lean ? sums : nullptr);
-    if (e) return e;
-    e = gla::launch_segment_scan(st, B, ts.pieces, ts.F, H, (int)DK, hidden_dtype, hidden_init, loc, nullptr, sums,
-                                 nullptr, 0, reverse, entering, nullptr);
-    if (e) return e;
     // 2. the cotangents of the states that leave the segments.  d(state) obeys the state's recurrence against time
     //    with query for key and dout for value, the decay between two steps being the later step's gate: the same
     //    forward kernels in the other direction with the gates taken one row further on.  The lean kernels read

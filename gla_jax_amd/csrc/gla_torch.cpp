@@ -183,8 +183,9 @@ struct Chunk : torch::autograd::Function<Chunk> {      // gla.py:483-550, 552-62
 };
 
 // ---- recurrent_gla ------------------------------------------------------------------------------
+// residual: what the forward can leave for the backward (undefined where sequences run whole), if that is wanted
 std::pair<Tensor, Tensor> recurrent_forward(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k,
-                                            const Tensor &q, bool reverse, bool out_fp32)
+                                            const Tensor &q, bool reverse, bool out_fp32, Tensor *residual = nullptr)
 {
     const c10::DeviceGuard guard(k.device());
     const Dims d = dims_of(k);
@@ -193,15 +194,19 @@ std::pair<Tensor, Tensor> recurrent_forward(const Tensor &h0, const Tensor &g, c
     // a workspace where the library can use one (head dimension 256, few sequences)
     const size_t nws = gla_recurrent_fwd_workspace_bytes(d.B, d.T, d.H, d.D, d.D, dt);
     if (nws) ws = bytes_like(nws, v);
-    check("gla_recurrent_fwd_ws",
-          gla_recurrent_fwd_ws(stream_of(k), d.B, d.T, d.H, d.D, d.D, dt, code(h0), out_fp32 ? GLA_F32 : dt, reverse,
+    const size_t nres = residual ? gla_recurrent_residual_bytes(d.B, d.T, d.H, d.D, d.D, dt) : 0;
+    if (nres) *residual = bytes_like(nres, v);
+    check("gla_recurrent_fwd_res",
+          gla_recurrent_fwd_res(stream_of(k), d.B, d.T, d.H, d.D, d.D, dt, code(h0), out_fp32 ? GLA_F32 : dt, reverse,
                                h0.data_ptr(), (const float *)g.data_ptr(), v.data_ptr(), k.data_ptr(), q.data_ptr(),
-                               hT.data_ptr(), out.data_ptr(), nws ? ws.data_ptr() : nullptr, nws));
+                               hT.data_ptr(), out.data_ptr(), nres ? residual->data_ptr() : nullptr,
+                               nws ? ws.data_ptr() : nullptr, nws));
     return {hT, out};
 }
 
 variable_list recurrent_backward(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q,
-                                 const Tensor &hT, const Tensor &dhT, const Tensor &dout, bool reverse, bool out_fp32)
+                                 const Tensor &hT, const Tensor &residual, const Tensor &dhT, const Tensor &dout, bool reverse,
+                                 bool out_fp32)
 {
     const c10::DeviceGuard guard(k.device());
     const Dims d = dims_of(k);
@@ -210,20 +215,21 @@ variable_list recurrent_backward(const Tensor &h0, const Tensor &g, const Tensor
            dq = at::empty_like(q), ws;
     const size_t nws = gla_recurrent_bwd_workspace_bytes(d.B, d.T, d.H, d.D, d.D, dt);
     if (nws) ws = bytes_like(nws, v);
-    check("gla_recurrent_bwd_ws",
-          gla_recurrent_bwd_ws(stream_of(k), d.B, d.T, d.H, d.D, d.D, dt, code(h0), out_fp32 ? GLA_F32 : dt, reverse,
+    check("gla_recurrent_bwd_res",
+          gla_recurrent_bwd_res(stream_of(k), d.B, d.T, d.H, d.D, d.D, dt, code(h0), out_fp32 ? GLA_F32 : dt, reverse,
                                h0.data_ptr(), (const float *)g.data_ptr(), v.data_ptr(), k.data_ptr(), q.data_ptr(),
                                hT.data_ptr(), dhT.data_ptr(), dout.data_ptr(), dh0.data_ptr(), (float *)dg.data_ptr(),
-                               dv.data_ptr(), dk.data_ptr(), dq.data_ptr(), nws ? ws.data_ptr() : nullptr, nws));
+                               dv.data_ptr(), dk.data_ptr(), dq.data_ptr(), residual.defined() ? residual.data_ptr() : nullptr,
+                               nws ? ws.data_ptr() : nullptr, nws));
     return {dh0, dg, dv, dk, dq};
 }
 
 struct RecurrentBackward : torch::autograd::Function<RecurrentBackward> {
     static variable_list forward(AutogradContext *, const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k,
-                                 const Tensor &q, const Tensor &hT, const Tensor &dhT, const Tensor &dout, bool reverse,
-                                 bool out_fp32)
+                                 const Tensor &q, const Tensor &hT, const std::optional<Tensor> &residual, const Tensor &dhT,
+                                 const Tensor &dout, bool reverse, bool out_fp32)
     {
-        return recurrent_backward(h0, g, v, k, q, hT, dhT, dout, reverse, out_fp32);
+        return recurrent_backward(h0, g, v, k, q, hT, residual.value_or(Tensor()), dhT, dout, reverse, out_fp32);
     }
     static variable_list backward(AutogradContext *, variable_list) { no_double_backward("recurrent_gla"); }
 };
@@ -232,8 +238,9 @@ struct Recurrent : torch::autograd::Function<Recurrent> {      // gla.py:99-170,
     static variable_list forward(AutogradContext *ctx, const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k,
                                  const Tensor &q, bool reverse, bool out_fp32)
     {
-        auto [hT, out] = recurrent_forward(h0, g, v, k, q, reverse, out_fp32);
-        ctx->save_for_backward({h0, g, v, k, q, hT});          // residuals of gla.py:169
+        Tensor residual;
+        auto [hT, out] = recurrent_forward(h0, g, v, k, q, reverse, out_fp32, &residual);
+        ctx->save_for_backward({h0, g, v, k, q, hT, residual});          // residuals of gla.py:169, and the segments' states
         ctx->saved_data["reverse"] = reverse;
         ctx->saved_data["out_fp32"] = out_fp32;
         ctx->set_materialize_grads(false);
@@ -246,8 +253,8 @@ struct Recurrent : torch::autograd::Function<Recurrent> {      // gla.py:99-170,
         const Tensor dhT = cotangent(d[0], s[0].sizes(), s[0].scalar_type(), s[0]);
         const Tensor dout = cotangent(d[1], s[2].sizes(), out_fp32 ? at::kFloat : s[2].scalar_type(), s[2]);
         variable_list r = at::GradMode::is_enabled()
-                              ? RecurrentBackward::apply(s[0], s[1], s[2], s[3], s[4], s[5], dhT, dout, reverse, out_fp32)
-                              : recurrent_backward(s[0], s[1], s[2], s[3], s[4], s[5], dhT, dout, reverse, out_fp32);
+                              ? RecurrentBackward::apply(s[0], s[1], s[2], s[3], s[4], s[5], std::optional<Tensor>(s[6]), dhT, dout, reverse, out_fp32)
+                              : recurrent_backward(s[0], s[1], s[2], s[3], s[4], s[5], s[6], dhT, dout, reverse, out_fp32);
         r.resize(7);
         return r;
     }
