@@ -241,24 +241,6 @@ int gla_chunk_bwd_stages(void *stream, int stages, int64_t B, int64_t T, int64_t
                          void *dhidden_init, float *dlog_fgate, void *dvalue, void *dkey, void *dquery,
                          void *workspace, size_t workspace_bytes);
 
-/* The same two rules with a residual: where sequences run as segments, the forward leaves the states that enter the
- * segments and the segments' gate sums in `residual` (gla_recurrent_residual_bytes, 0 where sequences run whole: then it is
- * ignored), and a backward of the same sizes that is given it does not form them again.  NULL: as the _ws entry points,
- * with the same workspaces and the same results to the bit. */
-size_t gla_recurrent_residual_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype);
-int gla_recurrent_fwd_res(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
-                          gla_dtype dtype, gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse,
-                          const void *hidden_init, const float *log_fgate, const void *value,
-                          const void *key, const void *query,
-                          void *hidden_final, void *out, void *residual, void *workspace, size_t workspace_bytes);
-int gla_recurrent_bwd_res(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
-                          gla_dtype dtype, gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse,
-                          const void *hidden_init, const float *log_fgate, const void *value,
-                          const void *key, const void *query, const void *hidden_final,
-                          const void *dhidden_final, const void *dout,
-                          void *dhidden_init, float *dlog_fgate, void *dvalue, void *dkey, void *dquery,
-                          const void *residual, void *workspace, size_t workspace_bytes);
-
 #ifdef __cplusplus
 }
 #endif
