@@ -284,11 +284,12 @@ def bench_scans(B, T, H, D, chunk, shift, steps, warmup):
     a = torch.nn.functional.logsigmoid(torch.randn(B * H, N, D, device="cuda")).contiguous()
     kv = torch.randn(B * H, N, D, D, device="cuda")
     oa, ob = torch.empty_like(a), torch.empty_like(kv)
+    ws = torch.empty(max(1, lib.gla_cumsum_workspace_bytes(B, T, H * D)), dtype=torch.uint8, device="cuda")
     st = torch.cuda.current_stream().cuda_stream
     p = lambda t: t.data_ptr()
 
     def cum():
-        _lib.check("gla_cumsum_f32", lib.gla_cumsum_f32(st, p(g), None, p(dst), B, T, H * D, 0))
+        _lib.check("gla_cumsum_f32", lib.gla_cumsum_f32_ws(st, p(g), None, p(dst), B, T, H * D, 0, p(ws), ws.numel()))
 
     def rnn():
         _lib.check("gla_rnn_scan_f32", lib.gla_rnn_scan_f32(st, p(a), p(kv), None, None, p(oa), p(ob), B * H, N, D,

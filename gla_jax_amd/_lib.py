@@ -22,6 +22,8 @@ SIGNATURES = {
     "gla_abi_version": (_int, []),
     "gla_status_string": (ctypes.c_char_p, [_int]),
     "gla_cumsum_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int]),
+    "gla_cumsum_workspace_bytes": (_sz, [_i64] * 3),
+    "gla_cumsum_f32_ws": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _sz]),
     "gla_rnn_scan_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int]),
     "gla_recurrent_fwd": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int] + [_vp] * 7),
     "gla_recurrent_bwd": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _int, _int] + [_vp] * 13),

@@ -169,6 +169,92 @@ __global__ __launch_bounds__(WAVES * 64) void cumsum_cached_kernel(const float *
     }
 }
 
+// Long rows (64 columns and more, a multiple of 4): a block owns a stretch of NG * ROWS rows of 4 CL neighbouring columns, a
+// lane 4 columns (16 bytes per access) of ROWS rows, held in registers from the only read of the source to the store.
+// An axis longer than a block's stretch takes two launches: SUMS leaves every stretch's column sums (all but the last's) in
+// `partial`, [n_outer][stretches][n_inner], and the second launch, whose source then lies in the last-level cache, adds those
+// in front of its own stretch.
+// Bound by memory.  The kernels above read row pieces of 64 and 256 bytes and run few blocks where the axis is long; here a
+// piece is 512 bytes and the axis fills the grid (fp32, sources and results not in cache, us before / after and at the rate of
+// a copy): 128 x [128,768] 27.3 / 22.7 / 20.4, 4 x [4096,768] 35.8 / 28.7 / 20.4, [32768,1024] 312 / 81 / 54,
+// 32 x [1024,512] 75 / 40 / 27, 3 x [1120,768] 62 / 10.2 / 4.2, 512 x [32,768] 26.5 / 21.2 / 20.4.
+template <int CL, int WAVES, int ROWS, bool SUMS>
+__global__ __launch_bounds__(WAVES * 64) void cumsum_rows_kernel(const float *__restrict__ src, const float *__restrict__ init,
+                                                                 float *__restrict__ dst, float *__restrict__ partial,
+                                                                 int64_t t_len, int64_t n_inner, int tiles, int stretches,
+                                                                 int reverse)
+{
+    constexpr int NG = WAVES * 64 / CL;            // groups of ROWS rows
+    __shared__ f32x4 totals[NG][CL], before[NG][CL];
+    const int cl = threadIdx.x % CL, grp = threadIdx.x / CL;
+    const int tile = blockIdx.x % tiles, s = blockIdx.x / tiles;
+    const int64_t col = ((int64_t)tile * CL + cl) * 4, outer = blockIdx.y;
+    const bool valid = col < n_inner;
+    const int64_t r0 = ((int64_t)s * NG + grp) * ROWS;
+    const int64_t left = valid ? t_len - r0 : 0;
+    const int len = left < 0 ? 0 : (left < ROWS ? (int)left : ROWS);
+    const int64_t step = reverse ? -n_inner : n_inner;
+    const int64_t at = len ? (outer * t_len + (reverse ? t_len - 1 - r0 : r0)) * n_inner + col : 0;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+    f32x4 a[ROWS];
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+        a[u] = zero;
+        if (u < len) a[u] = *reinterpret_cast<const f32x4 *>(src + at + u * step);
+    }
+    f32x4 pre = zero;
+    if (!SUMS && valid)
+        for (int w = grp; w < s; w += NG)
+            pre += *reinterpret_cast<const f32x4 *>(partial + (outer * stretches + w) * n_inner + col);
+    f32x4 sum = zero;
+#pragma unroll
+    for (int u = 0; u < ROWS; u += 4) sum += (a[u] + a[u + 1]) + (a[u + 2] + a[u + 3]);
+    totals[grp][cl] = sum;
+    if (!SUMS) before[grp][cl] = pre;
+    __syncthreads();
+    if (SUMS) {
+        if (grp != 0 || !valid) return;
+#pragma unroll
+        for (int w = 1; w < NG; ++w) sum += totals[w][cl];
+        *reinterpret_cast<f32x4 *>(partial + (outer * stretches + s) * n_inner + col) = sum;
+        return;
+    }
+    f32x4 run = zero;
+    if (init && valid) run = *reinterpret_cast<const f32x4 *>(init + outer * n_inner + col);
+    if (s > 0)
+#pragma unroll
+        for (int w = 0; w < NG; ++w) run += before[w][cl];
+    for (int w = 0; w < grp; ++w) run += totals[w][cl];
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+        run += a[u];
+        if (u < len) *reinterpret_cast<f32x4 *>(dst + at + u * step) = run;
+    }
+}
+
+template <int CL, int WAVES, int ROWS>
+static void launch_cumsum_rows(hipStream_t st, const float *src, const float *init, float *dst, float *partial, int64_t n_outer,
+                               int64_t t_len, int64_t n_inner, int reverse)
+{
+    constexpr int64_t kStretch = WAVES * 64 / CL * ROWS;
+    const int64_t tiles = (n_inner / 4 + CL - 1) / CL, stretches = (t_len + kStretch - 1) / kStretch;
+    if (stretches > 1)
+        hipLaunchKernelGGL((cumsum_rows_kernel<CL, WAVES, ROWS, true>), dim3((unsigned)(tiles * (stretches - 1)), (unsigned)n_outer),
+                           dim3(WAVES * 64), 0, st, src, init, dst, partial, t_len, n_inner, (int)tiles, (int)stretches, reverse);
+    hipLaunchKernelGGL((cumsum_rows_kernel<CL, WAVES, ROWS, false>), dim3((unsigned)(tiles * stretches), (unsigned)n_outer),
+                       dim3(WAVES * 64), 0, st, src, init, dst, partial, t_len, n_inner, (int)tiles, (int)stretches, reverse);
+}
+
+constexpr int64_t kRowsOneLaunch = 256;        // rows that one block holds
+// Axes of fewer than 32 rows leave most of a block idle, rows of fewer than 64 columns most of its lanes; the upper limits
+// keep the grid's size and the byte counts in range.
+static inline bool rows_kernel_fits(int64_t t_len, int64_t n_inner)
+{
+    return t_len >= 32 && n_inner >= 64 && n_inner % 4 == 0 && n_inner <= (1 << 24) && t_len <= (1 << 24) &&
+           t_len * n_inner <= ((int64_t)1 << 36);
+}
+
 // One thread = one (k, W consecutive v) strip of the state, walked over T in registers; the loads
 // of step n do not depend on the recurrence, so UNROLL of them are kept in flight.  W = 4 (one
 // 16-byte access per step) when V is a multiple of 4, W = 1 for every other V.
@@ -230,13 +316,46 @@ __global__ __launch_bounds__(256) void rnn_scan_kernel(const float *__restrict__
 
 }  // namespace gla
 
+extern "C" size_t gla_cumsum_workspace_bytes(int64_t n_outer, int64_t t_len, int64_t n_inner)
+{
+    if (n_outer <= 0 || n_outer > 65535 || t_len <= gla::kRowsOneLaunch || !gla::rows_kernel_fits(t_len, n_inner)) return 0;
+    return (size_t)(n_outer * ((t_len + 127) / 128) * n_inner) * sizeof(float);
+}
+
 extern "C" int gla_cumsum_f32(void *stream, const float *src, const float *init, float *dst,
                               int64_t n_outer, int64_t t_len, int64_t n_inner, int reverse)
 {
+    return gla_cumsum_f32_ws(stream, src, init, dst, n_outer, t_len, n_inner, reverse, nullptr, 0);
+}
+
+extern "C" int gla_cumsum_f32_ws(void *stream, const float *src, const float *init, float *dst,
+                                 int64_t n_outer, int64_t t_len, int64_t n_inner, int reverse, void *workspace,
+                                 size_t workspace_bytes)
+{
     if (!src || !dst) return GLA_ERR_NULL;
     if (n_outer <= 0 || t_len <= 0 || n_inner <= 0 || n_outer > 65535) return GLA_ERR_SHAPE;
-    dim3 grid((unsigned)((n_inner + 63) / 64), (unsigned)n_outer);
+    if (workspace && workspace_bytes < gla_cumsum_workspace_bytes(n_outer, t_len, n_inner)) return GLA_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t)stream;
+    if (gla::rows_kernel_fits(t_len, n_inner) && gla::aligned16(src) && gla::aligned16(dst) && (!init || gla::aligned16(init))) {
+        // One launch where a block of 4 or 8 waves holds the axis: 64 x [256,768] 24.7 us (two launches 29.7, before 26.3).
+        // Otherwise stretches of 128 rows, or of 256 rows and half as many columns where 128 leave fewer than two blocks per
+        // compute unit ([32768,128] 13.0 against 18.4 us, but 16 x [4096,512] 82 against 74).
+        if (t_len <= 128) {
+            gla::launch_cumsum_rows<32, 4, 16>(st, src, init, dst, nullptr, n_outer, t_len, n_inner, reverse);
+            return gla::launch_status();
+        }
+        if (t_len <= gla::kRowsOneLaunch) {
+            gla::launch_cumsum_rows<32, 8, 16>(st, src, init, dst, nullptr, n_outer, t_len, n_inner, reverse);
+            return gla::launch_status();
+        }
+        if (workspace && gla::aligned16(workspace)) {
+            const int64_t blocks = (t_len + 127) / 128 * ((n_inner + 127) / 128) * n_outer;
+            auto launch = blocks <= 512 ? gla::launch_cumsum_rows<16, 4, 16> : gla::launch_cumsum_rows<32, 4, 16>;
+            launch(st, src, init, dst, (float *)workspace, n_outer, t_len, n_inner, reverse);
+            return gla::launch_status();
+        }
+    }
+    dim3 grid((unsigned)((n_inner + 63) / 64), (unsigned)n_outer);
     // long axis over few columns: cut the axis finer so that the grid fills the machine
     if (t_len >= 2048 && (int64_t)grid.x * grid.y < 1024) {
         dim3 fine((unsigned)((n_inner + 15) / 16), (unsigned)n_outer);

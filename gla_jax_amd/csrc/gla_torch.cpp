@@ -296,10 +296,12 @@ std::optional<Tensor> cumsum(const Tensor &src, int64_t axis, const std::optiona
             if (init->size(i) != src.size(i < axis ? i : i + 1)) return std::nullopt;
     }
     const c10::DeviceGuard guard(src.device());
-    Tensor dst = at::empty_like(src);
-    check("gla_cumsum_f32", gla_cumsum_f32(stream_of(src), (const float *)src.data_ptr(),
-                                           init ? (const float *)init->data_ptr() : nullptr, (float *)dst.data_ptr(), outer,
-                                           src.size(axis), inner, reverse));
+    Tensor dst = at::empty_like(src), ws;
+    const size_t nws = gla_cumsum_workspace_bytes(outer, src.size(axis), inner);
+    if (nws) ws = bytes_like(nws, src);
+    check("gla_cumsum_f32", gla_cumsum_f32_ws(stream_of(src), (const float *)src.data_ptr(),
+                                              init ? (const float *)init->data_ptr() : nullptr, (float *)dst.data_ptr(), outer,
+                                              src.size(axis), inner, reverse, nws ? ws.data_ptr() : nullptr, nws));
     return dst;
 }
 

@@ -65,6 +65,11 @@ const char *gla_status_string(int status);
 /* Replaces cumsum_recursive(src, axis, init, reverse) (ops.py:234-284; kernel ops.py:152-162).
  * src/dst are viewed as [n_outer, t_len, n_inner] float32, the scan runs along t_len in fp32;
  * init is [n_outer, n_inner] or NULL (zero).  reverse != 0 sums from the far end.  dst must not alias src. */
+/* The _ws form takes a workspace (16-byte aligned, gla_cumsum_workspace_bytes; 0: none is needed and it may be NULL): a long axis
+ * then runs as stretches side by side.  Without one, or with arrays that are not 16-byte aligned, it is gla_cumsum_f32. */
+size_t gla_cumsum_workspace_bytes(int64_t n_outer, int64_t t_len, int64_t n_inner);
+int gla_cumsum_f32_ws(void *stream, const float *src, const float *init, float *dst,
+                      int64_t n_outer, int64_t t_len, int64_t n_inner, int reverse, void *workspace, size_t workspace_bytes);
 int gla_cumsum_f32(void *stream, const float *src, const float *init, float *dst,
                    int64_t n_outer, int64_t t_len, int64_t n_inner, int reverse);
 

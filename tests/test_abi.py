@@ -119,6 +119,8 @@ def test_entry_points_reject_bad_arguments_without_touching_the_gpu():
     assert lib.gla_recurrent_fwd(None, 1, 8, 1, 64, 64, 1, 1, 1, 0, None, a, a, a, a, a, a) == -1
     # shapes / dtypes
     assert lib.gla_cumsum_f32(None, a, None, a, 0, 8, 8, 0) == -2
+    assert lib.gla_cumsum_workspace_bytes(4, 4096, 768) == 4 * 32 * 768 * 4 and lib.gla_cumsum_workspace_bytes(4, 256, 768) == 0
+    assert lib.gla_cumsum_f32_ws(None, a, None, a, 4, 4096, 768, 0, a, 64) == -5
     assert lib.gla_recurrent_fwd(None, 1, 8, 1, 48, 48, 1, 1, 1, 0, a, a, a, a, a, a, a) == -2
     assert lib.gla_recurrent_fwd(None, 1, 8, 1, 64, 32, 1, 1, 1, 0, a, a, a, a, a, a, a) == -2   # DK != DV
     assert lib.gla_recurrent_fwd(None, 1, 8, 1, 64, 64, 5, 1, 1, 0, a, a, a, a, a, a, a) == -3
