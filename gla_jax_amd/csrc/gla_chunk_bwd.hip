@@ -625,9 +625,10 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
             }
             st8_row_once<D, DM>(dk + rowoff + fo, c, pack8<TG>(o), live);
         }
-        // -- dv: state term K~ dS' first, then the own and the later sub-blocks
+        // -- dv: state term K~ dS', and the own and the later sub-blocks in a sum of their own: the products differ in depth
+        // (see mma_t2), the vector addition at the end waits for both
         {
-            f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, rows[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
             for (int k2 = 0; k2 < KS; ++k2) {
 #pragma unroll
@@ -644,15 +645,15 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                     for (int tt = 0; tt < 2; ++tt) {
                         const T4 oa = lds_tr4(tO + L.k4 + fo + 4 * tt + 16 * I * LS, LS);
                         if constexpr (sizeof(T) == 2) {
-                            if (I == w) acc[tt] = mma_t(oa, Acl, acc[tt]);
+                            if (I == w) rows[tt] = mma_t(oa, Acl, rows[tt]);
                         }
-                        acc[tt] = mma_t(oa, b4, acc[tt]);
+                        rows[tt] = mma_t(oa, b4, rows[tt]);
                     }
                 }
             }
             float o[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = acc[e >> 2][e & 3];
+            for (int e = 0; e < 8; ++e) o[e] = acc[e >> 2][e & 3] + rows[e >> 2][e & 3];
             st8_row_once<D, DM>(dv + rowoff + fo, c, pack8<TG>(o), live);
         }
         // -- dL of the slice is complete: reverse cumsum inside the sub-block (gla.py:616-617), then, once

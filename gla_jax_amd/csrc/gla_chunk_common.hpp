@@ -60,9 +60,10 @@ __device__ __forceinline__ f32x4 mma_t(f32x4 a, f32x4 b, f32x4 c)
 // contracted values, and a lane's k-slots may hold any 8 of them as long as A and B agree, so the operands of two
 // 16-token contractions side by side fill the instruction of twice the depth: a third to a half of the matrix instructions of
 // recurrent_gla's kernels (B4 T4096 H16 D128: the two backward sweeps 238 -> 226 and 349 -> 325 us).
-// Never add a mma_t to the result of a mma_d or mma_t2 right behind it: the compiler leaves no wait between the two
-// instructions, and the shallower one then takes the sum too early (seen: the low half of the accumulators without the last
-// product).  recurrent_gla's kernels use the deeper instruction alone; elsewhere LDS reads or arithmetic lie between.
+// Never add a mma_t to the result of a mma_d or mma_t2: the compiler leaves no wait between the two instructions, and where
+// nothing else happens to lie between them the shallower one takes the sum too early (seen: the low half of the accumulators
+// without the last product).  recurrent_gla's kernels use the deeper instruction alone; chunk_gla's have a vector operation on
+// the sum between the two depths, which the compiler waits for, or keep two sums.
 __device__ __forceinline__ f32x4 mma_t2(bf16x4 a0, bf16x4 a1, bf16x4 b0, bf16x4 b1, f32x4 c)
 {
     return mma_d(__builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7),
