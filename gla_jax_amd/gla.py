@@ -114,20 +114,16 @@ def _native(entry, arrays, *args):
 def _merge_mapped(info, in_dims, tensors):
     """vmap rule helper: every Function below takes canonical arrays with ONE batch axis in front, so a mapped
     call is the same call with the mapped axis folded into that batch axis.  Unmapped arguments are
-    broadcast.  Flat byte buffers (the residual of chunk_gla) carry no axis of their own and pass through."""
+    broadcast."""
     out = []
     for a, d in zip(tensors, in_dims):
-        if a.dtype == torch.uint8:
-            out.append(a)
-            continue
         a = a.unsqueeze(0).expand(info.batch_size, *a.shape) if d is None else a.movedim(d, 0)
         out.append(a.reshape((a.shape[0] * a.shape[1],) + tuple(a.shape[2:])))
     return out
 
 
 def _split_mapped(info, outs):
-    return tuple(o if o.dtype == torch.uint8 else o.reshape((info.batch_size, -1) + tuple(o.shape[1:]))
-                 for o in outs)
+    return tuple(o.reshape((info.batch_size, -1) + tuple(o.shape[1:])) for o in outs)
 
 
 def _no_double_backward(name):
@@ -152,7 +148,8 @@ def _chunk_forward(h0, g, v, k, q, chunk_size, residual):
         _lib.check("gla_chunk_fwd", -7)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=v.device)
     # without a residual (nothing to differentiate) the scan skips the [dk][dv] copy of the chunk states
-    states = torch.empty(st_bytes, dtype=torch.uint8, device=v.device) if residual else None
+    # (the library's own layout over the whole batch; cut into B rows of bytes it maps over the batch axis as arrays do)
+    states = torch.empty(B, -(-st_bytes // B), dtype=torch.uint8, device=v.device) if residual else None
     hT = torch.empty_like(h0)
     out = torch.empty_like(v)
     rc = lib.gla_chunk_fwd(_stream(), B, T, H, DK, DV, chunk_size, dt, _DT[h0.dtype], _ptr(h0), _ptr(g), _ptr(v),
@@ -193,8 +190,7 @@ class _ChunkGLA(torch.autograd.Function):
     @staticmethod
     def vmap(info, in_dims, *args):
         outs = _ChunkGLA.apply(*_merge_mapped(info, in_dims[:5], args[:5]), args[5])
-        # the residual is one flat buffer over the merged batch; it carries no mapped axis of its own
-        return _split_mapped(info, outs), (0, 0, None)
+        return _split_mapped(info, outs), (0, 0, 0)
 
 
 class _ChunkGLABwd(torch.autograd.Function):
@@ -232,8 +228,15 @@ class _ChunkGLABwd(torch.autograd.Function):
 
     @staticmethod
     def vmap(info, in_dims, *args):
-        outs = _ChunkGLABwd.apply(*_merge_mapped(info, in_dims[:7], args[:7]), args[7])
-        return _split_mapped(info, outs), (0,) * 5
+        if in_dims[0] is not None:       # the forward was mapped as well: its states are those of the merged batch
+            outs = _ChunkGLABwd.apply(*_merge_mapped(info, in_dims[:7], args[:7]), args[7])
+            return _split_mapped(info, outs), (0,) * 5
+        if any(d is not None for d in in_dims[1:5]):
+            raise RuntimeError("chunk_gla: the rows are mapped and the states of their forward are not")
+        # several cotangents of one forward: its states fit the batch as it is, not the merged one
+        outs = [_ChunkGLABwd.apply(*args[:5], *(a if d is None else a.select(d, i) for a, d in zip(args[5:7], in_dims[5:7])),
+                                   args[7]) for i in range(info.batch_size)]
+        return tuple(torch.stack(o) for o in zip(*outs)), (0,) * 5
 
 
 def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_t: int = 64,
