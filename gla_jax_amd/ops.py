@@ -77,6 +77,8 @@ def rnn_recursive(log_fgate: torch.Tensor, kv: torch.Tensor,
     Bn, T, K, V = b.shape
     if tuple(a.shape) != (Bn, T, K):
         raise AssertionError(f"log_fgate shape {tuple(log_fgate.shape)} does not match kv")  # ops.py:405
+    if init_kv is not None and (init_log_fgate.numel() != Bn * K or init_kv.numel() != Bn * K * V):
+        raise AssertionError(f"init shapes {tuple(init_log_fgate.shape)}, {tuple(init_kv.shape)} do not match kv")
     af = a.contiguous().to(torch.float32)
     bf = b.contiguous().to(torch.float32)
     ia = ib = None
