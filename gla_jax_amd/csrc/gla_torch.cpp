@@ -59,20 +59,27 @@ Dims dims_of(const Tensor &k)
 }
 
 // The arrays can go to the kernels as they are: see gla.py's _prep for the contract.
-bool canonical(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q)
+bool canonical_rows(const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q)
 {
-    for (const Tensor *t : {&h0, &g, &v, &k, &q})
+    for (const Tensor *t : {&g, &v, &k, &q})
         if (!dense_on_gpu(*t) || t->device() != k.device()) return false;
     const auto s = k.sizes();
+    if (s.size() < 3 || q.sizes() != s || g.sizes() != s || v.sizes() != s) return false;
+    return g.scalar_type() == at::kFloat && known(v.scalar_type()) && k.scalar_type() == v.scalar_type() &&
+           q.scalar_type() == v.scalar_type();
+}
+std::vector<int64_t> state_sizes(const Tensor &k)
+{
+    std::vector<int64_t> s = k.sizes().vec();
     const size_t n = s.size();
-    if (n < 3 || q.sizes() != s || g.sizes() != s || v.sizes() != s) return false;
-    if (g.scalar_type() != at::kFloat || !known(h0.scalar_type()) || !known(v.scalar_type())) return false;
-    if (k.scalar_type() != v.scalar_type() || q.scalar_type() != v.scalar_type()) return false;
-    const auto hs = h0.sizes();
-    if (hs.size() != n || hs[n - 1] != s[n - 1] || hs[n - 2] != s[n - 1] || hs[n - 3] != s[n - 2]) return false;
-    for (size_t i = 0; i + 3 < n; ++i)
-        if (hs[i] != s[i]) return false;
-    return true;
+    s[n - 3] = s[n - 2];
+    s[n - 2] = s[n - 1];
+    return s;
+}
+bool canonical(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q)
+{
+    return canonical_rows(g, v, k, q) && dense_on_gpu(h0) && h0.device() == k.device() && known(h0.scalar_type()) &&
+           h0.sizes() == at::IntArrayRef(state_sizes(k));
 }
 
 Tensor bytes_like(size_t n, const Tensor &t) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
@@ -132,19 +139,29 @@ variable_list chunk_backward(const Tensor &states, const Tensor &g, const Tensor
     return {dh0, dg, dv, dk, dq};
 }
 
+// What autograd saved: a saved-tensor hook may hand it back in another layout (taken as it is, the kernels would read other
+// values), or as another array altogether (refused).
+void check_saved(bool as_saved)
+{
+    TORCH_CHECK(as_saved, "a saved-tensor hook handed back an array of another type, shape or device");
+}
+variable_list saved_dense(AutogradContext *ctx)
+{
+    variable_list s = ctx->get_saved_variables();
+    for (Tensor &t : s)
+        if (t.defined()) t = t.contiguous();
+    return s;
+}
+bool holds(const Tensor &bytes, size_t n, const Tensor &like)
+{
+    return bytes.scalar_type() == at::kByte && bytes.device() == like.device() && (size_t)bytes.numel() >= n;
+}
 // a cotangent as the kernels take it: zeros where autograd has none, dense, in the type of what it belongs to
 Tensor cotangent(const Tensor &d, at::IntArrayRef sizes, at::ScalarType type, const Tensor &like)
 {
     if (!d.defined()) return at::zeros(sizes, like.options().dtype(type));
+    check_saved(d.sizes() == sizes && d.device() == like.device());
     return d.to(type).contiguous();
-}
-std::vector<int64_t> state_sizes(const Tensor &k)
-{
-    std::vector<int64_t> s = k.sizes().vec();
-    const size_t n = s.size();
-    s[n - 3] = s[n - 2];
-    s[n - 2] = s[n - 1];
-    return s;
 }
 
 // The backward rules as functions of their own, used where a graph of the gradients is asked for: what they return can
@@ -171,8 +188,11 @@ struct Chunk : torch::autograd::Function<Chunk> {      // gla.py:483-550, 552-62
     }
     static variable_list backward(AutogradContext *ctx, variable_list d)
     {
-        const auto s = ctx->get_saved_variables();
+        const variable_list s = saved_dense(ctx);
         const int64_t chunk = ctx->saved_data["chunk"].toInt();
+        check_saved(canonical_rows(s[1], s[2], s[3], s[4]));
+        const Dims n = dims_of(s[3]);
+        check_saved(holds(s[0], gla_chunk_states_bytes(n.B, n.T, n.H, n.D, n.D, chunk, code(s[2])), s[3]));
         const Tensor dhT = cotangent(d[0], state_sizes(s[3]), (at::ScalarType)ctx->saved_data["hidden"].toInt(), s[3]);
         const Tensor dout = cotangent(d[1], s[2].sizes(), s[2].scalar_type(), s[2]);
         variable_list r = at::GradMode::is_enabled() ? ChunkBackward::apply(s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk)
@@ -248,7 +268,10 @@ struct Recurrent : torch::autograd::Function<Recurrent> {      // gla.py:99-170,
     }
     static variable_list backward(AutogradContext *ctx, variable_list d)
     {
-        const auto s = ctx->get_saved_variables();
+        const variable_list s = saved_dense(ctx);
+        check_saved(canonical(s[0], s[1], s[2], s[3], s[4]) && dense_on_gpu(s[5]) && s[5].sizes() == s[0].sizes());
+        const Dims n = dims_of(s[3]);
+        check_saved(!s[6].defined() || holds(s[6], gla_recurrent_residual_bytes(n.B, n.T, n.H, n.D, n.D, code(s[2])), s[3]));
         const bool reverse = ctx->saved_data["reverse"].toBool(), out_fp32 = ctx->saved_data["out_fp32"].toBool();
         const Tensor dhT = cotangent(d[0], s[0].sizes(), s[0].scalar_type(), s[0]);
         const Tensor dout = cotangent(d[1], s[2].sizes(), out_fp32 ? at::kFloat : s[2].scalar_type(), s[2]);
