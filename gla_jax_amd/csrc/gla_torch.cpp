@@ -2,13 +2,14 @@
 // element type): argument checks, buffers, launches and the autograd rules in one native call.  The same path in Python
 // took 23 us for a forward and 105 to 210 us for a forward and backward, more than the kernels of a small call; here it
 // is about a third of that.  Everything else (other layouts and types, function transforms, error messages) stays in
-// gla.py, which calls this again once the arrays are converted.
+// gla.py, which calls this again once the arrays are converted, and whose backward rules are called where a transform is active.
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <ATen/ops/zeros.h>
 #include <ATen/ops/zeros_like.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -113,7 +114,9 @@ ChunkOut chunk_forward(const Tensor &h0, const Tensor &g, const Tensor &v, const
     const size_t nws = gla_chunk_fwd_workspace_bytes(d.B, d.T, d.H, d.D, d.D, chunk, dt);
     const size_t nst = residual ? gla_chunk_states_bytes(d.B, d.T, d.H, d.D, d.D, chunk, dt) : 0;
     if (nws == 0) check("gla_chunk_fwd", GLA_ERR_UNSUPPORTED);
-    ChunkOut r{at::empty_like(h0), at::empty_like(v), residual ? bytes_like(nst, v) : Tensor()};
+    ChunkOut r{at::empty_like(h0), at::empty_like(v), Tensor()};
+    // as B rows of bytes, which is how gla.py's rules map them
+    if (residual) r.states = bytes_like((nst + d.B - 1) / d.B * d.B, v).view({d.B, -1});
     const Tensor ws = bytes_like(nws, v);
     check("gla_chunk_fwd",
           gla_chunk_fwd(stream_of(k), d.B, d.T, d.H, d.D, d.D, chunk, dt, code(h0), h0.data_ptr(), (const float *)g.data_ptr(),
@@ -156,12 +159,28 @@ bool holds(const Tensor &bytes, size_t n, const Tensor &like)
 {
     return bytes.scalar_type() == at::kByte && bytes.device() == like.device() && (size_t)bytes.numel() >= n;
 }
+// A function transform can be active in the backward alone (torch.func.vmap over torch.autograd.grad): the cotangents then
+// are wrappers without memory of their own, and the rules of gla.py, which know how to map, take over.  The older mapping
+// behind is_grads_batched reaches no rule of a custom function.
+bool transforms_active()
+{
+    return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
 // a cotangent as the kernels take it: zeros where autograd has none, dense, in the type of what it belongs to
 Tensor cotangent(const Tensor &d, at::IntArrayRef sizes, at::ScalarType type, const Tensor &like)
 {
     if (!d.defined()) return at::zeros(sizes, like.options().dtype(type));
     check_saved(d.sizes() == sizes && d.device() == like.device());
+    TORCH_CHECK_NOT_IMPLEMENTED(d.has_storage() || transforms_active(), "batched cotangents (is_grads_batched, jacobian with "
+                                "vectorize=True) are not provided: map torch.autograd.grad by torch.func.vmap");
     return d.to(type).contiguous();
+}
+
+template <typename... Args> variable_list python_rule(const char *name, Args &&...args)
+{
+    const py::gil_scoped_acquire gil;
+    const py::object r = py::module_::import("gla_jax_amd.gla").attr(name).attr("apply")(std::forward<Args>(args)...);
+    return r.cast<variable_list>();
 }
 
 // The backward rules as functions of their own, used where a graph of the gradients is asked for: what they return can
@@ -195,8 +214,9 @@ struct Chunk : torch::autograd::Function<Chunk> {      // gla.py:483-550, 552-62
         check_saved(holds(s[0], gla_chunk_states_bytes(n.B, n.T, n.H, n.D, n.D, chunk, code(s[2])), s[3]));
         const Tensor dhT = cotangent(d[0], state_sizes(s[3]), (at::ScalarType)ctx->saved_data["hidden"].toInt(), s[3]);
         const Tensor dout = cotangent(d[1], s[2].sizes(), s[2].scalar_type(), s[2]);
-        variable_list r = at::GradMode::is_enabled() ? ChunkBackward::apply(s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk)
-                                                     : chunk_backward(s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk);
+        variable_list r = transforms_active() ? python_rule("_ChunkGLABwd", s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk)
+                          : at::GradMode::is_enabled() ? ChunkBackward::apply(s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk)
+                                                       : chunk_backward(s[0], s[1], s[2], s[3], s[4], dhT, dout, chunk);
         r.emplace_back();
         return r;
     }
@@ -275,7 +295,9 @@ struct Recurrent : torch::autograd::Function<Recurrent> {      // gla.py:99-170,
         const bool reverse = ctx->saved_data["reverse"].toBool(), out_fp32 = ctx->saved_data["out_fp32"].toBool();
         const Tensor dhT = cotangent(d[0], s[0].sizes(), s[0].scalar_type(), s[0]);
         const Tensor dout = cotangent(d[1], s[2].sizes(), out_fp32 ? at::kFloat : s[2].scalar_type(), s[2]);
-        variable_list r = at::GradMode::is_enabled()
+        variable_list r = transforms_active()
+                              ? python_rule("_RecurrentGLABwd", s[0], s[1], s[2], s[3], s[4], s[5], dhT, dout, reverse, out_fp32)
+                          : at::GradMode::is_enabled()
                               ? RecurrentBackward::apply(s[0], s[1], s[2], s[3], s[4], s[5], std::optional<Tensor>(s[6]), dhT, dout, reverse, out_fp32)
                               : recurrent_backward(s[0], s[1], s[2], s[3], s[4], s[5], s[6], dhT, dout, reverse, out_fp32);
         r.resize(7);

@@ -73,3 +73,32 @@ def test_mapped_cotangents_of_a_mapped_forward(name):
     for a, b in zip(shared[1:], each[1:]):
         # the sum over the mapped axis is formed in the element type by both, from the same two terms
         assert torch.equal(a, b) or (a.float() - b.float()).norm() <= 2 ** -8 * b.float().norm()
+
+
+@pytest.mark.parametrize("name, D", [("chunk_gla", 64), ("recurrent_gla", 64), ("recurrent_gla", 8), ("recurrent_gla_naive", 128)])
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_mapped_backward_of_a_plain_forward(name, D, create_graph):
+    """The transform is active in the backward alone.  Sequences of 320 steps run as segments in recurrent_gla."""
+    fn = _bind(name)
+    for shape in ((2, 64, 2, D), (1, 320, 1, D)):
+        dev = [t.requires_grad_(True) for t in _inputs(*shape, seed=35)]
+        outs = fn(*dev)
+        ct = _cotangents(3, outs, 36)
+        grad = lambda y, *c: torch.autograd.grad(y, dev, c, retain_graph=True, create_graph=create_graph)
+        got = torch.func.vmap(lambda a, b: grad(outs, a, b))(*ct)
+        only_out = torch.func.vmap(lambda b: grad(outs[1], b))(ct[1])
+        for i in range(3):
+            for mapped, single in ((got, grad(outs, ct[0][i], ct[1][i])), (only_out, grad(outs[1], ct[1][i]))):
+                for a, b in zip(mapped, single):
+                    if shape[1] == 64 or name == "chunk_gla":
+                        assert torch.equal(a[i], b)
+                    # three times the sequences are cut into other segments: sums in another order, rounded once to bf16
+                    assert (a[i].float() - b.float()).norm() <= 2 ** -8 * b.float().norm()
+
+
+@pytest.mark.parametrize("name", ["chunk_gla", "recurrent_gla"])
+def test_batched_cotangents_of_the_older_mapping_are_refused(name):
+    dev = [t.requires_grad_(True) for t in _inputs(1, 64, 1, 64, seed=37)]
+    outs = _bind(name)(*dev)
+    with pytest.raises(NotImplementedError, match="torch.func.vmap"):
+        torch.autograd.grad(outs, dev, _cotangents(3, outs, 38), is_grads_batched=True)
