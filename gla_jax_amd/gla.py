@@ -5,7 +5,7 @@
 405-439 and 26-47 of zhixuan-lin/gla-jax.  Arrays are torch tensors on the GPU; the forward and
 backward rules of the reference's `jax.custom_vjp` (gla.py:628-655, 362-388, 441) are
 autograd functions whose bodies are single calls into libgla_hip.so: native ones (csrc/gla_torch.cpp) where no function
-transform is active, the Python ones below where one is.  Batching: the
+transform or tracer is active, the Python ones below where one is.  Batching: the
 reference uses `jax.vmap` over a leading axis of all five arrays (gla.py:1335); here any number of
 leading axes may simply be present, and `torch.func.vmap` works through the functions' vmap rule.
 
@@ -97,6 +97,12 @@ def _twin(cls):
 
     Twin.__name__ = Twin.__qualname__ = cls.__name__ + "Twin"
     return Twin
+
+
+def _plain_call():
+    """No function transform and no tracer looks on: the native host side can take the call.  A tracer records a Function
+    as a call of it; of a native call it would record the buffers that it allocates, and replay those."""
+    return not _transforms_active() and torch._C._get_tracing_state() is None
 
 
 def _apply(cls, *args):
@@ -251,7 +257,7 @@ def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_
     if interpret:
         raise ValueError("interpret=True asks for the reference's CPU interpreter; this build has no CPU path")
     chunk_size = int(chunk_size)
-    native = not _transforms_active()
+    native = _plain_call()
     if native:
         done = _native("chunk", (hidden_init, log_fgate, value, key, query), chunk_size)
         if done is not None:
@@ -264,7 +270,7 @@ def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_
     if T % chunk_size:
         raise AssertionError(f"sequence length {T} is not a multiple of chunk_size {chunk_size}")
     hT, out = (_native("chunk", (h0, g, v, k, q), chunk_size) if native
-               else _ChunkGLA.apply(h0, g, v, k, q, chunk_size)[:2])
+               else _apply(_ChunkGLA, h0, g, v, k, q, chunk_size)[:2])
     return _as(hT, lead + (H, DK, DV), hidden_init.dtype), _as(out, lead + (T, H, DV), out.dtype)
 
 
@@ -359,7 +365,7 @@ class _RecurrentGLABwd(torch.autograd.Function):
 
 def _recurrent(hidden_init, log_fgate, value, key, query, reverse, out_fp32):
     reverse = bool(reverse)
-    native = not _transforms_active()
+    native = _plain_call()
     if native:
         done = _native("recurrent", (hidden_init, log_fgate, value, key, query), reverse, out_fp32)
         if done is not None:
@@ -376,7 +382,7 @@ def _recurrent(hidden_init, log_fgate, value, key, query, reverse, out_fp32):
         h0 = F.pad(h0, (0, pad, 0, pad))
         g, v, k, q = (F.pad(x, (0, pad)) for x in (g, v, k, q))
     hT, out = (_native("recurrent", (h0, g, v, k, q), reverse, out_fp32) if native
-               else _RecurrentGLA.apply(h0, g, v, k, q, reverse, out_fp32))
+               else _apply(_RecurrentGLA, h0, g, v, k, q, reverse, out_fp32))
     if pad:
         hT, out = hT[..., :DK, :DV], out[..., :DV]
     return _as(hT, lead + (H, DK, DV), hidden_init.dtype), _as(out, lead + (T, H, DV), out.dtype)

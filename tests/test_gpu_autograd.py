@@ -60,3 +60,20 @@ def test_checkpoint(name, use_reentrant):
     torch.autograd.backward(checkpoint(fn, *args, use_reentrant=use_reentrant), ct)
     for a, b in zip(args, want):
         assert torch.equal(a.grad, b)
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("grad", [False, True])
+def test_traced_call_computes_on_new_inputs(name, grad):
+    """torch.jit.trace records the call itself, not the buffers it fills."""
+    fn = _bind(name)
+    dev, ct = _problem(name, 44)
+    new = [t.detach().clone().requires_grad_(grad) for t in _problem(name, 45)[0]]
+    traced = torch.jit.trace(fn, tuple(t.detach().requires_grad_(grad) for t in dev), check_trace=False)
+    got, want = traced(*new), fn(*new)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    if grad:
+        for a, b in zip(torch.autograd.grad(got, new, ct), torch.autograd.grad(want, new, ct)):
+            # (the traced forward hands no segment states to its backward, which forms them again to the same bits)
+            assert torch.equal(a, b)
