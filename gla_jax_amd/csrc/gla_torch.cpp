@@ -23,19 +23,15 @@ using at::Tensor;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-// A status of the library, raised as gla_jax_amd._lib.GlaError where Python can see it.
-struct GlaFailure : std::runtime_error {
-    const char *fn;
-    int status;
-    GlaFailure(const char *f, int s)
-        : std::runtime_error(std::string(f) + " failed with status " + std::to_string(s) + ": " + gla_status_string(s)),
-          fn(f), status(s)
-    {
-    }
-};
+// A status of the library as gla_jax_amd._lib.GlaError.  The Python error itself is thrown: out of a backward the autograd
+// engine carries it to the caller as it is, while any exception of this file's own would arrive as a plain RuntimeError.
+PyObject *gla_error = nullptr;
 void check(const char *fn, int status)
 {
-    if (status != 0) throw GlaFailure(fn, status);
+    if (status == 0) return;
+    const py::gil_scoped_acquire gil;
+    PyErr_SetObject(gla_error, py::handle(gla_error)(fn, status, gla_status_string(status)).ptr());
+    throw py::error_already_set();
 }
 
 void *stream_of(const Tensor &t)
@@ -376,14 +372,7 @@ std::optional<std::pair<Tensor, Tensor>> rnn(const Tensor &a, const Tensor &b, c
 
 PYBIND11_MODULE(_gla_torch, m)
 {
-    static py::handle error = py::object(py::module_::import("gla_jax_amd._lib").attr("GlaError")).release();
-    py::register_exception_translator([](std::exception_ptr p) {
-        try {
-            if (p) std::rethrow_exception(p);
-        } catch (const GlaFailure &e) {
-            PyErr_SetObject(error.ptr(), py::object(error(e.fn, e.status, gla_status_string(e.status))).ptr());
-        }
-    });
+    gla_error = py::object(py::module_::import("gla_jax_amd._lib").attr("GlaError")).release().ptr();
     typedef py::call_guard<py::gil_scoped_release> NoGil;
     m.def("chunk", &chunk, NoGil());
     m.def("recurrent", &recurrent, NoGil());

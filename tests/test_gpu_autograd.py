@@ -77,3 +77,21 @@ def test_traced_call_computes_on_new_inputs(name, grad):
         for a, b in zip(torch.autograd.grad(got, new, ct), torch.autograd.grad(want, new, ct)):
             # (the traced forward hands no segment states to its backward, which forms them again to the same bits)
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_status_of_a_backward_reaches_the_caller(name, create_graph):
+    """A cotangent that is dense but not 16-byte aligned is refused by the library; the status arrives as it does in a forward."""
+    from gla_jax_amd._lib import GlaError
+    fn = _bind(name)
+    dev, ct = _problem(name, 46)
+    outs = fn(*dev)
+    shifted = torch.zeros(ct[1].numel() + 1, device="cuda", dtype=ct[1].dtype)[1:].view(ct[1].shape)
+    with pytest.raises(GlaError) as e:
+        torch.autograd.grad(outs[1], dev, shifted, create_graph=create_graph)
+    assert e.value.status == -6
+    shifted = torch.zeros(dev[4].numel() + 1, device="cuda", dtype=dev[4].dtype)[1:].view(dev[4].shape)
+    with pytest.raises(GlaError) as e:
+        fn(*dev[:4], shifted)
+    assert e.value.status == -6
