@@ -171,6 +171,23 @@ __device__ __forceinline__ float dpp_f32(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 
+// 4 x 4 transpose inside a quad of lanes: lane j holds row j before and column j after (and the other way round).
+__device__ __forceinline__ void quad_transpose(float (&x)[4])
+{
+    const int j = threadIdx.x & 3;
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float other = dpp_f32<kDppQuadXor1>(x[e ^ 1]);
+        y[e] = ((j ^ e) & 1) ? other : x[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float other = dpp_f32<kDppQuadXor2>(y[e ^ 2]);
+        x[e] = ((j ^ e) & 2) ? other : y[e];
+    }
+}
+
 __device__ __forceinline__ float shfl_xor_f32(float v, int mask)
 {
     return __shfl_xor(v, mask, 64);

@@ -78,22 +78,24 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
     // instructions per tile; with the products of mma_t2 B4 T4096 H16 D128 went from 234 to 222 us.  The lean form
     // writes no copy and keeps (dv x dk) tiles, dk = 16(nt0 + j) + r and dv = 16(wv + i NDV) + 4c + e, whose decay is
     // one value per lane and tile (four take registers that it does not have: 71.6 -> 75 us).
+    // In memory the four values lie in four rows.  Lanes of a quad read (write) four neighbours of one of them each and
+    // exchange: one access per lane and tile, as in the lean form.  Two- and four-byte accesses, four times as many, cost more
+    // than all else where sequences are short (forward alone, bf16, B*H = 1024, D = 128, us: T = 33 137 / 92, T = 128 213 / 146).
     f32x4 S[RT][NTW];
+    auto state_at = [&](int i, int nt) {
+        const int64_t tile = bh * D * D + (int64_t)(16 * (nt0 + nt)) * D + 16 * (wv + i * NDV);
+        return STATE ? tile + r * D + 4 * c : tile + (4 * c + (r & 3)) * D + (r & 12);
+    };
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
             S[i][nt] = f32x4{0.f, 0.f, 0.f, 0.f};   // no initial state given: zeros (the lean pass of a segment)
             if (h0) {
-                if constexpr (STATE) {
-                    float t4[4];
-                    load_hidden<4>(h0, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + r) * D + 16 * (wv + i * NDV) + 4 * c, t4);
-                    S[i][nt] = f32x4{t4[0], t4[1], t4[2], t4[3]};
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        S[i][nt][e] = load_hidden1(h0, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + 4 * c + e) * D + 16 * (wv + i * NDV) + r);
-                }
+                float t4[4];
+                load_hidden<4>(h0, hdt, state_at(i, nt), t4);
+                if constexpr (!STATE) quad_transpose(t4);
+                S[i][nt] = f32x4{t4[0], t4[1], t4[2], t4[3]};
             }
         }
     auto publish_state = [&]() {
@@ -305,14 +307,9 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
     for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
-            if constexpr (STATE) {
-                float t4[4] = {S[i][nt][0], S[i][nt][1], S[i][nt][2], S[i][nt][3]};
-                store_hidden<4>(hT, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + r) * D + 16 * (wv + i * NDV) + 4 * c, t4);
-                continue;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                store_hidden1(hT, hdt, bh * D * D + (int64_t)(16 * (nt0 + nt) + 4 * c + e) * D + 16 * (wv + i * NDV) + r, S[i][nt][e]);
+            float t4[4] = {S[i][nt][0], S[i][nt][1], S[i][nt][2], S[i][nt][3]};
+            if constexpr (!STATE) quad_transpose(t4);
+            store_hidden<4>(hT, hdt, state_at(i, nt), t4);
         }
 }
 

@@ -52,20 +52,44 @@ def test_the_scan_sees_a_mixed_sum():
     assert _mixed_depth_sums([head, shallow, shallow, deep, deep]) == []
 
 
-def test_no_sum_goes_from_a_deep_product_to_a_shallow_one(tmp_path):
-    """A 16-value product that adds to the result of a 32-value one takes the sum too early when the two are close, and the
-    compiler puts no wait between them (gla_chunk_common.hpp, mma_t2): no kernel may hold such a pair, however far apart."""
+@pytest.fixture(scope="module")
+def listings(tmp_path_factory):
+    """The disassembly of the built library, one text per code object."""
     _lib.load()
     if not os.path.exists(OBJDUMP):
         pytest.skip("needs ROCm's llvm-objdump")
+    tmp_path = tmp_path_factory.mktemp("code")
     lib = shutil.copy(_lib.LIB_PATH, tmp_path / "lib.so")
     subprocess.run([OBJDUMP, "--offloading", str(lib)], cwd=tmp_path, check=True, capture_output=True)
     objects = glob.glob(str(tmp_path / "*gfx950"))
     assert objects
+    return [subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", o], check=True, capture_output=True, text=True).stdout for o in objects]
+
+
+def test_no_sum_goes_from_a_deep_product_to_a_shallow_one(listings):
+    """A 16-value product that adds to the result of a 32-value one takes the sum too early when the two are close, and the
+    compiler puts no wait between them (gla_chunk_common.hpp, mma_t2): no kernel may hold such a pair, however far apart."""
     products, found = 0, []
-    for obj in objects:
-        listing = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", obj], check=True, capture_output=True, text=True).stdout
+    for listing in listings:
         products += listing.count(DEEP)
         found += _mixed_depth_sums(listing.splitlines(keepends=True))
     assert products > 1000
     assert not found, f"{len(found)} in {sorted(set(found))}"
+
+
+def test_recurrent_forward_moves_its_state_in_wide_accesses(listings):
+    """The state's tiles lie across the rows of memory; lanes exchange them rather than access single values (2 to 4 bytes
+    each: a third of the time of a short forward pass of many sequences)."""
+    narrow = re.compile(r"global_(load|store)_(dword|ushort|short\w*)$")
+    kernels, found = 0, []
+    for listing in listings:
+        kernel = ""
+        for line in listing.splitlines():
+            if line.endswith(">:"):
+                kernel = line.split("<")[1].split(">")[0]
+                kernels += "recurrent_stream_fwd_kernel" in kernel
+            elif "recurrent_stream_fwd_kernel" in kernel and (op := line.split()[:1]) and narrow.match(op[0]):
+                found.append((kernel, op[0]))
+    assert kernels == 6
+    # (one gate sum per feature and sequence, in the two forms that leave nothing but states)
+    assert [op for _, op in found] == ["global_store_dword"] * 2, found
