@@ -173,7 +173,8 @@ __global__ __launch_bounds__(WAVES * 64) void cumsum_cached_kernel(const float *
 // lane 4 columns (16 bytes per access) of ROWS rows, held in registers from the only read of the source to the store.
 // An axis longer than a block's stretch takes two launches: SUMS leaves every stretch's column sums (all but the last's) in
 // `partial`, [n_outer][stretches][n_inner], and the second launch, whose source then lies in the last-level cache, adds those
-// in front of its own stretch.
+// in front of its own stretch; or, where there are many, takes their running sum, which launches in between have formed
+// (`scanned`).
 // Bound by memory.  The kernels above read row pieces of 64 and 256 bytes and run few blocks where the axis is long; here a
 // piece is 512 bytes and the axis fills the grid (fp32, sources and results not in cache, us before / after and at the rate of
 // a copy): 128 x [128,768] 27.3 / 22.7 / 20.4, 4 x [4096,768] 35.8 / 28.7 / 20.4, [32768,1024] 312 / 81 / 54,
@@ -182,7 +183,7 @@ template <int CL, int WAVES, int ROWS, bool SUMS>
 __global__ __launch_bounds__(WAVES * 64) void cumsum_rows_kernel(const float *__restrict__ src, const float *__restrict__ init,
                                                                  float *__restrict__ dst, float *__restrict__ partial,
                                                                  int64_t t_len, int64_t n_inner, int tiles, int stretches,
-                                                                 int reverse)
+                                                                 int scanned, int reverse)
 {
     constexpr int NG = WAVES * 64 / CL;            // groups of ROWS rows
     __shared__ f32x4 totals[NG][CL], before[NG][CL];
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(WAVES * 64) void cumsum_rows_kernel(const float *__
     }
     f32x4 pre = zero;
     if (!SUMS && valid)
-        for (int w = grp; w < s; w += NG)
+        for (int w = (scanned && s > 0 ? s - 1 : 0) + grp; w < s; w += NG)
             pre += *reinterpret_cast<const f32x4 *>(partial + (outer * stretches + w) * n_inner + col);
     f32x4 sum = zero;
 #pragma unroll
@@ -233,20 +234,58 @@ __global__ __launch_bounds__(WAVES * 64) void cumsum_rows_kernel(const float *__
     }
 }
 
+constexpr int64_t kRowsOneLaunch = 256;        // rows that one block holds
+// More stretches than this have their sums scanned in launches of their own: every block adding up all sums in front of it costs
+// the square of their number (us, added up / scanned: [65536,64], 256 stretches, 13.5 / 15.2; [65536,2048], 512, 314 / 300;
+// [262144,64], 2048, 86 / 39; [1048576,1024], 8192, 10 600 / 2260; [16777216,64], 131072, 309 000 / 2340, and 121 000 in one launch).
+constexpr int64_t kStretchesAddedUp = 256;
+// floats of workspace for an axis of t_len rows: stretches of 128 rows at least; their sums, and where these are scanned the
+// result and what scanning them takes
+static inline int64_t rows_workspace(int64_t n_outer, int64_t t_len, int64_t n_inner)
+{
+    if (t_len <= kRowsOneLaunch) return 0;
+    const int64_t stretches = (t_len + 127) / 128, sums = n_outer * stretches * n_inner;
+    return stretches > kStretchesAddedUp ? 2 * sums + rows_workspace(n_outer, stretches, n_inner) : sums;
+}
+
+static void cumsum_rows(hipStream_t st, const float *src, const float *init, float *dst, float *workspace, int64_t n_outer,
+                        int64_t t_len, int64_t n_inner, int reverse);
+
 template <int CL, int WAVES, int ROWS>
-static void launch_cumsum_rows(hipStream_t st, const float *src, const float *init, float *dst, float *partial, int64_t n_outer,
+static void launch_cumsum_rows(hipStream_t st, const float *src, const float *init, float *dst, float *workspace, int64_t n_outer,
                                int64_t t_len, int64_t n_inner, int reverse)
 {
     constexpr int64_t kStretch = WAVES * 64 / CL * ROWS;
     const int64_t tiles = (n_inner / 4 + CL - 1) / CL, stretches = (t_len + kStretch - 1) / kStretch;
-    if (stretches > 1)
-        hipLaunchKernelGGL((cumsum_rows_kernel<CL, WAVES, ROWS, true>), dim3((unsigned)(tiles * (stretches - 1)), (unsigned)n_outer),
-                           dim3(WAVES * 64), 0, st, src, init, dst, partial, t_len, n_inner, (int)tiles, (int)stretches, reverse);
-    hipLaunchKernelGGL((cumsum_rows_kernel<CL, WAVES, ROWS, false>), dim3((unsigned)(tiles * stretches), (unsigned)n_outer),
-                       dim3(WAVES * 64), 0, st, src, init, dst, partial, t_len, n_inner, (int)tiles, (int)stretches, reverse);
+    const bool scanned = stretches > kStretchesAddedUp;
+    const dim3 block(WAVES * 64);
+    float *before = workspace;
+    if (stretches > 1)      // (the last one's sums matter to nobody, but are read where they are scanned)
+        hipLaunchKernelGGL((cumsum_rows_kernel<CL, WAVES, ROWS, true>), dim3((unsigned)(tiles * (stretches - !scanned)), (unsigned)n_outer),
+                           block, 0, st, src, init, dst, workspace, t_len, n_inner, (int)tiles, (int)stretches, 0, reverse);
+    if (scanned) {
+        const int64_t sums = n_outer * stretches * n_inner;
+        before = workspace + sums;
+        cumsum_rows(st, workspace, nullptr, before, before + sums, n_outer, stretches, n_inner, 0);
+    }
+    hipLaunchKernelGGL((cumsum_rows_kernel<CL, WAVES, ROWS, false>), dim3((unsigned)(tiles * stretches), (unsigned)n_outer), block, 0, st,
+                       src, init, dst, before, t_len, n_inner, (int)tiles, (int)stretches, (int)scanned, reverse);
 }
 
-constexpr int64_t kRowsOneLaunch = 256;        // rows that one block holds
+static void cumsum_rows(hipStream_t st, const float *src, const float *init, float *dst, float *workspace, int64_t n_outer,
+                        int64_t t_len, int64_t n_inner, int reverse)
+{
+    // One launch where a block of 4 or 8 waves holds the axis: 64 x [256,768] 24.7 us (two launches 29.7, before 26.3).
+    // Otherwise stretches of 128 rows, or of 256 rows and half as many columns where 128 leave fewer than two blocks per
+    // compute unit ([32768,128] 13.0 against 18.4 us, but 16 x [4096,512] 82 against 74).
+    const int64_t blocks = (t_len + 127) / 128 * ((n_inner + 127) / 128) * n_outer;
+    auto launch = t_len <= 128              ? launch_cumsum_rows<32, 4, 16>
+                  : t_len <= kRowsOneLaunch ? launch_cumsum_rows<32, 8, 16>
+                  : blocks <= 512           ? launch_cumsum_rows<16, 4, 16>
+                                            : launch_cumsum_rows<32, 4, 16>;
+    launch(st, src, init, dst, workspace, n_outer, t_len, n_inner, reverse);
+}
+
 // Axes of fewer than 32 rows leave most of a block idle, rows of fewer than 64 columns most of its lanes; the upper limits
 // keep the grid's size and the byte counts in range.
 static inline bool rows_kernel_fits(int64_t t_len, int64_t n_inner)
@@ -319,7 +358,7 @@ __global__ __launch_bounds__(256) void rnn_scan_kernel(const float *__restrict__
 extern "C" size_t gla_cumsum_workspace_bytes(int64_t n_outer, int64_t t_len, int64_t n_inner)
 {
     if (n_outer <= 0 || n_outer > 65535 || t_len <= gla::kRowsOneLaunch || !gla::rows_kernel_fits(t_len, n_inner)) return 0;
-    return (size_t)(n_outer * ((t_len + 127) / 128) * n_inner) * sizeof(float);
+    return (size_t)gla::rows_workspace(n_outer, t_len, n_inner) * sizeof(float);
 }
 
 extern "C" int gla_cumsum_f32(void *stream, const float *src, const float *init, float *dst,
@@ -336,24 +375,10 @@ extern "C" int gla_cumsum_f32_ws(void *stream, const float *src, const float *in
     if (n_outer <= 0 || t_len <= 0 || n_inner <= 0 || n_outer > 65535) return GLA_ERR_SHAPE;
     if (workspace && workspace_bytes < gla_cumsum_workspace_bytes(n_outer, t_len, n_inner)) return GLA_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t)stream;
-    if (gla::rows_kernel_fits(t_len, n_inner) && gla::aligned16(src) && gla::aligned16(dst) && (!init || gla::aligned16(init))) {
-        // One launch where a block of 4 or 8 waves holds the axis: 64 x [256,768] 24.7 us (two launches 29.7, before 26.3).
-        // Otherwise stretches of 128 rows, or of 256 rows and half as many columns where 128 leave fewer than two blocks per
-        // compute unit ([32768,128] 13.0 against 18.4 us, but 16 x [4096,512] 82 against 74).
-        if (t_len <= 128) {
-            gla::launch_cumsum_rows<32, 4, 16>(st, src, init, dst, nullptr, n_outer, t_len, n_inner, reverse);
-            return gla::launch_status();
-        }
-        if (t_len <= gla::kRowsOneLaunch) {
-            gla::launch_cumsum_rows<32, 8, 16>(st, src, init, dst, nullptr, n_outer, t_len, n_inner, reverse);
-            return gla::launch_status();
-        }
-        if (workspace && gla::aligned16(workspace)) {
-            const int64_t blocks = (t_len + 127) / 128 * ((n_inner + 127) / 128) * n_outer;
-            auto launch = blocks <= 512 ? gla::launch_cumsum_rows<16, 4, 16> : gla::launch_cumsum_rows<32, 4, 16>;
-            launch(st, src, init, dst, (float *)workspace, n_outer, t_len, n_inner, reverse);
-            return gla::launch_status();
-        }
+    if (gla::rows_kernel_fits(t_len, n_inner) && gla::aligned16(src) && gla::aligned16(dst) && (!init || gla::aligned16(init)) &&
+        (t_len <= gla::kRowsOneLaunch || (workspace && gla::aligned16(workspace)))) {
+        gla::cumsum_rows(st, src, init, dst, (float *)workspace, n_outer, t_len, n_inner, reverse);
+        return gla::launch_status();
     }
     dim3 grid((unsigned)((n_inner + 63) / 64), (unsigned)n_outer);
     // long axis over few columns: cut the axis finer so that the grid fills the machine

@@ -32,6 +32,39 @@ def test_cumsum_of_long_rows(outer, T, inner, reverse, form):
     assert bool(((got - reference(x, init, reverse)).abs() <= bound).all())
 
 
+# 256 stretches (of 256 rows) are added up, more of them (of 128) scanned, 66000 in turn as stretches of stretches
+@pytest.mark.parametrize("outer,T,inner", [(1, 65536, 64), (1, 65537, 64), (2, 40000, 132), (1, 128 * 66000 + 3, 64)])
+@pytest.mark.parametrize("reverse", [False, True])
+def test_cumsum_of_long_axes(outer, T, inner, reverse):
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(outer, T, inner, generator=gen, device="cuda")
+    init = torch.randn(outer, inner, generator=gen, device="cuda")
+    got = cumsum_recursive(x, 1, init=init, reverse=reverse)
+    # a lane's rows and a block's groups three times over, and 256 stretches added up by 8 or 16 groups: at most 150 additions
+    step = 44
+    for c in range(0, inner, step):          # (a few columns at a time: the reference holds 64 bits)
+        part = x[..., c:c + step]
+        bound = 150 * 2.0 ** -24 * (part.abs().double().sum(1, keepdim=True) + init[:, None, c:c + step].abs().double())
+        assert bool(((got[..., c:c + step] - reference(part, init[:, c:c + step], reverse)).abs() <= bound).all())
+
+
+def test_cumsum_grows_with_its_axis():
+    """Four times the rows take four times as long, not sixteen (the sums of 32768 stretches added up by each of them)."""
+    def seconds(T):
+        x = torch.zeros(1, T, 64, device="cuda")
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            cumsum_recursive(x, 1)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    assert seconds(1 << 22) < 8 * seconds(1 << 20)
+
+
 def test_a_value_that_is_not_finite_stays_behind_its_row():
     x = torch.ones(1, 1000, 64, device="cuda")
     x[0, 300, 5], x[0, 640, 6] = float("inf"), float("nan")
