@@ -293,6 +293,14 @@ static inline bool rows_kernel_fits(int64_t t_len, int64_t n_inner)
     return t_len >= 32 && n_inner >= 64 && n_inner % 4 == 0 && n_inner <= (1 << 24) && t_len <= (1 << 24) &&
            t_len * n_inner <= ((int64_t)1 << 36);
 }
+// Two launches read a source twice that the last-level cache (256 MB) does not hold, and just above 256 rows a third of the blocks
+// is nearly empty: the wide rows of such an axis go to cumsum_kernel, which has blocks enough there and reads its 64 columns again from
+// L2 (us, two launches / cumsum_kernel: [257,1048576] 665 / 603, 5 x [272,65536] 205 / 191, [300,1048576] 726 / 725,
+// 13 x [300,65536] 533 / 542; narrow rows, 481 x [272,512], 142 / 153).
+static inline bool rows_kernel_reads_twice(int64_t n_outer, int64_t t_len, int64_t n_inner)
+{
+    return t_len > kRowsOneLaunch && t_len < 300 && n_inner >= 65536 && n_outer * t_len * n_inner > ((int64_t)1 << 26);
+}
 
 // One thread = one (k, W consecutive v) strip of the state, walked over T in registers; the loads
 // of step n do not depend on the recurrence, so UNROLL of them are kept in flight.  W = 4 (one
@@ -375,7 +383,7 @@ extern "C" int gla_cumsum_f32_ws(void *stream, const float *src, const float *in
     if (n_outer <= 0 || t_len <= 0 || n_inner <= 0 || n_outer > 65535) return GLA_ERR_SHAPE;
     if (workspace && workspace_bytes < gla_cumsum_workspace_bytes(n_outer, t_len, n_inner)) return GLA_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t)stream;
-    if (gla::rows_kernel_fits(t_len, n_inner) && gla::aligned16(src) && gla::aligned16(dst) && (!init || gla::aligned16(init)) &&
+    if (gla::rows_kernel_fits(t_len, n_inner) && !gla::rows_kernel_reads_twice(n_outer, t_len, n_inner) && gla::aligned16(src) && gla::aligned16(dst) && (!init || gla::aligned16(init)) &&
         (t_len <= gla::kRowsOneLaunch || (workspace && gla::aligned16(workspace)))) {
         gla::cumsum_rows(st, src, init, dst, (float *)workspace, n_outer, t_len, n_inner, reverse);
         return gla::launch_status();

@@ -33,7 +33,8 @@ def test_cumsum_of_long_rows(outer, T, inner, reverse, form):
 
 
 # 256 stretches (of 256 rows) are added up, more of them (of 128) scanned, 66000 in turn as stretches of stretches
-@pytest.mark.parametrize("outer,T,inner", [(1, 65536, 64), (1, 65537, 64), (2, 40000, 132), (1, 128 * 66000 + 3, 64)])
+@pytest.mark.parametrize("outer,T,inner", [(1, 65536, 64), (1, 65537, 64), (2, 40000, 132), (1, 128 * 66000 + 3, 64),
+                                           (1, 257, 65536 * 4)])    # (256 MB read by the kernel for any layout)
 @pytest.mark.parametrize("reverse", [False, True])
 def test_cumsum_of_long_axes(outer, T, inner, reverse):
     gen = torch.Generator(device="cuda").manual_seed(T)
@@ -41,7 +42,7 @@ def test_cumsum_of_long_axes(outer, T, inner, reverse):
     init = torch.randn(outer, inner, generator=gen, device="cuda")
     got = cumsum_recursive(x, 1, init=init, reverse=reverse)
     # a lane's rows and a block's groups three times over, and 256 stretches added up by 8 or 16 groups: at most 150 additions
-    step = 44
+    step = 44 if T > 1000 else inner
     for c in range(0, inner, step):          # (a few columns at a time: the reference holds 64 bits)
         part = x[..., c:c + step]
         bound = 150 * 2.0 ** -24 * (part.abs().double().sum(1, keepdim=True) + init[:, None, c:c + step].abs().double())
