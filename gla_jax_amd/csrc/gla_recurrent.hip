@@ -464,12 +464,16 @@ struct TimeSplit {
         // iterations at least (with four the small shapes left compute units idle: B1 T2048 H4 D128 0.31 -> 0.20 ms)
         const int64_t unit = !lean ? 1 : (heavy && ceil_div(T, most) >= 2 * kMinLeanPiece ? 128 : 64);
         auto rounded = [&](int64_t steps) { return ceil_div(steps, unit) * unit; };
-        int64_t L = rounded(ceil_div(T, most));
-        if (L < kMinSegment) L = kMinSegment;
-        // segments of one length, if that is hardly longer
+        auto pieces_of = [&](int64_t steps) { return heavy && steps % 2 == 0 && steps / 2 >= kMinLeanPiece ? 2 : 1; };
+        const int64_t share = ceil_div(T, most) < kMinSegment ? kMinSegment : ceil_div(T, most);
+        int64_t L = rounded(share);
+        // Segments of one length, if that takes hardly more iterations and as many pieces: segments that
+        // start whole iterations apart meet in the same memory channels (forward + backward, bf16, us, L = 640 / 600 at B4 T3000
+        // H12 D128 675 / 594, 1280 / 1200 at T = 6000 1276 / 1061, 512 / 450 at B4 T1800 H16 D64 196 / 170; but 512
+        // in two pieces and 500 in one 493 / 506 at B4 T2000 H16 D128).
         for (int64_t s = most; s > 1; --s)
-            if (T % s == 0 && T / s >= L) {
-                if (rounded(T / s) * 4 <= L * 5) L = T / s;
+            if (T % s == 0 && T / s >= share && rounded(T / s) * 4 <= L * 5 && pieces_of(T / s) >= pieces_of(L)) {
+                L = T / s;
                 break;
             }
         // At 128 features segments of one iteration still pay while they leave half of the compute units idle or more
@@ -490,7 +494,7 @@ struct TimeSplit {
         // kernels fit once: its passes take every segment in two pieces (512 workgroups: 100 -> 70 us at 1024 steps
         // per segment), and the scan puts the pieces together.  Pieces of 128 steps are two iterations of the kernel
         // and lose what the second workgroup gains.
-        if (heavy && L % 2 == 0 && L / 2 >= kMinLeanPiece) F = 2;
+        F = pieces_of(L);
         pieces.L = (int)(L / F);
         pieces.S = (int)ceil_div(T, pieces.L);
         nseg = B * S;

@@ -110,6 +110,20 @@ def test_chunk_plan_and_sizes():
     assert lib.gla_recurrent_fwd_workspace_bytes(B, T, H, 256, 128, _lib.GLA_BF16) == 0      # DK != DV: unsupported
 
 
+def test_segments_of_one_length_where_there_are_some():
+    """Bytes that a forward hands to its backward: a state and the gate sums of every segment (and, of 128 features, of both
+    pieces of a long one)."""
+    lib = _lib.load()
+    r256 = lambda x: (x + 255) & ~255
+    size = lambda B, S, H, D, F=1: r256(B * S * H * D * D * 4) + r256(B * S * F * H * D * 4)
+    for D in (64, 128):
+        # 48 sequences: at most 5 segments; 5 x 200 rather than 3 x 256 + 232, 5 x 280 rather than 4 x 320 + 120
+        assert lib.gla_recurrent_residual_bytes(4, 1000, 12, D, D, _lib.GLA_BF16) == size(4, 5, 12, D)
+        assert lib.gla_recurrent_residual_bytes(4, 1400, 12, D, D, _lib.GLA_BF16) == size(4, 5, 12, D)
+    # 64 sequences: 4 x 512 in two pieces each rather than 4 x 500 in one
+    assert lib.gla_recurrent_residual_bytes(4, 2000, 16, 128, 128, _lib.GLA_BF16) == size(4, 4, 16, 128, 2)
+
+
 def test_entry_points_reject_bad_arguments_without_touching_the_gpu():
     lib = _lib.load()
     buf = (ctypes.c_char * 4096)()
