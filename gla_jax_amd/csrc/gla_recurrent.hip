@@ -478,8 +478,10 @@ struct TimeSplit {
             }
         // At 128 features segments of one iteration still pay while they leave half of the compute units idle or more
         // (B1 T2048 H4 D128 0.20 -> 0.17 ms); beyond that a segment's own state, read and written once per pass,
-        // outweighs its 64 rows (B1 T8192 H2 D128 0.27 -> 0.29 ms).
-        if (heavy && L == kMinSegment && seqs * ceil_div(T, 64) <= kComputeUnits / 2) L = 64;
+        // outweighs its 64 rows (B1 T8192 H2 D128 0.27 -> 0.29 ms).  fp32 data, whose kernels go step by step, the same
+        // (8 sequences of 128 features, forward + backward, us, segments of 128 and more / of 64: T = 256 388 / 212, T = 300 452 / 216,
+        // T = 1000 404 / 245).
+        if ((lean ? heavy && L == kMinSegment : DK >= 128) && seqs * ceil_div(T, 64) <= kComputeUnits / 2) L = 64;
         const int64_t S = ceil_div(T, L);
         // From which length on the passes over shorter segments outweigh the pass they add (forward + backward, whole /
         // in segments, us).  64 features: 61 / 68 at T = 256 and 76 / 69 at 288 with 8 sequences, 63 / 75 and 78 / 79 with

@@ -124,6 +124,19 @@ def test_segments_of_one_length_where_there_are_some():
     assert lib.gla_recurrent_residual_bytes(4, 2000, 16, 128, 128, _lib.GLA_BF16) == size(4, 4, 16, 128, 2)
 
 
+def test_short_segments_of_wide_float_states():
+    """128 features and more run as segments of 64 steps while those leave half of the 256 compute units idle, fp32 data too."""
+    lib = _lib.load()
+    r256 = lambda x: (x + 255) & ~255
+    size = lambda S, H, D: r256(S * H * D * D * 4) + r256(S * H * D * 4)
+    for T in (256, 300, 520, 1000):
+        for D in (128, 256):
+            assert lib.gla_recurrent_residual_bytes(1, T, 4, D, D, _lib.GLA_F32) == size(-(-T // 64), 4, D)
+    assert lib.gla_recurrent_residual_bytes(1, 8192, 1, 128, 128, _lib.GLA_F32) == size(128, 1, 128)
+    assert lib.gla_recurrent_residual_bytes(1, 8256, 1, 128, 128, _lib.GLA_F32) < size(129, 1, 128)
+    assert lib.gla_recurrent_residual_bytes(1, 300, 4, 64, 64, _lib.GLA_F32) <= size(3, 4, 64)
+
+
 def test_entry_points_reject_bad_arguments_without_touching_the_gpu():
     lib = _lib.load()
     buf = (ctypes.c_char * 4096)()

@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     (torch.bfloat16, 2, 517, 1, 32, False),
     (torch.float32, 1, 645, 1, 64, True),
     (torch.float32, 1, 513, 1, 256, False),
+    (torch.float32, 1, 449, 2, 128, True),        # 7 x 64 + 1
 ])
 def test_uneven_segments_match_oracle(dtype, B, T, H, D, reverse):
     from gla_jax_amd import _lib, recurrent_gla
