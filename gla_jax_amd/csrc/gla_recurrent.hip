@@ -637,7 +637,11 @@ extern "C" int gla_recurrent_fwd_res(void *stream, int64_t B, int64_t T, int64_t
     if (!workspace || workspace_bytes < need) return GLA_ERR_WORKSPACE;
     if (!gla::aligned16(workspace)) return GLA_ERR_ALIGN;
     const gla::TimeSplit ts(B, T, H, DK, dtype);
-    if (!ts.on())
+    // Where the pass before the segments is a full one, a forward by itself walks a segment's steps twice, and what lies around
+    // the two passes takes the time of 40 steps: two segments are slower than the whole sequence (8 sequences, us, whole /
+    // in segments: fp32, 64 features, 64 / 73 at T = 256, 79 / 88 in 2 x 160, 95 / 73 in 3 x 128; bf16, 16 features, 54 / 63 at 256).
+    // With a backward behind it that takes the states they pay (forward + backward 302 / 238 at 256).
+    if (!ts.on() || (!residual && !gla::has_lean_pass(dtype, DK) && T < 2 * ts.sg.L + 40))
         return recurrent_fwd_inner(stream, B, whole(T), H, DK, DV, dtype, hidden_dtype, out_dtype, reverse, hidden_init,
                                    log_fgate, value, key, query, hidden_final, out, workspace);
     hipStream_t st = (hipStream_t)stream;

@@ -151,7 +151,8 @@ int gla_recurrent_bwd_ws(void *stream, int64_t B, int64_t T, int64_t H, int64_t 
 /* The same two rules with a residual: where sequences run as segments, the forward leaves the states that enter the
  * segments and the segments' gate sums in `residual` (gla_recurrent_residual_bytes, 0 where sequences run whole: then it is
  * ignored), and a backward of the same sizes that is given it does not form them again.  NULL: as the _ws entry points,
- * with the same workspaces and the same results to the bit. */
+ * with the same workspaces; the gradients are the same to the bit, hidden_final and out but for the order of fp32 sums (a
+ * forward whose states nobody takes may run a sequence whole that would be two segments). */
 size_t gla_recurrent_residual_bytes(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, gla_dtype dtype);
 int gla_recurrent_fwd_res(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
                           gla_dtype dtype, gla_dtype hidden_dtype, gla_dtype out_dtype, int reverse,

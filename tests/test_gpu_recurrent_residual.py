@@ -62,3 +62,25 @@ def test_states_kept_for_the_backward_serve_several_backward_passes():
         assert torch.equal(a, b)
     with pytest.raises(NotImplementedError, match="second-order"):
         grads[0].float().sum().backward()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,H,D,dtype,out_fp32", [(1, 256, 8, 16, torch.bfloat16, True), (2, 295, 4, 32, torch.float32, False),
+                                                    (1, 300, 2, 64, torch.float32, False)])
+def test_forward_alone_runs_two_segments_whole(B, T, H, D, dtype, out_fp32):
+    """Where the pass before the segments is a full one: the bits of the call without a workspace."""
+    lib = _lib.load()
+    _, (h0, g, v, k, q) = gpu_inputs(B, T, H, D, 3.0, seed=13, dtype=dtype)
+    code = _lib.GLA_F32 if dtype == torch.float32 else _lib.GLA_BF16
+    nf = lib.gla_recurrent_fwd_workspace_bytes(B, T, H, D, D, code)
+    assert nf > 0
+    head = (torch.cuda.current_stream().cuda_stream, B, T, H, D, D, code, code, _lib.GLA_F32 if out_fp32 else code, 0)
+    results = []
+    for ws in (None, torch.empty(nf, dtype=torch.uint8, device="cuda")):
+        hT, out = torch.empty_like(h0), torch.empty_like(v, dtype=torch.float32 if out_fp32 else dtype)
+        arrays = [t.data_ptr() for t in (h0, g, v, k, q, hT, out)]
+        _lib.check("fwd", lib.gla_recurrent_fwd(*head, *arrays) if ws is None else
+                   lib.gla_recurrent_fwd_ws(*head, *arrays, ws.data_ptr(), nf))
+        results.append((hT, out))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
