@@ -3,6 +3,7 @@
 // took 23 us for a forward and 105 to 210 us for a forward and backward, more than the kernels of a small call; here it
 // is about a third of that.  Everything else (other layouts and types, function transforms, error messages) stays in
 // gla.py, which calls this again once the arrays are converted, and whose backward rules are called where a transform is active.
+#include <ATen/TracerMode.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
@@ -112,7 +113,7 @@ ChunkOut chunk_forward(const Tensor &h0, const Tensor &g, const Tensor &v, const
     if (nws == 0) check("gla_chunk_fwd", GLA_ERR_UNSUPPORTED);
     ChunkOut r{at::empty_like(h0), at::empty_like(v), Tensor()};
     // as B rows of bytes, which is how gla.py's rules map them
-    if (residual) r.states = bytes_like((nst + d.B - 1) / d.B * d.B, v).view({d.B, -1});
+    if (residual) r.states = at::empty({d.B, (int64_t)(nst + d.B - 1) / d.B}, v.options().dtype(at::kByte));
     const Tensor ws = bytes_like(nws, v);
     check("gla_chunk_fwd",
           gla_chunk_fwd(stream_of(k), d.B, d.T, d.H, d.D, d.D, chunk, dt, code(h0), h0.data_ptr(), (const float *)g.data_ptr(),
@@ -148,7 +149,7 @@ variable_list saved_dense(AutogradContext *ctx)
 {
     variable_list s = ctx->get_saved_variables();
     for (Tensor &t : s)
-        if (t.defined()) t = t.contiguous();
+        if (t.defined() && !t.is_contiguous()) t = t.contiguous();
     return s;
 }
 bool holds(const Tensor &bytes, size_t n, const Tensor &like)
@@ -169,7 +170,8 @@ Tensor cotangent(const Tensor &d, at::IntArrayRef sizes, at::ScalarType type, co
     check_saved(d.sizes() == sizes && d.device() == like.device());
     TORCH_CHECK_NOT_IMPLEMENTED(d.has_storage() || transforms_active(), "batched cotangents (is_grads_batched, jacobian with "
                                 "vectorize=True) are not provided: map torch.autograd.grad by torch.func.vmap");
-    return d.to(type).contiguous();
+    // (each operation on a tensor that changes nothing costs a microsecond of a small step's hundred)
+    return d.scalar_type() == type && d.is_contiguous() ? d : d.to(type).contiguous();
 }
 
 template <typename... Args> variable_list python_rule(const char *name, Args &&...args)
@@ -304,9 +306,13 @@ struct Recurrent : torch::autograd::Function<Recurrent> {      // gla.py:99-170,
 // ---- module -------------------------------------------------------------------------------------
 typedef std::optional<std::vector<Tensor>> Result;       // none: not for this path
 
+// A tracer records an autograd function of Python's as a call of it; of a native call it would record the buffers that are
+// allocated here, and replay those.
+bool traced() { return at::tracer::impl::is_dispatch_enabled(); }
+
 Result chunk(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q, int64_t size)
 {
-    if (!canonical(h0, g, v, k, q) || size <= 0 || (size & (size - 1)) || dims_of(k).T % size) return std::nullopt;
+    if (traced() || !canonical(h0, g, v, k, q) || size <= 0 || (size & (size - 1)) || dims_of(k).T % size) return std::nullopt;
     if (wants_grad(h0, g, v, k, q)) return Chunk::apply(h0, g, v, k, q, size);
     ChunkOut r = chunk_forward(h0, g, v, k, q, size, false);
     return std::vector<Tensor>{r.hT, r.out};
@@ -315,7 +321,7 @@ Result chunk(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k
 Result recurrent(const Tensor &h0, const Tensor &g, const Tensor &v, const Tensor &k, const Tensor &q, bool reverse,
                  bool out_fp32)
 {
-    if (!canonical(h0, g, v, k, q) || k.size(-1) < 16) return std::nullopt;
+    if (traced() || !canonical(h0, g, v, k, q) || k.size(-1) < 16) return std::nullopt;
     if (wants_grad(h0, g, v, k, q)) return Recurrent::apply(h0, g, v, k, q, reverse, out_fp32);
     auto [hT, out] = recurrent_forward(h0, g, v, k, q, reverse, out_fp32);
     return std::vector<Tensor>{hT, out};

@@ -100,8 +100,7 @@ def _twin(cls):
 
 
 def _plain_call():
-    """No function transform and no tracer looks on: the native host side can take the call.  A tracer records a Function
-    as a call of it; of a native call it would record the buffers that it allocates, and replay those."""
+    """No function transform and no tracer looks on: the native host side can take the call."""
     return not _transforms_active() and torch._C._get_tracing_state() is None
 
 
@@ -111,8 +110,9 @@ def _apply(cls, *args):
 
 def _native(entry, arrays, *args):
     """One call of the native host side (csrc/gla_torch.cpp), which allocates, launches and keeps the autograd rule.
-    None: the arrays are not as the kernels take them (`_prep` makes them so, or says what is wrong)."""
-    if not all(isinstance(t, torch.Tensor) for t in arrays):
+    None: the arrays are not as the kernels take them (`_prep` makes them so, or says what is wrong), or a function transform or
+    a tracer looks on."""
+    if _transforms_active() or not all(isinstance(t, torch.Tensor) for t in arrays):
         return None
     return getattr(_lib.binding(), entry)(*arrays, *args)
 
@@ -257,11 +257,9 @@ def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_
     if interpret:
         raise ValueError("interpret=True asks for the reference's CPU interpreter; this build has no CPU path")
     chunk_size = int(chunk_size)
-    native = _plain_call()
-    if native:
-        done = _native("chunk", (hidden_init, log_fgate, value, key, query), chunk_size)
-        if done is not None:
-            return tuple(done)
+    done = _native("chunk", (hidden_init, log_fgate, value, key, query), chunk_size)
+    if done is not None:
+        return tuple(done)
     (h0, g, v, k, q), lead, (B, T, H, DK, DV) = _prep(hidden_init, log_fgate, value, key, query)
     if DK != DV:
         raise AssertionError("chunk_gla needs key and value head dims to be equal")   # gla.py:499
@@ -269,7 +267,7 @@ def chunk_gla(hidden_init, log_fgate, value, key, query, chunk_size, block_size_
         raise AssertionError(f"Chunk length must be power of 2, but got {chunk_size}")  # gla.py:500
     if T % chunk_size:
         raise AssertionError(f"sequence length {T} is not a multiple of chunk_size {chunk_size}")
-    hT, out = (_native("chunk", (h0, g, v, k, q), chunk_size) if native
+    hT, out = (_native("chunk", (h0, g, v, k, q), chunk_size) if _plain_call()
                else _apply(_ChunkGLA, h0, g, v, k, q, chunk_size)[:2])
     return _as(hT, lead + (H, DK, DV), hidden_init.dtype), _as(out, lead + (T, H, DV), out.dtype)
 
@@ -365,11 +363,9 @@ class _RecurrentGLABwd(torch.autograd.Function):
 
 def _recurrent(hidden_init, log_fgate, value, key, query, reverse, out_fp32):
     reverse = bool(reverse)
-    native = _plain_call()
-    if native:
-        done = _native("recurrent", (hidden_init, log_fgate, value, key, query), reverse, out_fp32)
-        if done is not None:
-            return tuple(done)
+    done = _native("recurrent", (hidden_init, log_fgate, value, key, query), reverse, out_fp32)
+    if done is not None:
+        return tuple(done)
     (h0, g, v, k, q), lead, (B, T, H, DK, DV) = _prep(hidden_init, log_fgate, value, key, query)
     if DK != DV:
         raise AssertionError("Not supported yet: key and value head dims differ")      # gla.py:120, 391
@@ -381,7 +377,7 @@ def _recurrent(hidden_init, log_fgate, value, key, query, reverse, out_fp32):
         F = torch.nn.functional
         h0 = F.pad(h0, (0, pad, 0, pad))
         g, v, k, q = (F.pad(x, (0, pad)) for x in (g, v, k, q))
-    hT, out = (_native("recurrent", (h0, g, v, k, q), reverse, out_fp32) if native
+    hT, out = (_native("recurrent", (h0, g, v, k, q), reverse, out_fp32) if _plain_call()
                else _apply(_RecurrentGLA, h0, g, v, k, q, reverse, out_fp32))
     if pad:
         hT, out = hT[..., :DK, :DV], out[..., :DV]
