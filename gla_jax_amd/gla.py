@@ -41,6 +41,8 @@ def _prep(hidden_init, log_fgate, value, key, query):
             raise TypeError(f"{name} must be a torch.Tensor")
         if not t.is_cuda:
             raise ValueError(f"{name} must live on the GPU; gla_jax_amd has no CPU path")
+        if t.device != hidden_init.device:
+            raise ValueError(f"{name} lies on another device ({t.device}) than hidden_init ({hidden_init.device})")
     if key.ndim < 3:
         raise AssertionError("key must be [..., T, H, DK]")
     lead = tuple(key.shape[:-3])

@@ -22,6 +22,8 @@ def _require_cuda(*ts):
     for t in ts:
         if t is not None and not t.is_cuda:
             raise ValueError("gla_jax_amd operators need tensors on the GPU; there is no CPU path")
+        if t is not None and t.device != ts[0].device:
+            raise ValueError(f"the tensors lie on different devices ({ts[0].device}, {t.device})")
 
 
 def cumsum_recursive(src: torch.Tensor, axis: int, init: Optional[torch.Tensor] = None,
