@@ -198,7 +198,8 @@ __device__ __forceinline__ void st8_row_once(P *row_ks, int c, const V &v, bool 
 // other token alone), and stores its results to a row that nobody reads.  Both are a scalar choice between two base
 // pointers: the kernels' instructions stay as they are (with the stores under a branch the gradient kernel lost 1 to 2 %
 // at full tiles, the branch being a wall to the scheduler).
-static __device__ float zero_row[128], spare_row[128];
+// (as aligned as the rows that they stand for: the kernels access them 16 bytes at a time)
+static __device__ __align__(16) float zero_row[128], spare_row[128];
 template <typename P> __device__ __forceinline__ const P *rows_or_zeros(bool live, const P *rows)
 {
     return live ? rows : reinterpret_cast<const P *>(zero_row);
