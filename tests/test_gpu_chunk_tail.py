@@ -56,3 +56,54 @@ def test_float_data_at_128_features_on_64_token_tiles(T, shift):
     hT, out = chunk_gla(*dev, 32)
     grads = torch.autograd.grad((hT, out), dev, (to_dev(dhT, dtype), to_dev(dout, dtype)))
     check_chunk_outputs(dtype, arrs, 32, hT, out, grads, dhT, dout)
+
+
+def _clean_and_filled(dtype, B, T, H, D, full, poison=None):
+    """Outputs and gradients of a call of T tokens, and of the same call with zeros up to `full` tokens."""
+    from gla_jax_amd import chunk_gla
+    arrs, dev = gpu_inputs(B, T, H, D, 3.0, seed=T + D, dtype=dtype)
+    dhT, dout = (to_dev(t, dtype) for t in cotangents(arrs[0], arrs[2], 5, dtype))
+    results = []
+    for n in (T, full):
+        args = [dev[0].clone()] + [torch.nn.functional.pad(t, (0, 0, 0, 0, 0, n - T)) for t in dev[1:]]
+        if poison is not None:
+            poison(args)
+        args = [t.requires_grad_(True) for t in args]
+        outs = chunk_gla(*args, 32)
+        grads = torch.autograd.grad(outs, args, (dhT, torch.nn.functional.pad(dout, (0, 0, 0, 0, 0, n - T))))
+        results.append([outs[0], grads[0]] + [t[:, :T] for t in (outs[1],) + grads[1:]])
+    return results
+
+
+# (128-token tiles; at 256 features as two passes of 128 with float results)
+@pytest.mark.parametrize("dtype,B,T,H,D,full", [
+    (torch.bfloat16, 2, 1056, 8, 256, 1152),
+    (torch.bfloat16, 2, 1120, 8, 256, 1152),
+    (torch.bfloat16, 2, 1056, 8, 128, 1152),
+    (torch.float32, 2, 2080, 2, 128, 2112),
+])
+def test_tail_is_what_a_caller_would_fill_up(dtype, B, T, H, D, full):
+    for got, want in zip(*_clean_and_filled(dtype, B, T, H, D, full)):
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_a_value_that_is_not_finite_in_the_last_tile_stays_with_its_sequence(D, value):
+    """One key feature of one token in the filled-up tile: every other (batch, head) pair and the outputs of the tiles before
+    keep their bits."""
+    def poison(args):
+        args[3][0, 1050, 1, 7] = value
+
+    clean = _clean_and_filled(torch.bfloat16, 2, 1056, 16, D, 1152)[0]
+    got = _clean_and_filled(torch.bfloat16, 2, 1056, 16, D, 1152, poison)[0]
+    others = torch.ones(2, 16, dtype=torch.bool)
+    others[0, 1] = False
+    for i, (a, b) in enumerate(zip(got, clean)):
+        a, b = (a, b) if i < 2 else (a.transpose(1, 2), b.transpose(1, 2))
+        assert torch.equal(a[others], b[others])
+        if i in (1, 5):          # the gradients of the initial state and of the keys have no key in them
+            assert torch.equal(a, b)
+        else:
+            assert not bool(a[0, 1].isfinite().all())
+    assert torch.equal(got[2][0, :1024, 1], clean[2][0, :1024, 1])
