@@ -223,15 +223,17 @@ def bench_recurrent(B, T, H, D, shift, steps, warmup):
     n_b = lib.gla_recurrent_bwd_workspace_bytes(B, T, H, D, D, dt)
     ws_f = torch.empty(max(n_f, 16), dtype=torch.uint8, device="cuda")
     ws_b = torch.empty(max(n_b, 16), dtype=torch.uint8, device="cuda")
+    # the forward hands the segments' states to the backward, as the public function's does
+    res = torch.empty(max(lib.gla_recurrent_residual_bytes(B, T, H, D, D, dt), 16), dtype=torch.uint8, device="cuda")
 
     def fwd():
-        _lib.check("gla_recurrent_fwd_ws", lib.gla_recurrent_fwd_ws(st, B, T, H, D, D, dt, dt, dt, 0, p(h0), p(g), p(v),
-                                                                    p(k), p(q), p(hT), p(out), p(ws_f), n_f))
+        _lib.check("gla_recurrent_fwd_res", lib.gla_recurrent_fwd_res(st, B, T, H, D, D, dt, dt, dt, 0, p(h0), p(g), p(v),
+                                                                      p(k), p(q), p(hT), p(out), p(res), p(ws_f), n_f))
 
     def bwd():
-        _lib.check("gla_recurrent_bwd_ws", lib.gla_recurrent_bwd_ws(st, B, T, H, D, D, dt, dt, dt, 0, p(h0), p(g), p(v),
-                                                                    p(k), p(q), p(hT), p(dhT), p(dout), p(dh0), p(dg),
-                                                                    p(dv), p(dk), p(dq), p(ws_b), n_b))
+        _lib.check("gla_recurrent_bwd_res", lib.gla_recurrent_bwd_res(st, B, T, H, D, D, dt, dt, dt, 0, p(h0), p(g), p(v),
+                                                                      p(k), p(q), p(hT), p(dhT), p(dout), p(dh0), p(dg),
+                                                                      p(dv), p(dk), p(dq), p(res), p(ws_b), n_b))
 
     def step():
         fwd()
