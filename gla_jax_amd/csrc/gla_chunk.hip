@@ -31,7 +31,8 @@ struct ChunkPlan {
     {
         return prod + decay + bwd_states * states + (split ? 2 * rows + (wide ? 7 : 4) * rows_f32 + 4 * hid : 0);
     }
-    // fp32 data at 128 features ran on 32-token tiles only: callers may count on a forward workspace of that size
+    // fp32 data at 128 features ran on 32-token tiles only, and the size of their forward workspace has stayed the one that is
+    // asked for: twice what the 64-token tiles use (404 MB of which 202 at B4 T4096 H6)
     size_t fwd_least = 0;
     size_t resid_bytes() const { return split ? 2 * resid : resid; }
 };
@@ -41,24 +42,41 @@ static size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 // The tile: tokens per workgroup, 128, 64 or 32 (fp32 data: 64 or 32).  The result does not
 // depend on it (only its rounding does), so whatever chunk_size asks for, the lengths and the number of sequences decide; a
 // tile need not divide T, the last one is filled up with zeros.  Wide tiles mean fewer chunk states to write, scan
-// and read; narrow ones more workgroups with less to do each while there are not enough for the 256 compute units.
-// Forward + backward, bf16, us per tile 128 / 64 / 32 (wg: workgroups of 64-token tiles):
+// and read; narrow ones more workgroups with less to do each while there are not enough for the 256 compute units, and fewer
+// zeros.  Forward + backward, bf16, us per tile 128 / 64 / 32 (wg: workgroups of 64-token tiles):
 //   128 features  B4 T4096 H6 213 / 298 / 680    B4 T1056 H6 (408 wg) 81 / 101 / 130    B16 T160 H8 (384 wg) 87 / 99 / 121
 //                 B4 T512 H6 (192 wg) 76 / 62 / 73    B16 T96 H8 (256 wg) 80 / 69 / 75    B1 T160 H1 69 / 52 / 50
+//                 one tile per sequence, 1024 of them: T32 289 / 246 / 212    T64 313 / 270 / 341    T96 325 / 447 / 500
+//                 96 sequences: T288 127 / 102 / 135 (288 workgroups go round twice, 480 fit side by side), T352 132 / 141 / 172
 //   64 features   B16 T2048 H8 242 / 269 / 385   B16 T1056 H8 (1152 against 1088 rows) 154 / 143 / 183
 //                 B4 T2048 H6 69 / 67 / 91   B1 T16384 H2 75 / 107 (a scan of 256 chunks)   B1 T2048 H1 43 / 37 / 43
+//                 192 sequences: T160 66 / 52 / 47    T352 (576 workgroups of 128: two rounds and a quarter) 96 / 83 / 86
+//   32 features   1024 sequences: T96 78 / 73 / 67    T160 137 / 101 / 98    T544 322 / 278 / 307    128: T4128 293 / 264 / 281
 // and fp32, 64 / 32: 64 features B4 T1056 H6 84 / 93, B1 T512 H2 45 / 39, B1 T2048 H2 51 / 52; 128 features B4 T4096 H6
-// 671 / 1030, B4 T512 H6 110 / 140, B4 T288 H6 103 / 91, B1 T512 H2 94 / 75.
+// 671 / 1030, B4 T512 H6 110 / 140, B4 T288 H6 103 / 91, B1 T512 H2 94 / 75, T32 510 / 456 with 1024 sequences, T160
+// 180 / 154 with 96; 32 features, 384 sequences, T96 50 / 44, T160 70 / 62, T224 84 / 78.
 static int64_t choose_tile(int64_t seqs, int64_t T, int64_t D, int dtype)
 {
-    auto tiles = [&](int64_t c) { return (T + c - 1) / c; };
     constexpr int64_t kUnits = 256;                          // compute units
-    if (dtype == GLA_F32) return T < 2048 && seqs * tiles(32) <= kUnits ? 32 : 64;
-    if (T <= (D > 64 ? 256 : 576) && seqs * tiles(32) <= kUnits) return 32;
-    if (seqs * tiles(64) <= kUnits && tiles(64) <= (D >= 64 ? 64 : 32)) return 64;
-    // 64 features: where a 128-token tile would carry over 5 % more zeros
-    if (D == 64 && T <= 4096 && tiles(128) * 128 * 20 > tiles(64) * 64 * 21) return 64;
-    return 128;
+    auto tiles = [&](int64_t c) { return (T + c - 1) / c; };
+    auto wg = [&](int64_t c) { return seqs * tiles(c); };
+    if (T <= 32) return 32;
+    if (dtype == GLA_F32) {
+        if (T < 2048 && wg(32) <= kUnits) return 32;
+        if (T % 64 == 0 || wg(64) <= kUnits) return 64;
+        // half of the last 64-token tile would be zeros
+        if (D > 64) return wg(32) <= 2 * kUnits ? 32 : 64;
+        return T <= (D > 32 ? 160 : 416) && wg(32) <= (D > 32 ? 8 : 16) * kUnits ? 32 : 64;
+    }
+    if (T <= (D > 64 ? 256 : 576) && wg(32) <= kUnits) return 32;
+    if (T <= 64) return 64;
+    if (wg(64) <= kUnits) return tiles(64) <= (D >= 64 ? 64 : 32) ? 64 : 128;
+    if (T % 128 == 0 || T > 4224) return 128;
+    if (D > 64) return wg(64) <= 2 * kUnits && wg(128) > kUnits ? 64 : 128;
+    if (T <= 160 && T % 64 != 0 && wg(32) <= (D > 32 ? 4 : 32) * kUnits) return 32;
+    // 64 features: where a 128-token tile would carry over 5 % more zeros, or leaves a tenth of its last round idle
+    const int64_t rounds = (wg(128) + kUnits - 1) / kUnits;
+    return D <= 32 || tiles(128) * 128 * 20 > tiles(64) * 64 * 21 || (rounds <= 4 && wg(128) * 10 <= rounds * kUnits * 9) ? 64 : 128;
 }
 
 // chunk_size is checked as the reference checks it.  Sizes below 32 tokens are refused: the leaf of the reference needs
@@ -105,7 +123,8 @@ static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, i
     if (dtype == GLA_F32 && Dk == 128)
         plan->fwd_least = round256((size_t)B * H * (size_t)(T / 32) * (2 * DK * DV + DK) * sizeof(float));
     plan->bwd_states = dtype == GLA_BF16 ? 1 : 2;
-    // the residual is handed out with room for the states of the largest tile that divides T, which callers may count on
+    // The residual has room for the states of the largest tile that divides T, as when the tile had to: the size that is asked
+    // for stays what it was, though a filled-up last tile needs less (B3 T1120 H6 D128: 21.2 MB, 5.9 written).
     int64_t Cd = dtype == GLA_BF16 ? 128 : (DK > 64 ? 32 : 64);
     while (T % Cd != 0) Cd /= 2;
     const size_t slots = 1 + (N > (size_t)(T / Cd) ? N : (size_t)(T / Cd));

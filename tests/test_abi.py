@@ -110,6 +110,24 @@ def test_chunk_plan_and_sizes():
     assert lib.gla_recurrent_fwd_workspace_bytes(B, T, H, 256, 128, _lib.GLA_BF16) == 0      # DK != DV: unsupported
 
 
+def test_tiles_of_lengths_that_128_tokens_do_not_divide():
+    """The workspace goes by the number of tiles: that of a length which the tile divides as often."""
+    lib = _lib.load()
+    size = lambda seqs, T, D, dt: lib.gla_chunk_bwd_workspace_bytes(seqs // 16, T, 16, D, D, 32, dt)
+    bf, f32 = _lib.GLA_BF16, _lib.GLA_F32
+    for D in (16, 32):
+        assert size(1024, 96, D, bf) == size(1024, 3 * 128, D, bf)            # three of 32 tokens
+        assert size(1024, 160, D, bf) == size(1024, 5 * 128, D, bf)
+        assert size(1024, 544, D, bf) == size(1024, 9 * 128, D, bf)           # nine of 64
+        assert size(384, 224, D, f32) == size(384, 7 * 64, D, f32)            # seven of 32
+    assert size(192, 160, 64, bf) == size(192, 5 * 128, 64, bf)
+    assert size(192, 352, 64, bf) == size(192, 6 * 128, 64, bf)               # six of 64: 576 of 128 go round three times
+    assert size(256, 480, 64, bf) == size(256, 4 * 128, 64, bf)
+    assert size(96, 288, 128, bf) == size(96, 5 * 128, 128, bf)               # five of 64: 288 of 128 go round twice
+    assert size(96, 352, 128, bf) == size(96, 3 * 128, 128, bf)
+    assert size(96, 160, 128, f32) == size(96, 5 * 64, 128, f32)
+
+
 def test_segments_of_one_length_where_there_are_some():
     """Bytes that a forward hands to its backward: a state and the gate sums of every segment (and, of 128 features, of both
     pieces of a long one)."""
