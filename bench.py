@@ -4,7 +4,7 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload chunk|recurrent|long] [--no-cpu]
 
 A step is one pass of the hot path over one batch of synthetic input resident in HBM: chunk_gla
-forward + backward (all five gradients) through the C ABI of libgla_hip.so at BASELINE.json's
+forward + backward (all five gradients) through the C ABI of libgla_hip.so at the reference's
 headline shape (B4, T4096, H6, D128, chunk 128, bf16 q/k/v/hidden, fp32 gates).  Prints ONE JSON line.
 
 `roofline` describes the dominant kernel (the per-chunk gradient kernel): algorithmic HBM bytes per
@@ -42,7 +42,7 @@ KERNEL_SOURCES = {
 }
 MEASURED_TRAFFIC = {
     # (kernel, B, T, H, D, chunk, source hash): bytes per launch
-    ("chunk_grad_kernel", 4, 4096, 6, 128, 128, "7777fc4c77fd"): 394.7e6,
+    ("chunk_grad_kernel", 4, 4096, 6, 128, 128, "eef6e68a7086"): 394.4e6,
 }
 
 
@@ -60,9 +60,9 @@ def measured_traffic(kernel, B, T, H, D, chunk):
 
 WORKLOADS = {
     # name: (kind, B, T, H, D, chunk, gate shift)
-    "chunk": ("chunk", 4, 4096, 6, 128, 128, 5.0),       # BASELINE configs[1]/[2] (headline metric)
-    "long": ("chunk", 1, 32768, 8, 128, 128, 0.0),
-    "recurrent": ("recurrent", 16, 2048, 16, 64, 0, 3.0),
+    "chunk": ("chunk", 4, 4096, 6, 128, 128, 5.0),       # the headline metric
+    "long": ("chunk", 1, 32768, 8, 128, 128, 0.0),       # one long sequence, strong decay
+    "recurrent": ("recurrent", 16, 2048, 16, 64, 0, 3.0),  # one sequence per compute unit
     # the shape of the reference's own script (gla.py:1405-1410): 64 sequences, which run as 4 segments each
     "recurrent_few": ("recurrent", 4, 4096, 16, 128, 0, 3.0),
     # the two scan operators of ops.py on their own, at the sizes chunk_gla gives them at the headline shape

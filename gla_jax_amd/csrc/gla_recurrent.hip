@@ -437,8 +437,8 @@ extern "C" int gla_recurrent_fwd(void *stream, int64_t B, int64_t T, int64_t H, 
 }
 
 // ---- a sequence as S segments side by side (gla_timesplit.hip) -------------------------------------------------
-// With few (batch, head) pairs (at most half of the GPU's compute units), a call with a workspace runs every sequence as S segments at once: one pass from zero states for
-// the segments' own contributions, a scan over the segments, and the real pass with the states that enter each segment
+// With few (batch, head) pairs (at most half of the GPU's compute units), a call with a workspace runs every sequence as S
+// segments at once: one pass from zero states for the segments' own contributions, a scan over the segments, and the real pass with the states that enter each segment
 // (fp32); the backward does the same for the states' cotangents.
 namespace gla {
 constexpr int64_t kComputeUnits = 256;       // MI355X
@@ -484,10 +484,11 @@ struct TimeSplit {
         if ((lean ? heavy && L == kMinSegment : DK >= 128) && seqs * ceil_div(T, 64) <= kComputeUnits / 2) L = 64;
         const int64_t S = ceil_div(T, L);
         // From which length on the passes over shorter segments outweigh the pass they add (forward + backward, whole /
-        // in segments, us).  64 features: 61 / 68 at T = 256 and 76 / 69 at 288 with 8 sequences, 63 / 75 and 78 / 79 with
-        // 64; two segments per sequence 190 / 192 at 896 and 215 / 203 at 1024.  128 features: 206 / 200 at 193 (161 / 200
-        // at 129), and less where segments of 64 steps fit (156 / 120 at 129); two segments 251 / 283 at 288 and 297 / 286
-        // at 384.  Full first pass (fp32, 64 features, 8 sequences): 350 / 360 at 300, 593 / 278 at 512.
+        // in segments, us).  64 features: 61 / 59 at T = 256 and 75 / 59 at 288 with 8 sequences, 63 / 64 and 78 / 67 with
+        // 64; two segments per sequence 190 / 192 at 896 and 215 / 203 at 1024.  128 features: 189 / 103 at 201 with 8 sequences,
+        // 196 / 168 with 64; two segments 251 / 283 at 288 and 297 / 286 at 384.  Up to 200 steps they stay whole for another
+        // reason: segments of 64 would pay there as well (156 / 120 at 129), but few sequences of that length have never asked
+        // for a workspace.  Full first pass (fp32, 64 features, 8 sequences): 302 / 238 at 256, 595 / 241 at 512.
         const int64_t from = heavy ? (most == 2 ? 384 : 201) : lean ? (most == 2 ? 1024 : (most == 3 ? 384 : 256)) : 256;
         if (T < from || S < 2 || S * 2 > 65535) return;
         sg.S = (int)S;

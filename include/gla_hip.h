@@ -121,7 +121,7 @@ int gla_recurrent_bwd(void *stream, int64_t B, int64_t T, int64_t H, int64_t DK,
  * workspace (the two entry points above) head dimension 256 runs on per-timestep vector kernels, an order of
  * magnitude slower.
  * (2) With few sequences (B*H, at head dimension 256 2*B*H, at most half of the GPU's 256 compute units) that are long
- * enough (from 129 to 1024 steps on, by head dimension and number of sequences), every sequence runs as S segments side
+ * enough (from 201 to 1024 steps on, by head dimension and number of sequences), every sequence runs as S segments side
  * by side, the last one shorter where S does not divide T:
  * the recurrence is linear in the state, so one pass from zero states gives each segment's own contribution, a scan
  * over the segments the state that enters each (fp32, in the workspace), and a second pass the outputs; the
