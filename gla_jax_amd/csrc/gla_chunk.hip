@@ -55,6 +55,10 @@ static size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 // and fp32, 64 / 32: 64 features B4 T1056 H6 84 / 93, B1 T512 H2 45 / 39, B1 T2048 H2 51 / 52; 128 features B4 T4096 H6
 // 671 / 1030, B4 T512 H6 110 / 140, B4 T288 H6 103 / 91, B1 T512 H2 94 / 75, T32 510 / 456 with 1024 sequences, T160
 // 180 / 154 with 96; 32 features, 384 sequences, T96 50 / 44, T160 70 / 62, T224 84 / 78.
+static inline bool wide_tiles_carry_zeros(int64_t T)         // a 128-token tile over 5 % more of them than one of 64
+{
+    return (T + 127) / 128 * 128 * 20 > (T + 63) / 64 * 64 * 21;
+}
 static int64_t choose_tile(int64_t seqs, int64_t T, int64_t D, int dtype)
 {
     constexpr int64_t kUnits = 256;                          // compute units
@@ -74,15 +78,16 @@ static int64_t choose_tile(int64_t seqs, int64_t T, int64_t D, int dtype)
     if (T % 128 == 0 || T > 4224) return 128;
     if (D > 64) return wg(64) <= 2 * kUnits && wg(128) > kUnits ? 64 : 128;
     if (T <= 160 && T % 64 != 0 && wg(32) <= (D > 32 ? 4 : 32) * kUnits) return 32;
-    // 64 features: where a 128-token tile would carry over 5 % more zeros, or leaves a tenth of its last round idle
+    // 64 features: also where 128-token tiles leave a tenth of their rounds idle
     const int64_t rounds = (wg(128) + kUnits - 1) / kUnits;
-    return D <= 32 || tiles(128) * 128 * 20 > tiles(64) * 64 * 21 || (rounds <= 4 && wg(128) * 10 <= rounds * kUnits * 9) ? 64 : 128;
+    return D <= 32 || wide_tiles_carry_zeros(T) || (rounds <= 4 && wg(128) * 10 <= rounds * kUnits * 9) ? 64 : 128;
 }
 
 // chunk_size is checked as the reference checks it.  Sizes below 32 tokens are refused: the leaf of the reference needs
 // 32 rows as well (gla.py:975-977).
+// `beside`: bytes that the caller adds to the forward's workspace.
 static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, int64_t chunk, int dtype,
-                      ChunkPlan *plan, int hidden_dtype = GLA_BF16)
+                      ChunkPlan *plan, int hidden_dtype = GLA_BF16, size_t beside = 0)
 {
     if (hidden_dtype != GLA_F32 && hidden_dtype != GLA_BF16) return GLA_ERR_DTYPE;
     if (B <= 0 || T <= 0 || H <= 0 || DK <= 0 || DV <= 0) return GLA_ERR_SHAPE;
@@ -92,16 +97,27 @@ static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, i
     if (!is_pow2(chunk) || T % chunk != 0) return GLA_ERR_CHUNK;   // gla.py:500, 674
     if (chunk < 32) return GLA_ERR_UNSUPPORTED;
     if (DK == 256) {
-        int rc = plan_chunk(B, T, 2 * H, 128, 128, chunk, dtype, plan, hidden_dtype);
-        if (rc) return rc;
         plan->split = true;
         plan->wide = dtype == GLA_BF16;
         plan->rows = round256((size_t)B * T * H * 256 * (dtype == GLA_BF16 ? 2 : 4));
         plan->rows_f32 = round256((size_t)B * T * H * 256 * sizeof(float));
         plan->hid = round256((size_t)B * 2 * H * 128 * 128 * sizeof(float));
-        return GLA_OK;
+        return plan_chunk(B, T, 2 * H, 128, 128, chunk, dtype, plan, hidden_dtype, plan->fwd_bytes());
     }
-    const int64_t C = choose_tile(B * H, T, DK, dtype);
+    int64_t C = choose_tile(B * H, T, DK, dtype);
+    // More tiles mean a larger workspace, and gla_chunk_fwd_static takes what fits its array: a tile that was chosen for speed
+    // is no reason to refuse a call there (the tile is one of the shape, whoever calls).
+    const int64_t esize = dtype == GLA_BF16 ? 2 : 4, Ds = DK < 32 ? 32 : DK;
+    const int64_t widest = dtype == GLA_F32 || (DK == 64 && wide_tiles_carry_zeros(T)) ? 64 : 128;
+    auto fits = [&](int64_t c) {
+        const size_t chunks = (size_t)B * H * ((T + c - 1) / c), state = (size_t)Ds * Ds;
+        return beside + chunks * (state * 2 * esize + state / 16 + Ds * sizeof(float)) + 1024 <= GLA_CHUNK_FWD_STATIC_BYTES;
+    };
+    for (int64_t c = C; c <= widest; c *= 2)
+        if (fits(c)) {
+            C = c;
+            break;
+        }
     int Dk = 0;
 #define GLA_PLAN_CASE(T_, C_, D_, DM_) \
     if (((dtype == GLA_BF16) == (sizeof(T_) == 2)) && C == C_ && DK == DM_) Dk = D_;

@@ -128,6 +128,24 @@ def test_tiles_of_lengths_that_128_tokens_do_not_divide():
     assert size(96, 160, 128, f32) == size(96, 5 * 64, 128, f32)
 
 
+def test_narrow_tiles_do_not_outgrow_the_static_workspace():
+    """gla_chunk_fwd_static takes what fits 80 MiB: a tile is widened where only its number of chunk states stands in the way."""
+    lib = _lib.load()
+    bf, f32, room = _lib.GLA_BF16, _lib.GLA_F32, 80 << 20
+    fwd = lambda seqs, T, D, dt: lib.gla_chunk_fwd_workspace_bytes(seqs // 16, T, 16, D, D, 32, dt)
+    bwd = lambda seqs, T, D, dt: lib.gla_chunk_bwd_workspace_bytes(seqs // 16, T, 16, D, D, 32, dt)
+    # 4096 sequences of 160 tokens, 32 features: five tiles of 32 would take 88 MB, three of 64 fit; of 8192 two of 128 do
+    assert fwd(4096, 160, 32, bf) <= room and bwd(4096, 160, 32, bf) == bwd(4096, 3 * 128, 32, bf)
+    assert fwd(8192, 160, 32, bf) <= room and bwd(8192, 160, 32, bf) == bwd(8192, 2 * 128, 32, bf)
+    # as two passes of 128 features, with what lies beside them: 96 heads of 288 tokens on three tiles of 128
+    assert fwd(48, 288, 256, bf) <= room and bwd(32, 288, 256, bf) < bwd(48, 288, 256, bf)
+    # where none fits the choice stands: 64-token tiles, 64 features, nine of them
+    assert fwd(4096, 544, 64, bf) > room and bwd(4096, 544, 64, bf) == bwd(4096, 9 * 128, 64, bf)
+    # and a length whose wide tiles carry more zeros keeps its 64-token tiles
+    assert bwd(1536, 192, 64, bf) == bwd(1536, 3 * 128, 64, bf)
+    assert fwd(2048, 96, 32, f32) <= room
+
+
 def test_segments_of_one_length_where_there_are_some():
     """Bytes that a forward hands to its backward: a state and the gate sums of every segment (and, of 128 features, of both
     pieces of a long one)."""
