@@ -31,9 +31,10 @@ def cumsum_recursive(src: torch.Tensor, axis: int, init: Optional[torch.Tensor] 
     """Inclusive cumulative sum of `src` along `axis` plus `init` (shape = src.shape without `axis`),
     from the far end when `reverse` (ops.py:234-284).  Computed in float32, returned in src.dtype."""
     axis = axis % src.ndim
-    done = _lib.binding().cumsum(src, axis, init, bool(reverse))      # float32, dense, on the GPU: the usual case
-    if done is not None:
-        return done
+    if src.dtype == torch.float32:                  # and dense, on the GPU: the usual case
+        done = _lib.binding().cumsum(src, axis, init, bool(reverse))
+        if done is not None:
+            return done
     _require_cuda(src, init)
     pre, T, post = src.shape[:axis], src.shape[axis], src.shape[axis + 1:]
     if init is not None and tuple(init.shape) != tuple(pre + post):
@@ -46,6 +47,9 @@ def cumsum_recursive(src: torch.Tensor, axis: int, init: Optional[torch.Tensor] 
         n_inner *= s
     x = src.contiguous().to(torch.float32)
     i = None if init is None else init.contiguous().to(torch.float32)
+    done = _lib.binding().cumsum(x, axis, i, bool(reverse))
+    if done is not None:
+        return done.to(src.dtype)
     dst = torch.empty_like(x)
     lib = _lib.load()
     # grid.y carries the outer index: split very large outer counts

@@ -66,6 +66,20 @@ def test_cumsum_grows_with_its_axis():
     assert seconds(1 << 22) < 8 * seconds(1 << 20)
 
 
+@pytest.mark.parametrize("shape,axis", [((2, 1000, 128), 1), ((3, 40, 64), 1), ((70000, 33), 0), ((70000, 3, 2), 1)])
+def test_converted_arrays_take_the_same_way(shape, axis):
+    """16-bit and strided arrays are converted first: the bits of a call with the converted ones."""
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn(*shape, generator=gen, device="cuda")
+    init = torch.randn(*shape[:axis], *shape[axis + 1:], generator=gen, device="cuda").bfloat16()
+    spread = torch.stack((x, x), -1)[..., 0]
+    for reverse in (False, True):
+        assert torch.equal(cumsum_recursive(spread, axis, reverse=reverse), cumsum_recursive(x, axis, reverse=reverse))
+        low = x.bfloat16()
+        want = cumsum_recursive(low.float(), axis, init=init.float(), reverse=reverse)
+        assert torch.equal(cumsum_recursive(low, axis, init=init, reverse=reverse), want.bfloat16())
+
+
 def test_a_value_that_is_not_finite_stays_behind_its_row():
     x = torch.ones(1, 1000, 64, device="cuda")
     x[0, 300, 5], x[0, 640, 6] = float("inf"), float("nan")
