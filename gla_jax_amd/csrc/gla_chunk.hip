@@ -22,6 +22,7 @@ struct ChunkPlan {
     size_t rows = 0;                          // one [B,T,H,256] array of the element type
     size_t rows_f32 = 0;                      // ... of floats
     size_t hid = 0;                           // one [B,2H,128,128] array of states (sized for fp32 states)
+    size_t beside = 0;                        // what lies beside a pass's own workspace: a pass is planned with it again
     bool wide = false;                        // bf16 data: both passes leave their results in fp32, summed and rounded once
     // forward: value rows with their halves exchanged, the second pass's out (fp32 data) or both passes' (bf16 data),
     // hidden_init and hidden_final in blocks; backward: value and dout rows exchanged, the second pass's dq, dk, dv
@@ -102,7 +103,8 @@ static int plan_chunk(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV, i
         plan->rows = round256((size_t)B * T * H * 256 * (dtype == GLA_BF16 ? 2 : 4));
         plan->rows_f32 = round256((size_t)B * T * H * 256 * sizeof(float));
         plan->hid = round256((size_t)B * 2 * H * 128 * 128 * sizeof(float));
-        return plan_chunk(B, T, 2 * H, 128, 128, chunk, dtype, plan, hidden_dtype, plan->fwd_bytes());
+        plan->beside = plan->fwd_bytes();
+        return plan_chunk(B, T, 2 * H, 128, 128, chunk, dtype, plan, hidden_dtype, plan->beside);
     }
     int64_t C = choose_tile(B * H, T, DK, dtype);
     // More tiles mean a larger workspace, and gla_chunk_fwd_static takes what fits its array: a tile that was chosen for speed
@@ -215,15 +217,16 @@ extern "C" size_t gla_chunk_bwd_workspace_bytes(int64_t B, int64_t T, int64_t H,
     return plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p) == GLA_OK ? p.bwd_bytes() : 0;
 }
 
-// wide != 0 (bf16 data at head dimension 128 only): `out` is a float array
+// wide != 0 (bf16 data at head dimension 128 only): `out` is a float array.  `beside` is not 0 in a pass of head dimension
+// 256: its tile has to be the one that the whole call was planned (and its workspace cut up) with.
 static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
                          int64_t chunk_size, gla_dtype dtype, gla_dtype hidden_dtype, const void *hidden_init,
                          const float *log_fgate, const void *value, const void *key, const void *query,
                          void *hidden_final, void *out, void *states, void *workspace, size_t workspace_bytes,
-                         int wide)
+                         int wide, size_t beside = 0)
 {
     ChunkPlan p;
-    int rc = plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p, hidden_dtype);
+    int rc = plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p, hidden_dtype, beside);
     if (rc) return rc;
     const void *req[] = {hidden_init, log_fgate, value, key, query, hidden_final, out};
     for (const void *ptr : req) {
@@ -249,11 +252,11 @@ static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         e = launch_swap_halves(st, dtype, B * T * H, v_sw, value);
         if (e) return e;
         e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_same, log_fgate, value,
-                          key, query, hT_same, p.wide ? (void *)out1 : out, states, ws, sub, p.wide);
+                          key, query, hT_same, p.wide ? (void *)out1 : out, states, ws, sub, p.wide, p.beside);
         if (e) return e;
         e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_cross, log_fgate, v_sw,
                           key, query, hT_cross, out2, states ? (unsigned char *)states + p.resid : nullptr, ws, sub,
-                          p.wide);
+                          p.wide, p.beside);
         if (e) return e;
         e = p.wide ? launch_sum_rows(st, dtype, B * T * H, out, (const float *)out1, (const float *)out2, 1)
                    : launch_add_rows(st, dtype, B * T * H, out, out2, 1);
@@ -341,15 +344,16 @@ extern "C" int gla_chunk_fwd_static(void *stream, int64_t B, int64_t T, int64_t 
                                 value, key, query, hidden_final, out, states, ws, kStaticScratchBytes);
 }
 
-// wide != 0 (bf16 data at head dimension 128 only): `dvalue`, `dkey`, `dquery` are float arrays
+// wide != 0 (bf16 data at head dimension 128 only): `dvalue`, `dkey`, `dquery` are float arrays; `beside` as in the forward
 static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
                          int64_t chunk_size, gla_dtype dtype, gla_dtype hidden_dtype, const float *log_fgate,
                          const void *value, const void *key, const void *query, const void *states,
                          const void *dhidden_final, const void *dout, void *dhidden_init, float *dlog_fgate,
-                         void *dvalue, void *dkey, void *dquery, void *workspace, size_t workspace_bytes, int wide)
+                         void *dvalue, void *dkey, void *dquery, void *workspace, size_t workspace_bytes, int wide,
+                         size_t beside = 0)
 {
     ChunkPlan p;
-    int rc = plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p, hidden_dtype);
+    int rc = plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p, hidden_dtype, beside);
     if (rc) return rc;
     const void *req[] = {log_fgate, value, key, query, states, dhidden_final, dout,
                          dhidden_init, dlog_fgate, dvalue, dkey, dquery};
@@ -381,11 +385,11 @@ static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         if (e) return e;
         e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, value, key,
                           query, states, dhT_same, dout, dh0_same, dlog_fgate, p.wide ? (void *)dv1 : dvalue,
-                          p.wide ? (void *)dk1 : dkey, p.wide ? (void *)dq1 : dquery, ws, sub, p.wide);
+                          p.wide ? (void *)dk1 : dkey, p.wide ? (void *)dq1 : dquery, ws, sub, p.wide, p.beside);
         if (e) return e;
         e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, v_sw, key, query,
                           (const unsigned char *)states + p.resid, dhT_cross, do_sw, dh0_cross, (float *)dg2, dv2, dk2,
-                          dq2, ws, sub, p.wide);
+                          dq2, ws, sub, p.wide, p.beside);
         if (e) return e;
         if (p.wide) {
             e = launch_sum_rows(st, dtype, rows, dquery, (const float *)dq1, (const float *)dq2, 0);

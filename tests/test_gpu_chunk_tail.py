@@ -95,6 +95,14 @@ def test_tail_is_what_a_caller_would_fill_up(dtype, B, T, H, D, full):
         assert torch.equal(got, want)
 
 
+# (the workspace that head dimension 256 needs beside its passes' own makes their tiles wider than the passes would choose by
+# themselves: 128 for 64, and 64 for 32)
+@pytest.mark.parametrize("dtype,B,T,H,full", [(torch.bfloat16, 3, 288, 16, 384), (torch.float32, 3, 160, 16, 192)])
+def test_passes_of_256_features_take_the_tile_of_the_whole_call(dtype, B, T, H, full):
+    for got, want in zip(*_clean_and_filled(dtype, B, T, H, 256, full)):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_a_value_that_is_not_finite_in_the_last_tile_stays_with_its_sequence(D, value):
