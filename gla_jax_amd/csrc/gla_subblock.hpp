@@ -16,16 +16,35 @@
 
 namespace gla {
 
-// Head and remainder of 8 values in the element type: x = hi + lo up to 16 bits of mantissa for bf16.
+// Head and remainder of a pair of values, each pair in one register: x = hi + lo up to 16 bits of mantissa.  The heads are
+// widened again from the packed register (six instructions a pair); taken from the values one by one, every head is converted
+// a second time for it.
+__device__ __forceinline__ void split2(float x0, float x1, bf16x2 &hi, bf16x2 &lo)
+{
+    hi[0] = (__bf16)x0;
+    hi[1] = (__bf16)x1;
+    const uint32_t both = __builtin_bit_cast(uint32_t, hi);
+    lo[0] = (__bf16)(x0 - __uint_as_float(both << 16));
+    lo[1] = (__bf16)(x1 - __uint_as_float(both & 0xffff0000u));
+}
+// Head and remainder of 8 values in the element type.
 template <typename T>
 __device__ __forceinline__ void split8(const float *x, typename FragTypes<T>::d8 &hi, typename FragTypes<T>::d8 &lo)
 {
-    float h[8];
-    hi = pack8<T>(x);
-    unpack8(hi, h);
+    if constexpr (sizeof(T) == 4) {                            // (a float is its own head)
+        const float none[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        hi = pack8<T>(x);
+        lo = pack8<T>(none);
+        return;
+    } else {
+    bf16x2 h[4], l[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = x[e] - h[e];
-    lo = pack8<T>(h);
+    for (int e = 0; e < 4; ++e) split2(x[2 * e], x[2 * e + 1], h[e], l[e]);
+    const bf16x4 h0 = __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3), h1 = __builtin_shufflevector(h[2], h[3], 0, 1, 2, 3);
+    const bf16x4 l0 = __builtin_shufflevector(l[0], l[1], 0, 1, 2, 3), l1 = __builtin_shufflevector(l[2], l[3], 0, 1, 2, 3);
+    hi = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+    lo = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
 }
 // a b^T with both operands given as head + remainder (the remainder x remainder term is dropped)
 template <typename D8> __device__ __forceinline__ f32x4 mma_d_split(D8 ah, D8 al, D8 bh, D8 bl, f32x4 acc)
@@ -39,10 +58,17 @@ template <typename D8> __device__ __forceinline__ f32x4 mma_d_split(D8 ah, D8 al
 template <typename T>
 __device__ __forceinline__ void split4(f32x4 x, typename FragTypes<T>::t4 &hi, typename FragTypes<T>::t4 &lo)
 {
-    hi = pack4<T>(x);
+    if constexpr (sizeof(T) == 4) {
+        hi = x;
+        lo = f32x4{0.f, 0.f, 0.f, 0.f};
+        return;
+    } else {
+    bf16x2 h[2], l[2];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] -= (float)hi[e];
-    lo = pack4<T>(x);
+    for (int e = 0; e < 2; ++e) split2(x[2 * e], x[2 * e + 1], h[e], l[e]);
+    hi = __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3);
+    lo = __builtin_shufflevector(l[0], l[1], 0, 1, 2, 3);
+    }
 }
 // (the remainder x remainder term comes with the second product; A's registers serve both)
 template <typename T4> __device__ __forceinline__ f32x4 mma_t_split(T4 ah, T4 al, T4 bh, T4 bl, f32x4 acc)
