@@ -1,4 +1,5 @@
-// recurrent_gla forward for bf16 inputs on the matrix cores: one workgroup streams over the sequence of
+// recurrent_gla forward for bf16 inputs on the matrix cores (head dimension 64, and the lean form of both 64 and 128; the whole
+// forward at 128: gla_recurrent_stream_fwd2.hip): one workgroup streams over the sequence of
 // one (batch, head) pair with the [DK,DV] state in fp32 accumulator registers; no hidden state ever
 // touches HBM (gla.py:50-96 keeps the state of a program in registers the same way).
 //
@@ -74,8 +75,8 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
 
     // state: S[i][j][e] = state[dk = 16(nt0 + j) + 4c + e][dv = 16(wv + i NDV) + r]  (accumulator layout of a
     // (dk x dv) product tile): a lane's four values of a tile are neighbours in the [dv][dk] copy below, one 8-byte
-    // store per tile and precision.  (dv x dk) tiles needed an exchange inside the quads of lanes first, 16 vector
-    // instructions per tile; with the products of mma_t2 B4 T4096 H16 D128 went from 234 to 222 us.  The lean form
+    // store per tile and precision ((dv x dk) tiles needed an exchange inside the quads of lanes first, 16 vector
+    // instructions per tile).  The lean form
     // writes no copy and keeps (dv x dk) tiles, dk = 16(nt0 + j) + r and dv = 16(wv + i NDV) + 4c + e, whose decay is
     // one value per lane and tile (four take registers that it does not have: 71.6 -> 75 us).
     // In memory the four values lie in four rows.  Lanes of a quad read (write) four neighbours of one of them each and
@@ -231,9 +232,7 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
         }
 
         // ---- out^T[dv][i] in slices of 32 output features: state term, then the score blocks --------
-        // (a real loop at D = 128: one slice's temporaries live at a time)
-        constexpr int kSliceUnroll = KS > 2 ? 1 : KS;
-#pragma unroll kSliceUnroll
+#pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const int fo = 32 * ks;
             f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -338,7 +337,7 @@ int launch_recurrent_stream_fwd(hipStream_t st, int B, Segments sg, int H, int D
                                 void *hT, void *out)
 {
     if (D == 64) return launch_one<TO, 128, 64>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, out);
-    if (D == 128) return launch_one<TO, 64, 128>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, out);
+    if (D == 128) return launch_recurrent_stream_fwd2<TO>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, out);
     return GLA_ERR_UNSUPPORTED;
 }
 

@@ -31,6 +31,11 @@ int launch_recurrent_stream_fwd(hipStream_t st, int B, Segments sg, int H, int D
                                 const void *h0, const float *g, const void *v, const void *k, const void *q,
                                 void *hT, void *out);
 
+// The same with two waves per sub-block (head dimension 128).
+template <typename TO>
+int launch_recurrent_stream_fwd2(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0,
+                                 const float *g, const void *v, const void *k, const void *q, void *hT, void *out);
+
 // The forward in fp32 vector arithmetic (gla_recurrent_steps.hip): any element types and head dimension.
 // h0 may be null: the states start from zeros.
 template <typename T, typename TO>
