@@ -63,6 +63,11 @@ int launch_recurrent_stream_dq2(hipStream_t st, int B, Segments sg, int H, int D
                                 const void *h0, const float *g, const void *v, const void *k, const void *q,
                                 const void *dhT, const void *dout, void *dq, float *qdq);
 
+// The same sweep with two waves per sub-block (head dimension 128, `dout` in bf16).
+int launch_recurrent_stream_dq128(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0,
+                                  const float *g, const void *v, const void *k, const void *q, const void *dhT,
+                                  const void *dout, void *dq, float *qdq, int wide);
+
 // Sweep 2: dk, dv, dh0 and dlog_fgate (`dg` holds sweep 1's q*dq on entry).  wide != 0 (head dimension 128 only):
 // `dv` and `dk` are float arrays.
 int launch_recurrent_stream_rev(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, int dout_f32,

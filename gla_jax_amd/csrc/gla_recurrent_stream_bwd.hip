@@ -852,12 +852,10 @@ int launch_recurrent_stream_dq(hipStream_t st, int B, Segments sg, int H, int D,
         return launch_recurrent_stream_dq2(st, B, sg, H, D, reverse, hdt, dout_f32, h0, g, v, k, q, dhT, dout, dq,
                                            qdq);
     if (D != 128) return GLA_ERR_UNSUPPORTED;
-    if (wide)
-        return dout_f32
-                   ? launch_dq<float, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
-                   : launch_dq<BT, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
-    return dout_f32 ? launch_dq<float, 64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
-                    : launch_dq<BT, 64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
+    if (!dout_f32)
+        return launch_recurrent_stream_dq128(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq, wide);
+    return wide ? launch_dq<float, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
+                : launch_dq<float, 64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
 }
 
 }  // namespace gla
