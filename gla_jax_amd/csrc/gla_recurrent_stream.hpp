@@ -74,6 +74,11 @@ int launch_recurrent_stream_rev(hipStream_t st, int B, Segments sg, int H, int D
                                 const float *g, const void *v, const void *k, const void *q, const void *dhT,
                                 const void *dout, void *dh0, float *dg, void *dv, void *dk, int wide = 0);
 
+// The same sweep with two waves per sub-block (head dimension 128, `dout` in bf16).
+int launch_recurrent_stream_rev128(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const float *g,
+                                   const void *v, const void *k, const void *q, const void *dhT, const void *dout, void *dh0,
+                                   float *dg, void *dv, void *dk, int wide);
+
 // The same sweep with two waves per sub-block (head dimension 64).
 int launch_recurrent_stream_rev2(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, int dout_f32,
                                  const float *g, const void *v, const void *k, const void *q, const void *dhT,

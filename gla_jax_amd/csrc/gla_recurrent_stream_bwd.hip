@@ -14,6 +14,10 @@
 //   dq_i = e^{l_i} ((((S_in do_i) r_0 + G_0) r_1 + G_1) ... r_{I-1} + G_{I-1}) + e^{-s_i} G_I' + dA_ii k_i
 //          G_J = sum_{j in J} dA_ij (k e^{s})_j,  G_I' the same over j < i of the own sub-block,  dA = dO V^T
 // with the dyadic levels of the reference replacing the G_I' term when the gates of the sub-block are hard.
+//
+// These kernels, one wave per sub-block, are for head dimension 128 with `dout` in fp32, which enters the products as bf16 head +
+// remainder: the tile of the remainder is what does not fit beside the two-waves form of gla_recurrent_stream_bwd128.hip, which
+// takes a dout in bf16 (B4 T4096 H16 D128, sweep 2: 320 us in this form, 244 there).  Head dimension 64: gla_recurrent_stream_bwd2.hip.
 #include "gla_recurrent_stream_bwd.hpp"
 #include "gla_recurrent_stream.hpp"
 
@@ -25,10 +29,10 @@ typedef __bf16 BT;
 // sweep 1
 // ---------------------------------------------------------------------------------------------------
 // WIDE: dq is a float array (head dimension 256 adds two such runs and rounds once, gla_split.hip)
-template <typename TO, int C, int D, bool WIDE>
+template <int C, int D, bool WIDE>
 __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k,
-    const BT *__restrict__ q, const void *__restrict__ dhT, const TO *__restrict__ dout,
+    const BT *__restrict__ q, const void *__restrict__ dhT, const float *__restrict__ dout,
     std::conditional_t<WIDE, float, BT> *__restrict__ dq, float *__restrict__ qdq, Segments sg, int H, int reverse,
     int hdt)
 {
@@ -48,7 +52,6 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
     T *Sl = Sh + D * LS;                           // [D][LS]  ... and remainder
     T *xs = Sl + D * LS;                           // [NB][2][16][XS] per-wave scratch (hard gates only)
     float *rtab = reinterpret_cast<float *>(xs + NB * 2 * 16 * XS);   // [NB][D] exp(tau_m)
-    constexpr bool kSplitDout = sizeof(TO) == 4;   // an fp32 dout enters the products as bf16 head + remainder
 
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -92,7 +95,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
 
     f32x8 gN[KS];
     D8 qN[KS], kN[KS], vN[KS];
-    DoutRow<TO> dN[KS];
+    DoutRow<float> dN[KS];
     bool validN;
     int64_t rowN;
     auto fetch = [&](int n) {
@@ -138,7 +141,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
                 kf[ks] = kN[ks];
                 vf[ks] = vN[ks];
                 dof[ks] = dN[ks].operand();
-                if constexpr (kSplitDout) dofl[ks] = dN[ks].remainder();
+                dofl[ks] = dN[ks].remainder();
                 st8(Vn + wrow + 32 * ks, vf[ks]);
             }
 
@@ -146,7 +149,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
             f32x4 dAn = {0.f, 0.f, 0.f, 0.f}, dAt = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                if constexpr (kSplitDout) {
+                {
                     dAn = mma_d(dofl[ks], vf[ks], dAn);
                     dAt = mma_d(vf[ks], dofl[ks], dAt);
                 }
@@ -237,7 +240,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
 #pragma unroll
                 for (int k2 = 0; k2 < KS; ++k2) {
                     const D8 vj = ld8(Vn + L.nat + 16 * J * LS + 32 * k2);
-                    if constexpr (kSplitDout) da = mma_d(vj, dofl[k2], da);
+                    da = mma_d(vj, dofl[k2], da);
                     da = mma_d(vj, dof[k2], da);
                 }
             }
@@ -256,7 +259,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
                 for (int tt = 0; tt < 2; ++tt) {
                     acc[tt] = mma_d(ld8(Sl + L.own + (fo + 4 * tt) * LS + 32 * k2), dof[k2], acc[tt]);
                     const D8 sh = ld8(Sh + L.own + (fo + 4 * tt) * LS + 32 * k2);
-                    if constexpr (kSplitDout) acc[tt] = mma_d(sh, dofl[k2], acc[tt]);
+                    acc[tt] = mma_d(sh, dofl[k2], acc[tt]);
                     acc[tt] = mma_d(sh, dof[k2], acc[tt]);
                 }
             }
@@ -361,10 +364,10 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_dq_kernel(
 // dS' is the gradient w.r.t. the state after the block.
 // ---------------------------------------------------------------------------------------------------
 // WIDE: dv and dk are float arrays (see sweep 1)
-template <typename TO, int C, int D, bool WIDE>
+template <int C, int D, bool WIDE>
 __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
     const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k, const BT *__restrict__ q,
-    const void *__restrict__ dhT, const TO *__restrict__ dout, void *__restrict__ dh0,
+    const void *__restrict__ dhT, const float *__restrict__ dout, void *__restrict__ dh0,
     float *__restrict__ dg, std::conditional_t<WIDE, float, BT> *__restrict__ dv,
     std::conditional_t<WIDE, float, BT> *__restrict__ dk, Segments sg, int H, int reverse, int hdt)
 {
@@ -388,8 +391,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
     float *rtab = reinterpret_cast<float *>(xs + NB * 2 * 16 * XS);   // [NB][D] exp(tau_m)
     float *dltab = rtab + NB * D;                  // [NB][D] sub-block sums of q*dq - k*dk
     float *runtab = dltab + NB * D;                // [2][D]  sum over the later blocks of q*dq - k*dk, double-buffered
-    constexpr bool kSplitDout = sizeof(TO) == 4;   // an fp32 dout enters the products as bf16 head + remainder
-    T *tOl = reinterpret_cast<T *>(runtab + 2 * D);   // [C][LS]  the remainder of dout (fp32 dout only)
+    T *tOl = reinterpret_cast<T *>(runtab + 2 * D);   // [C][LS]  the remainder of dout
 
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -435,7 +437,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
 
     f32x8 gN[KS];
     D8 qN[KS], kN[KS], vN[KS];
-    DoutRow<TO> dN[KS];
+    DoutRow<float> dN[KS];
     bool validN;
     int64_t rowN;
     auto fetch = [&](int n) {
@@ -487,7 +489,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
                 vf[ks] = vN[ks];
                 dof[ks] = dN[ks].operand();
                 st8(tO + wrow + 32 * ks, dof[ks]);
-                if constexpr (kSplitDout) {
+                {
                     const D8 dofl = dN[ks].remainder();
                     st8(tOl + wrow + 32 * ks, dofl);
                     dAn = mma_d(dofl, vf[ks], dAn);
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
                         split8<T>(kch + 8 * ks, kh, kl);
                         a = mma_d_split(ld8(Qh + L.nat + 16 * I * LS + 32 * ks), ld8(Ql + L.nat + 16 * I * LS + 32 * ks),
                                         kh, kl, a);
-                        if constexpr (kSplitDout) da = mma_d(ld8(tOl + L.nat + 16 * I * LS + 32 * ks), vf[ks], da);
+                        da = mma_d(ld8(tOl + L.nat + 16 * I * LS + 32 * ks), vf[ks], da);
                         da = mma_d(ld8(tO + L.nat + 16 * I * LS + 32 * ks), vf[ks], da);
                         f32x8 rr = ld8(rtab + I * D + 32 * ks + 8 * c);
 #pragma unroll
@@ -681,10 +683,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
 #pragma unroll
                         for (int tt = 0; tt < 2; ++tt) {
                             const T4 oa = lds_tr4(tO + L.k4 + fo + 4 * tt + 16 * I * LS, LS);
-                            if constexpr (kSplitDout)
-                                acc[tt] = mma_t_split(oa, lds_tr4(tOl + L.k4 + fo + 4 * tt + 16 * I * LS, LS), bh4, bl4, acc[tt]);
-                            else
-                                acc[tt] = mma_t2(oa, oa, bl4, bh4, acc[tt]);
+                            acc[tt] = mma_t_split(oa, lds_tr4(tOl + L.k4 + fo + 4 * tt + 16 * I * LS, LS), bh4, bl4, acc[tt]);
                         }
                     }
                 }
@@ -751,10 +750,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
 #pragma unroll
                     for (int e = 0; e < 4; ++e) DS[i][nt][e] *= rr[e];
                     const T4 ob = lds_tr4(tO + ptl + 16 * I * LS + 16 * nt, LS);
-                    if constexpr (kSplitDout)
-                        DS[i][nt] = mma_t_split(qah, qal, ob, lds_tr4(tOl + ptl + 16 * I * LS + 16 * nt, LS), DS[i][nt]);
-                    else
-                        DS[i][nt] = mma_t2(qah, qal, ob, ob, DS[i][nt]);
+                    DS[i][nt] = mma_t_split(qah, qal, ob, lds_tr4(tOl + ptl + 16 * I * LS + 16 * nt, LS), DS[i][nt]);
                 }
             }
         }
@@ -788,7 +784,7 @@ __global__ __launch_bounds__(C * 4) void recurrent_stream_rev_kernel(
                 store_hidden1(dh0, hdt, bh * D * D + (int64_t)(16 * (w + i * NB) + 4 * c + e) * D + 16 * nt + r, DS[i][nt][e]);
 }
 
-template <typename TO, int C, int D, bool WIDE>
+template <int C, int D, bool WIDE>
 static int launch_dq(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
                      const void *v, const void *k, const void *q, const void *dhT, const void *dout, void *dq,
                      float *qdq)
@@ -798,16 +794,16 @@ static int launch_dq(hipStream_t st, int B, Segments sg, int H, int reverse, int
     constexpr int XS = 32 + 16 / (int)sizeof(T);
     const size_t lds = ((size_t)(3 * C + 2 * D) * LS + (size_t)(C / 16) * 2 * 16 * XS) * sizeof(T) +
                        (size_t)(C / 16) * D * sizeof(float);
-    auto kern = recurrent_stream_dq_kernel<TO, C, D, WIDE>;
+    auto kern = recurrent_stream_dq_kernel<C, D, WIDE>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q,
-                       dhT, (const TO *)dout, (std::conditional_t<WIDE, float, T> *)dq, qdq, sg, H, reverse, hdt);
+                       dhT, (const float *)dout, (std::conditional_t<WIDE, float, T> *)dq, qdq, sg, H, reverse, hdt);
     return launch_status();
 }
 
-template <typename TO, int C, int D, bool WIDE>
+template <int C, int D, bool WIDE>
 static int launch_rev(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const float *g, const void *v,
                       const void *k, const void *q, const void *dhT, const void *dout, void *dh0,
                       float *dg, void *dv, void *dk)
@@ -815,15 +811,15 @@ static int launch_rev(hipStream_t st, int B, Segments sg, int H, int reverse, in
     typedef BT T;
     constexpr int LS = TileGeom<T, D>::kStride;
     constexpr int XS = 32 + 16 / (int)sizeof(T);
-    const size_t lds = ((size_t)(3 * C + 2 * D + (sizeof(TO) == 4 ? C : 0)) * LS + (size_t)(C / 16) * 2 * 16 * XS) *
+    const size_t lds = ((size_t)(4 * C + 2 * D) * LS + (size_t)(C / 16) * 2 * 16 * XS) *
                            sizeof(T) +
                        (size_t)(2 * (C / 16) + 2) * D * sizeof(float);
-    auto kern = recurrent_stream_rev_kernel<TO, C, D, WIDE>;
+    auto kern = recurrent_stream_rev_kernel<C, D, WIDE>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q,
-                       dhT, (const TO *)dout, dh0, dg, (std::conditional_t<WIDE, float, T> *)dv,
+                       dhT, (const float *)dout, dh0, dg, (std::conditional_t<WIDE, float, T> *)dv,
                        (std::conditional_t<WIDE, float, T> *)dk, sg, H, reverse, hdt);
     return launch_status();
 }
@@ -836,12 +832,10 @@ int launch_recurrent_stream_rev(hipStream_t st, int B, Segments sg, int H, int D
         return launch_recurrent_stream_rev2(st, B, sg, H, D, reverse, hdt, dout_f32, g, v, k, q, dhT, dout, dh0, dg,
                                             dv, dk);
     if (D != 128) return GLA_ERR_UNSUPPORTED;
-    if (wide)
-        return dout_f32
-                   ? launch_rev<float, 64, 128, true>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
-                   : launch_rev<BT, 64, 128, true>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
-    return dout_f32 ? launch_rev<float, 64, 128, false>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
-                    : launch_rev<BT, 64, 128, false>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
+    if (!dout_f32)
+        return launch_recurrent_stream_rev128(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk, wide);
+    return wide ? launch_rev<64, 128, true>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
+                : launch_rev<64, 128, false>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
 }
 
 int launch_recurrent_stream_dq(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, int dout_f32,
@@ -854,8 +848,8 @@ int launch_recurrent_stream_dq(hipStream_t st, int B, Segments sg, int H, int D,
     if (D != 128) return GLA_ERR_UNSUPPORTED;
     if (!dout_f32)
         return launch_recurrent_stream_dq128(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq, wide);
-    return wide ? launch_dq<float, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
-                : launch_dq<float, 64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
+    return wide ? launch_dq<64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
+                : launch_dq<64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
 }
 
 }  // namespace gla
