@@ -217,13 +217,14 @@ extern "C" size_t gla_chunk_bwd_workspace_bytes(int64_t B, int64_t T, int64_t H,
     return plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p) == GLA_OK ? p.bwd_bytes() : 0;
 }
 
-// wide != 0 (bf16 data at head dimension 128 only): `out` is a float array.  `beside` is not 0 in a pass of head dimension
+// wide (bf16 data at head dimension 128 only): the pass of head dimension 256 that this is, 1 (`out` is a float array) or 2 (the
+// other half's value rows; `out1`, what pass 1 left, is added), see launch_chunk_out.  `beside` is not 0 in a pass of head dimension
 // 256: its tile has to be the one that the whole call was planned (and its workspace cut up) with.
 static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
                          int64_t chunk_size, gla_dtype dtype, gla_dtype hidden_dtype, const void *hidden_init,
                          const float *log_fgate, const void *value, const void *key, const void *query,
                          void *hidden_final, void *out, void *states, void *workspace, size_t workspace_bytes,
-                         int wide, size_t beside = 0)
+                         int wide, size_t beside = 0, const float *out1 = nullptr)
 {
     ChunkPlan p;
     int rc = plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p, hidden_dtype, beside);
@@ -244,23 +245,35 @@ static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         hipStream_t st = (hipStream_t)stream;
         const size_t sub = p.prod + p.decay + p.states;
         if (wide) return GLA_ERR_UNSUPPORTED;
-        unsigned char *v_sw = ws + sub, *out2 = v_sw + p.rows, *out1 = out2 + p.rows_f32,
+        unsigned char *v_sw = ws + sub, *out2 = v_sw + p.rows, *out1_ws = out2 + p.rows_f32,
                       *h0_same = out2 + (p.wide ? 2 : 1) * p.rows_f32, *h0_cross = h0_same + p.hid,
                       *hT_same = h0_cross + p.hid, *hT_cross = hT_same + p.hid;
         int e = launch_hidden_blocks(st, hidden_dtype, B * H, const_cast<void *>(hidden_init), h0_same, h0_cross, 1);
         if (e) return e;
-        e = launch_swap_halves(st, dtype, B * T * H, v_sw, value);
-        if (e) return e;
-        e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_same, log_fgate, value,
-                          key, query, hT_same, p.wide ? (void *)out1 : out, states, ws, sub, p.wide, p.beside);
-        if (e) return e;
-        e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_cross, log_fgate, v_sw,
-                          key, query, hT_cross, out2, states ? (unsigned char *)states + p.resid : nullptr, ws, sub,
-                          p.wide, p.beside);
-        if (e) return e;
-        e = p.wide ? launch_sum_rows(st, dtype, B * T * H, out, (const float *)out1, (const float *)out2, 1)
-                   : launch_add_rows(st, dtype, B * T * H, out, out2, 1);
-        if (e) return e;
+        void *states2 = states ? (unsigned char *)states + p.resid : nullptr;
+        if (p.wide) {
+            // bf16 data: the second pass's kernels take the other half's value rows where they lie and add what the first left
+            // in fp32, so that `out` is rounded once (B2 T4096 H6, with an exchanged copy
+            // and a kernel for the sum: 195 -> 166 us).  The workspace's size, which a caller asks for and which decides what the static
+            // array takes, is still the one with the copies.
+            e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_same, log_fgate, value, key,
+                              query, hT_same, out1_ws, states, ws, sub, 1, p.beside);
+            if (e) return e;
+            e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_cross, log_fgate, value, key,
+                              query, hT_cross, out, states2, ws, sub, 2, p.beside, (const float *)out1_ws);
+            if (e) return e;
+        } else {
+            e = launch_swap_halves(st, dtype, B * T * H, v_sw, value);
+            if (e) return e;
+            e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_same, log_fgate, value, key,
+                              query, hT_same, out, states, ws, sub, 0, p.beside);
+            if (e) return e;
+            e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_cross, log_fgate, v_sw, key,
+                              query, hT_cross, out2, states2, ws, sub, 0, p.beside);
+            if (e) return e;
+            e = launch_add_rows(st, dtype, B * T * H, out, out2, 1);
+            if (e) return e;
+        }
         return launch_hidden_blocks(st, hidden_dtype, B * H, hidden_final, hT_same, hT_cross, 0);
     }
     void *prodT = (void *)ws;
@@ -284,7 +297,7 @@ static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         int e = 0;
         if (stages & 1)
             e = launch_chunk_outer<E, C_, D_, DM_>(st, 0, (int)B, (int)T, (int)H, log_fgate, value, key, prodT, decay,
-                                                   pexp);
+                                                   pexp, wide == 2);
         if (e) return e;
         if (stages & 2)
             e = launch_chunk_scan<E, D_, DM_>(st, (int)(B * H), N, 0, hidden_dtype, hidden_init, prodT, decay, pexp,
@@ -295,8 +308,10 @@ static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
                                                  slots, out);
         if ((stages & 4) && wide) {
             if constexpr (sizeof(E) == 2 && D_ == 128 && DM_ == 128)
-                e = launch_chunk_out<E, C_, D_, DM_, true>(st, (int)B, (int)T, (int)H, log_fgate, value, key, query,
-                                                           out_states, slots, out);
+                e = wide == 1 ? launch_chunk_out<E, C_, D_, DM_, 1>(st, (int)B, (int)T, (int)H, log_fgate, value, key, query,
+                                                                    out_states, slots, out)
+                              : launch_chunk_out<E, C_, D_, DM_, 2>(st, (int)B, (int)T, (int)H, log_fgate, value, key, query,
+                                                                    out_states, slots, out, out1);
             else
                 e = GLA_ERR_UNSUPPORTED;
         }
@@ -344,13 +359,15 @@ extern "C" int gla_chunk_fwd_static(void *stream, int64_t B, int64_t T, int64_t 
                                 value, key, query, hidden_final, out, states, ws, kStaticScratchBytes);
 }
 
-// wide != 0 (bf16 data at head dimension 128 only): `dvalue`, `dkey`, `dquery` are float arrays; `beside` as in the forward
+// wide, `beside` as in the forward: in pass 1 `dvalue`, `dkey`, `dquery` are float arrays, in pass 2 `dv1`, `dk1`, `dq1` are what
+// they were left as, and `dlog_fgate` holds pass 1's
 static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t H, int64_t DK, int64_t DV,
                          int64_t chunk_size, gla_dtype dtype, gla_dtype hidden_dtype, const float *log_fgate,
                          const void *value, const void *key, const void *query, const void *states,
                          const void *dhidden_final, const void *dout, void *dhidden_init, float *dlog_fgate,
                          void *dvalue, void *dkey, void *dquery, void *workspace, size_t workspace_bytes, int wide,
-                         size_t beside = 0)
+                         size_t beside = 0, const float *dv1 = nullptr, const float *dk1 = nullptr,
+                         const float *dq1 = nullptr)
 {
     ChunkPlan p;
     int rc = plan_chunk(B, T, H, DK, DV, chunk_size, dtype, &p, hidden_dtype, beside);
@@ -372,42 +389,44 @@ static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         const size_t sub = p.prod + p.decay + p.bwd_states * p.states;
         if (wide) return GLA_ERR_UNSUPPORTED;
         unsigned char *v_sw = ws + sub, *do_sw = v_sw + p.rows, *dg2 = do_sw + p.rows, *dq2 = dg2 + p.rows_f32,
-                      *dk2 = dq2 + p.rows_f32, *dv2 = dk2 + p.rows_f32, *dq1 = dv2 + p.rows_f32,
-                      *dk1 = dq1 + p.rows_f32, *dv1 = dk1 + p.rows_f32,
+                      *dk2 = dq2 + p.rows_f32, *dv2 = dk2 + p.rows_f32, *dq1_ws = dv2 + p.rows_f32,
+                      *dk1_ws = dq1_ws + p.rows_f32, *dv1_ws = dk1_ws + p.rows_f32,
                       *dhT_same = dv2 + (p.wide ? 4 : 1) * p.rows_f32, *dhT_cross = dhT_same + p.hid,
                       *dh0_same = dhT_cross + p.hid, *dh0_cross = dh0_same + p.hid;
         const int64_t rows = B * T * H;
         int e = launch_hidden_blocks(st, hidden_dtype, B * H, const_cast<void *>(dhidden_final), dhT_same, dhT_cross, 1);
         if (e) return e;
-        e = launch_swap_halves(st, dtype, rows, v_sw, value);
-        if (e) return e;
-        e = launch_swap_halves(st, dtype, rows, do_sw, dout);
-        if (e) return e;
-        e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, value, key,
-                          query, states, dhT_same, dout, dh0_same, dlog_fgate, p.wide ? (void *)dv1 : dvalue,
-                          p.wide ? (void *)dk1 : dkey, p.wide ? (void *)dq1 : dquery, ws, sub, p.wide, p.beside);
-        if (e) return e;
-        e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, v_sw, key, query,
-                          (const unsigned char *)states + p.resid, dhT_cross, do_sw, dh0_cross, (float *)dg2, dv2, dk2,
-                          dq2, ws, sub, p.wide, p.beside);
-        if (e) return e;
+        const unsigned char *states2 = (const unsigned char *)states + p.resid;
         if (p.wide) {
-            e = launch_sum_rows(st, dtype, rows, dquery, (const float *)dq1, (const float *)dq2, 0);
+            // as in the forward (a training step of B2 T4096 H6: 637 -> 535 us; the second pass's gradient kernel 162 against
+            // 120 us, but two copies of 12, three sums of 25 and one of 30 less)
+            e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, value, key, query,
+                              states, dhT_same, dout, dh0_same, dlog_fgate, dv1_ws, dk1_ws, dq1_ws, ws, sub, 1, p.beside);
             if (e) return e;
-            e = launch_sum_rows(st, dtype, rows, dkey, (const float *)dk1, (const float *)dk2, 0);
-            if (e) return e;
-            e = launch_sum_rows(st, dtype, rows, dvalue, (const float *)dv1, (const float *)dv2, 1);
+            e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, value, key, query,
+                              states2, dhT_cross, dout, dh0_cross, dlog_fgate, dvalue, dkey, dquery, ws, sub, 2, p.beside,
+                              (const float *)dv1_ws, (const float *)dk1_ws, (const float *)dq1_ws);
             if (e) return e;
         } else {
+            e = launch_swap_halves(st, dtype, rows, v_sw, value);
+            if (e) return e;
+            e = launch_swap_halves(st, dtype, rows, do_sw, dout);
+            if (e) return e;
+            e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, value, key, query,
+                              states, dhT_same, dout, dh0_same, dlog_fgate, dvalue, dkey, dquery, ws, sub, 0, p.beside);
+            if (e) return e;
+            e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, v_sw, key, query,
+                              states2, dhT_cross, do_sw, dh0_cross, (float *)dg2, dv2, dk2, dq2, ws, sub, 0, p.beside);
+            if (e) return e;
             e = launch_add_rows(st, dtype, rows, dquery, dq2, 0);
             if (e) return e;
             e = launch_add_rows(st, dtype, rows, dkey, dk2, 0);
             if (e) return e;
             e = launch_add_rows(st, dtype, rows, dvalue, dv2, 1);
             if (e) return e;
+            e = launch_add_rows(st, GLA_F32, rows, dlog_fgate, dg2, 0);
+            if (e) return e;
         }
-        e = launch_add_rows(st, GLA_F32, rows, dlog_fgate, dg2, 0);
-        if (e) return e;
         return launch_hidden_blocks(st, hidden_dtype, B * H, dhidden_init, dh0_same, dh0_cross, 0);
     }
     void *prodT = (void *)ws;
@@ -424,7 +443,7 @@ static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         int e = 0;
         if (stages & 1)
             e = launch_chunk_outer<E, C_, D_, DM_>(st, 1, (int)B, (int)T, (int)H, log_fgate, dout, query, prodT, decay,
-                                                   pexp);
+                                                   pexp, wide == 2);
         if (e) return e;
         if (stages & 2)
             e = launch_chunk_scan<E, D_, DM_>(st, (int)(B * H), N, 1, hidden_dtype, dhidden_final, prodT, decay, pexp,
@@ -435,9 +454,12 @@ static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
                                                   states, dstatesT, dstatesN, dlog_fgate, dvalue, dkey, dquery);
         if ((stages & 4) && wide) {
             if constexpr (sizeof(E) == 2 && D_ == 128 && DM_ == 128)
-                e = launch_chunk_grad<E, C_, D_, DM_, true>(st, (int)B, (int)T, (int)H, log_fgate, value, key, query,
-                                                            dout, states, dstatesT, dstatesN, dlog_fgate, dvalue, dkey,
-                                                            dquery);
+                e = wide == 1 ? launch_chunk_grad<E, C_, D_, DM_, 1>(st, (int)B, (int)T, (int)H, log_fgate, value, key, query,
+                                                                     dout, states, dstatesT, dstatesN, dlog_fgate, dvalue,
+                                                                     dkey, dquery)
+                              : launch_chunk_grad<E, C_, D_, DM_, 2>(st, (int)B, (int)T, (int)H, log_fgate, value, key, query,
+                                                                     dout, states, dstatesT, dstatesN, dlog_fgate, dvalue,
+                                                                     dkey, dquery, dv1, dk1, dq1);
             else
                 e = GLA_ERR_UNSUPPORTED;
         }

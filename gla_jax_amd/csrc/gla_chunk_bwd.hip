@@ -33,17 +33,18 @@
 
 namespace gla {
 
-// WIDE: dv, dk and dq are float arrays (the sums of two such runs are rounded once: head dimension 256,
-// gla_split.hip).
-template <typename T, int C, int D, int DM, bool WIDE>
+// WIDE: the passes of head dimension 256 (gla_split.hip).  1: dv, dk and dq are float arrays; 2: the value-side rows of the
+// other half, and what the first pass left (dv1, dk1, dq1, and dg in its place) is added before the one rounding.
+template <typename T, int C, int D, int DM, int WIDE>
 __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
     const float *__restrict__ g, const T *__restrict__ v, const T *__restrict__ k,
     const T *__restrict__ q, const T *__restrict__ dout, const T *__restrict__ statesN,
     const T *__restrict__ dstatesT, const T *__restrict__ dstatesN, float *__restrict__ dg,
-    std::conditional_t<WIDE, float, T> *__restrict__ dv, std::conditional_t<WIDE, float, T> *__restrict__ dk,
-    std::conditional_t<WIDE, float, T> *__restrict__ dq, int T_len, int H)
+    std::conditional_t<WIDE == 1, float, T> *__restrict__ dv, std::conditional_t<WIDE == 1, float, T> *__restrict__ dk,
+    std::conditional_t<WIDE == 1, float, T> *__restrict__ dq, const float *__restrict__ dv1,
+    const float *__restrict__ dk1, const float *__restrict__ dq1, int T_len, int H)
 {
-    typedef std::conditional_t<WIDE, float, T> TG;      // element type of dv, dk, dq
+    typedef std::conditional_t<WIDE == 1, float, T> TG;      // element type of dv, dk, dq
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4;
     constexpr int LS = TileGeom<T, D>::kStride;
     constexpr int XS = 32 + 16 / (int)sizeof(T);   // row stride of the per-wave slice scratch
@@ -75,14 +76,20 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
     const int64_t tok = (int64_t)b * T_len + (int64_t)n * C + 16 * w + r;
     const int64_t rowoff = live ? (tok * H + h) * DM : 0;     // DM features per row in memory (DM < D: see RowMap)
     g = rows_or_zeros(live, g);
-    v = rows_or_zeros(live, v);
+    const int other = WIDE == 2 ? ((h ^ 1) - h) * DM : 0;    // from the key side's rows to the value side's
+    v = rows_or_zeros(live, v + other);
     k = rows_or_zeros(live, k);
     q = rows_or_zeros(live, q);
-    dout = rows_or_zeros(live, dout);
+    dout = rows_or_zeros(live, dout + other);
     dg = rows_or_spare(live, dg);
-    dv = rows_or_spare(live, dv);
+    dv = rows_or_spare(live, dv + other);
     dk = rows_or_spare(live, dk);
     dq = rows_or_spare(live, dq);
+    if constexpr (WIDE == 2) {
+        dv1 = rows_or_zeros(live, dv1 + other);
+        dk1 = rows_or_zeros(live, dk1);
+        dq1 = rows_or_zeros(live, dq1);
+    }
     const int64_t bhn = ((int64_t)b * H + h) * N + n;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
@@ -566,6 +573,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                 o[e] = fast_exp2(p8[e]) * hacc + dq8[e];
                 dl8[e] += qr[e] * hacc;
             }
+            if constexpr (WIDE == 2) add_row_once<D, DM>(o, dq1 + rowoff + fo, c);
             st8_row_once<D, DM>(dq + rowoff + fo, c, pack8<TG>(o), live);
         }
         // -- dk: state term V dS'^T first, then the later sub-blocks in descending order
@@ -623,6 +631,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
                 o[e] = fast_exp2(s8[e]) * hacc + dk8[e];
                 dl8[e] -= krt[e] * hacc;
             }
+            if constexpr (WIDE == 2) add_row_once<D, DM>(o, dk1 + rowoff + fo, c);
             st8_row_once<D, DM>(dk + rowoff + fo, c, pack8<TG>(o), live);
         }
         // -- dv: state term K~ dS', and the own and the later sub-blocks in a sum of their own: the products differ in depth
@@ -654,6 +663,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
             float o[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = acc[e >> 2][e & 3] + rows[e >> 2][e & 3];
+            if constexpr (WIDE == 2) add_row_once<D, DM>(o, dv1 + rowoff + fo, c);
             st8_row_once<D, DM>(dv + rowoff + fo, c, pack8<TG>(o), live);
         }
         // -- dL of the slice is complete: reverse cumsum inside the sub-block (gla.py:616-617), then, once
@@ -686,6 +696,7 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o.v[e] += t.v[e];
             }
+            if constexpr (WIDE == 2) add_row_once<D, DM>(o.v, dg + rowoff + fo, c);
             st8_row_once<D, DM>(dg + rowoff + fo, c, o, live);
         }
         if (ks + 1 < KS) {
@@ -695,10 +706,11 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
     }
 }
 
-template <typename T, int C, int D, int DM, bool WIDE>
+template <typename T, int C, int D, int DM, int WIDE>
 int launch_chunk_grad(hipStream_t st, int B, int T_len, int H, const float *g, const void *v, const void *k,
                       const void *q, const void *dout, const void *statesN, const void *dstatesT,
-                      const void *dstatesN, float *dg, void *dv, void *dk, void *dq)
+                      const void *dstatesN, float *dg, void *dv, void *dk, void *dq, const float *dv1, const float *dk1,
+                      const float *dq1)
 {
     constexpr int LS = TileGeom<T, D>::kStride;
     constexpr int XS = 32 + 16 / (int)sizeof(T);
@@ -708,24 +720,28 @@ int launch_chunk_grad(hipStream_t st, int B, int T_len, int H, const float *g, c
                        ((size_t)(3 * NB + 1) * D + NB * 32) * sizeof(float) +
                        ((C - 96) * LS >= NB * 16 * 32 || sizeof(T) != 2 ? 0 : (size_t)NB * 16 * 32 * sizeof(T));
     auto kern = chunk_grad_kernel<T, C, D, DM, WIDE>;
-    typedef std::conditional_t<WIDE, float, T> TG;
+    typedef std::conditional_t<WIDE == 1, float, T> TG;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid((T_len + C - 1) / C * H, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q,
                        (const T *)dout, (const T *)statesN, (const T *)dstatesT, (const T *)dstatesN, dg,
-                       (TG *)dv, (TG *)dk, (TG *)dq, T_len, H);
+                       (TG *)dv, (TG *)dk, (TG *)dq, dv1, dk1, dq1, T_len, H);
     return launch_status();
 }
 
 #define GLA_INST_GRAD_AS(T, C, D, DM, WIDE)                                                                    \
     template int launch_chunk_grad<T, C, D, DM, WIDE>(hipStream_t, int, int, int, const float *, const void *, \
                                                       const void *, const void *, const void *, const void *, \
-                                                      const void *, const void *, float *, void *, void *, void *);
-#define GLA_INST_GRAD(T, C, D, DM) GLA_INST_GRAD_AS(T, C, D, DM, false)
+                                                      const void *, const void *, float *, void *, void *, void *, \
+                                                      const float *, const float *, const float *);
+#define GLA_INST_GRAD(T, C, D, DM) GLA_INST_GRAD_AS(T, C, D, DM, 0)
 GLA_FOR_EACH_CHUNK_CONFIG(GLA_INST_GRAD)
-GLA_INST_GRAD_AS(__bf16, 128, 128, 128, true)
-GLA_INST_GRAD_AS(__bf16, 64, 128, 128, true)
-GLA_INST_GRAD_AS(__bf16, 32, 128, 128, true)
+GLA_INST_GRAD_AS(__bf16, 128, 128, 128, 1)
+GLA_INST_GRAD_AS(__bf16, 128, 128, 128, 2)
+GLA_INST_GRAD_AS(__bf16, 64, 128, 128, 1)
+GLA_INST_GRAD_AS(__bf16, 64, 128, 128, 2)
+GLA_INST_GRAD_AS(__bf16, 32, 128, 128, 1)
+GLA_INST_GRAD_AS(__bf16, 32, 128, 128, 2)
 
 }  // namespace gla

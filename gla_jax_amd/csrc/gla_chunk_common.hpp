@@ -193,6 +193,14 @@ __device__ __forceinline__ void st8_row_once(P *row_ks, int c, const V &v, bool 
     if ((DM == D || live) && RowMap<D, DM>::live(c)) st8_once(row_ks + 8 * c, v);
 }
 
+// Adds the first pass's 8 values of a row to the second pass's (head dimension 256).
+template <int D, int DM> __device__ __forceinline__ void add_row_once(float (&o)[8], const float *row_ks, int c)
+{
+    const f32x8 t = ld8_row_once<D, DM>(row_ks, c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] += t.v[e];
+}
+
 // The last chunk of a sequence may have fewer than C tokens (a multiple of 16): a wave past the end reads a row of zeros
 // in place of its rows, which is what padded tokens are (a zero log-gate, key, query, value and cotangent leave every
 // other token alone), and stores its results to a row that nobody reads.  Both are a scalar choice between two base

@@ -22,11 +22,13 @@ namespace gla {
 // Resources: two tiles (keys of all but the last sub-block, values), 32 staged state rows and a table
 // fit twice into a CU's LDS, and the register budget is held to what lets two workgroups share a CU, so
 // that one loads while the other computes.
-// WIDE: `out` is a float array (the sum of two such runs is rounded once: head dimension 256, gla_split.hip).
-template <typename T, int C, int D, int DM, bool WIDE>
+// WIDE: the passes of head dimension 256 (gla_split.hip).  1: `out` is a float array; 2: the value rows of the other half, and
+// `out1`, what the first pass left, is added before the one rounding.
+template <typename T, int C, int D, int DM, int WIDE>
 __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C < 128 && D < 128 ? 8 : C / 32))) void chunk_out_kernel(
     const float *__restrict__ g, const T *__restrict__ v, const T *__restrict__ k, const T *__restrict__ q,
-    const T *__restrict__ states, int slots, std::conditional_t<WIDE, float, T> *__restrict__ out, int T_len, int H)
+    const T *__restrict__ states, int slots, std::conditional_t<WIDE == 1, float, T> *__restrict__ out,
+    const float *__restrict__ out1, int T_len, int H)
 {
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4;
     constexpr int LS = TileGeom<T, D>::kStride;
@@ -54,10 +56,12 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
     const int64_t tok = (int64_t)b * T_len + (int64_t)n * C + 16 * w + r;
     const int64_t rowoff = live ? (tok * H + h) * DM : 0;     // DM features per row in memory (DM < D: see RowMap)
     g = rows_or_zeros(live, g);
-    v = rows_or_zeros(live, v);
+    const int other = WIDE == 2 ? ((h ^ 1) - h) * DM : 0;    // from the key side's rows to the value side's
+    v = rows_or_zeros(live, v + other);
     k = rows_or_zeros(live, k);
     q = rows_or_zeros(live, q);
-    out = rows_or_spare(live, out);
+    out = rows_or_spare(live, out + other);
+    if constexpr (WIDE == 2) out1 = rows_or_zeros(live, out1 + other);
     const TrLane<T> L = make_tr_lane<T>(LS);
     const int wrow = 16 * w * LS + L.nat;          // this lane's row of a [token][feature] tile
 
@@ -203,7 +207,8 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
         float o[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = acc[e >> 2][e & 3];
-        st8_row_once<D, DM>(out + rowoff + fo, c, pack8<std::conditional_t<WIDE, float, T>>(o), live);
+        if constexpr (WIDE == 2) add_row_once<D, DM>(o, out1 + rowoff + fo, c);
+        st8_row_once<D, DM>(out + rowoff + fo, c, pack8<std::conditional_t<WIDE == 1, float, T>>(o), live);
         if (ks + 1 < KS) {
             __syncthreads();             // every wave is done with the staged rows
             stage_store();
@@ -213,9 +218,9 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
     }
 }
 
-template <typename T, int C, int D, int DM, bool WIDE>
+template <typename T, int C, int D, int DM, int WIDE>
 int launch_chunk_out(hipStream_t st, int B, int T_len, int H, const float *g, const void *v, const void *k,
-                     const void *q, const void *states, int slots, void *out)
+                     const void *q, const void *states, int slots, void *out, const float *out1)
 {
     constexpr int LS = TileGeom<T, D>::kStride;
     const size_t lds = (size_t)(2 * C - 16 + 32) * LS * sizeof(T) + (size_t)(C / 16) * D * sizeof(float);
@@ -224,17 +229,20 @@ int launch_chunk_out(hipStream_t st, int B, int T_len, int H, const float *g, co
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid((T_len + C - 1) / C * H, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q,
-                       (const T *)states, slots, (std::conditional_t<WIDE, float, T> *)out, T_len, H);
+                       (const T *)states, slots, (std::conditional_t<WIDE == 1, float, T> *)out, out1, T_len, H);
     return launch_status();
 }
 
 #define GLA_INST_OUT_AS(T, C, D, DM, WIDE)                                                                   \
     template int launch_chunk_out<T, C, D, DM, WIDE>(hipStream_t, int, int, int, const float *, const void *, \
-                                                     const void *, const void *, const void *, int, void *);
-#define GLA_INST_OUT(T, C, D, DM) GLA_INST_OUT_AS(T, C, D, DM, false)
+                                                     const void *, const void *, const void *, int, void *, const float *);
+#define GLA_INST_OUT(T, C, D, DM) GLA_INST_OUT_AS(T, C, D, DM, 0)
 GLA_FOR_EACH_CHUNK_CONFIG(GLA_INST_OUT)
-GLA_INST_OUT_AS(__bf16, 128, 128, 128, true)
-GLA_INST_OUT_AS(__bf16, 64, 128, 128, true)
-GLA_INST_OUT_AS(__bf16, 32, 128, 128, true)
+GLA_INST_OUT_AS(__bf16, 128, 128, 128, 1)
+GLA_INST_OUT_AS(__bf16, 128, 128, 128, 2)
+GLA_INST_OUT_AS(__bf16, 64, 128, 128, 1)
+GLA_INST_OUT_AS(__bf16, 64, 128, 128, 2)
+GLA_INST_OUT_AS(__bf16, 32, 128, 128, 1)
+GLA_INST_OUT_AS(__bf16, 32, 128, 128, 2)
 
 }  // namespace gla

@@ -37,8 +37,9 @@ namespace gla {
 
 template <typename T, int C, int D, int DM>
 // prodT: the per-chunk products in the library's own layout and type (gla_chunk_state.hip), pexp: their exponents
+// other_half != 0: head h takes the rows of x of head h ^ 1 (the second pass of head dimension 256)
 int launch_chunk_outer(hipStream_t st, int mode, int B, int T_len, int H, const float *g, const void *x,
-                       const void *y, void *prodT, float *decay, unsigned char *pexp);
+                       const void *y, void *prodT, float *decay, unsigned char *pexp, int other_half);
 
 template <typename T, int D, int DM>
 // hdt = gla_dtype of hin / hout (hidden_init and hidden_final, or their cotangents)
@@ -46,17 +47,19 @@ int launch_chunk_scan(hipStream_t st, int BH, int N, int reverse, int hdt, const
                       const float *decay, const unsigned char *pexp, void *statesT, void *statesN, void *hout,
                       int tail, int tiled);
 
-// WIDE (built for bf16 at D = 128 only): `out`, or `dv`, `dk`, `dq`, are float arrays, for the two passes that make
-// up head dimension 256
-template <typename T, int C, int D, int DM, bool WIDE = false>
+// WIDE (built for bf16 at D = 128 only): the two passes that make up head dimension 256.  1: `out`, or `dv`, `dk`, `dq`, are
+// float arrays.  2: head h takes the value-side rows (v, dout, out, dv) of head h ^ 1, and the first pass's results, `out1` or
+// `dv1`, `dk1`, `dq1` (in the places of `out`, `dv`, `dk`, `dq`) and `dg`, are added before the one rounding.
+template <typename T, int C, int D, int DM, int WIDE = 0>
 // states: the chunk-start states the kernel contracts over dk: for 16-bit data the tiled [dk][dv] array with `slots`
 // states per (b,h) (the residual, or its stand-in in the workspace), for fp32 data the [dv][dk] array of the workspace
 int launch_chunk_out(hipStream_t st, int B, int T_len, int H, const float *g, const void *v, const void *k,
-                     const void *q, const void *states, int slots, void *out);
+                     const void *q, const void *states, int slots, void *out, const float *out1 = nullptr);
 
-template <typename T, int C, int D, int DM, bool WIDE = false>
+template <typename T, int C, int D, int DM, int WIDE = 0>
 int launch_chunk_grad(hipStream_t st, int B, int T_len, int H, const float *g, const void *v, const void *k,
                       const void *q, const void *dout, const void *statesN, const void *dstatesT,
-                      const void *dstatesN, float *dg, void *dv, void *dk, void *dq);
+                      const void *dstatesN, float *dg, void *dv, void *dk, void *dq, const float *dv1 = nullptr,
+                      const float *dk1 = nullptr, const float *dq1 = nullptr);
 
 }  // namespace gla

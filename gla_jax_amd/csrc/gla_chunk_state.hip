@@ -46,7 +46,7 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
                                                             const T *__restrict__ y,
                                                             typename Prod<T>::type *__restrict__ prodT,
                                                             float *__restrict__ decay,
-                                                            unsigned char *__restrict__ pexp, int T_len, int H)
+                                                            unsigned char *__restrict__ pexp, int T_len, int H, int other_half)
 {
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4, NT = D / 16;
     constexpr int LS = TileGeom<T, D>::kStride;
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
     const int64_t tok = (int64_t)b * T_len + (int64_t)n * C + 16 * w + r;
     const int64_t rowoff = live ? (tok * H + h) * DM : 0;     // DM features per row in memory (DM < D: see RowMap)
     g = rows_or_zeros(live, g);
-    x = rows_or_zeros(live, x);
+    x = rows_or_zeros(live, x + ((h ^ other_half) - h) * DM);
     y = rows_or_zeros(live, y);
 
     float p[NV];
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(64) void chunk_scan_kernel(const void *__restrict__
 
 template <typename T, int C, int D, int DM>
 int launch_chunk_outer(hipStream_t st, int mode, int B, int T_len, int H, const float *g, const void *x,
-                       const void *y, void *prodT, float *decay, unsigned char *pexp)
+                       const void *y, void *prodT, float *decay, unsigned char *pexp, int other_half)
 {
     typedef typename Prod<T>::type P;
     constexpr int LS = TileGeom<T, D>::kStride;
@@ -335,13 +335,13 @@ int launch_chunk_outer(hipStream_t st, int mode, int B, int T_len, int H, const 
         static LdsGrant grant;
         if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
         hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)x, (const T *)y, (P *)prodT, decay, pexp, T_len,
-                           H);
+                           H, other_half);
     } else {
         auto kern = chunk_outer_kernel<T, C, D, DM, 1>;
         static LdsGrant grant;
         if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
         hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)x, (const T *)y, (P *)prodT, decay, pexp, T_len,
-                           H);
+                           H, other_half);
     }
     return launch_status();
 }
@@ -366,7 +366,7 @@ int launch_chunk_scan(hipStream_t st, int BH, int N, int reverse, int hdt, const
 
 #define GLA_INST_OUTER(T, C, D, DM)                                                                   \
     template int launch_chunk_outer<T, C, D, DM>(hipStream_t, int, int, int, int, const float *, const void *, \
-                                                 const void *, void *, float *, unsigned char *);
+                                                 const void *, void *, float *, unsigned char *, int);
 #define GLA_INST_SCAN(T, D, DM)                                                                       \
     template int launch_chunk_scan<T, D, DM>(hipStream_t, int, int, int, int, const void *, const void *, \
                                              const float *, const unsigned char *, void *, void *, void *, int, int);
