@@ -379,7 +379,9 @@ static int check_recurrent(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t 
 }  // namespace gla
 
 // ---- head dimension 256 as four problems of head dimension 128 (gla_split.hip) ---------------------------------
-// Two passes of the 128-feature kernels over 2H heads, their results left in fp32 and added with one rounding.
+// Two passes of the 128-feature kernels over 2H heads, the first one's results left in fp32 and added with one rounding by the
+// second, or, where the vector kernels run or dout is fp32, both left and added by kernels of their own (the workspace is sized
+// for that).
 // rows: one [B,T,H,256] array; hid: one [B,2H,128,128] array of states per segment (sized for fp32 states).
 namespace gla {
 struct SplitSizes {
@@ -583,28 +585,34 @@ static int recurrent_fwd_inner(void *stream, int64_t B, gla::Segments sg, int64_
         e = gla::launch_hidden_blocks(st, hidden_dtype, states * H, const_cast<void *>(hidden_init), h0_same, h0_cross, 1);
         if (e) return e;
     }
-    e = gla::launch_swap_halves(st, dtype, rows * H, v_sw, value);
-    if (e) return e;
-    // key half a with value half a on the arrays as they lie, then key half a with the other value half; `out` of
-    // both in fp32 (the recurrent_gla_naive flavour of the 128-feature kernels)
+    // key half a with value half a on the arrays as they lie, then key half a with the other value half's rows; `out` of the first
+    // in fp32 (the recurrent_gla_naive flavour of the 128-feature kernels), which the second adds before the one rounding
     if (lean) {
         e = gla::launch_recurrent_stream_state(st, B, sg, 2 * H, 128, reverse, hidden_dtype, hidden_init ? h0_same : nullptr,
                                                log_fgate, value, key, query, hT_same, g_shift, gate_sums);
         if (e) return e;
         e = gla::launch_recurrent_stream_state(st, B, sg, 2 * H, 128, reverse, hidden_dtype,
-                                               hidden_init ? h0_cross : nullptr, log_fgate, v_sw, key, query, hT_cross,
-                                               g_shift);
+                                               hidden_init ? h0_cross : nullptr, log_fgate, value, key, query, hT_cross,
+                                               g_shift, nullptr, 1);
         if (e) return e;
         return gla::launch_hidden_blocks(st, hidden_dtype, states * H, hidden_final, hT_same, hT_cross, 0);
     }
     e = recurrent_fwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_same, log_fgate,
                           value, key, query, hT_same, out1);
     if (e) return e;
-    e = recurrent_fwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_cross, log_fgate, v_sw,
-                          key, query, hT_cross, out2);
-    if (e) return e;
-    e = gla::launch_sum_rows(st, out_dtype, rows * H, out, (const float *)out1, (const float *)out2, 1);
-    if (e) return e;
+    if (sg.L > gla::kFewSteps) {
+        auto run = out_dtype == GLA_F32 ? gla::launch_recurrent_stream_fwd2<float> : gla::launch_recurrent_stream_fwd2<__bf16>;
+        e = run(st, B, sg, 2 * H, reverse, hidden_dtype, h0_cross, log_fgate, value, key, query, hT_cross, out, (const float *)out1);
+        if (e) return e;
+    } else {        // the vector kernels: a copy with the halves of every row exchanged, and the sum behind
+        e = gla::launch_swap_halves(st, dtype, rows * H, v_sw, value);
+        if (e) return e;
+        e = recurrent_fwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_cross, log_fgate, v_sw,
+                              key, query, hT_cross, out2);
+        if (e) return e;
+        e = gla::launch_sum_rows(st, out_dtype, rows * H, out, (const float *)out1, (const float *)out2, 1);
+        if (e) return e;
+    }
     return gla::launch_hidden_blocks(st, hidden_dtype, states * H, hidden_final, hT_same, hT_cross, 0);
 }
 
@@ -738,25 +746,38 @@ static int recurrent_bwd_inner(void *stream, int64_t B, gla::Segments sg, int64_
     if (e) return e;
     e = gla::launch_hidden_blocks(st, hidden_dtype, states * H, const_cast<void *>(dhidden_final), dhT_same, dhT_cross, 1);
     if (e) return e;
-    e = gla::launch_swap_halves(st, dtype, rows, v_sw, value);
-    if (e) return e;
-    e = gla::launch_swap_halves(st, out_dtype, rows, do_sw, dout);
-    if (e) return e;
     // hidden_final is not read by the kernels (sweep 1 forms the final state again in fp32); it is handed on as it is
     e = recurrent_bwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, out_dtype, reverse, h0_same, log_fgate,
                           value, key, query, hidden_final, dhT_same, dout, dh0_same, dlog_fgate, dv1, dk1, dq1, 1);
     if (e) return e;
-    e = recurrent_bwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, out_dtype, reverse, h0_cross, log_fgate,
-                          v_sw, key, query, hidden_final, dhT_cross, do_sw, dh0_cross, (float *)dg2, dv2, dk2, dq2, 1);
-    if (e) return e;
-    e = gla::launch_sum_rows(st, dtype, rows, dquery, (const float *)dq1, (const float *)dq2, 0);
-    if (e) return e;
-    e = gla::launch_sum_rows(st, dtype, rows, dkey, (const float *)dk1, (const float *)dk2, 0);
-    if (e) return e;
-    e = gla::launch_sum_rows(st, dtype, rows, dvalue, (const float *)dv1, (const float *)dv2, 1);
-    if (e) return e;
-    e = gla::launch_add_rows(st, GLA_F32, rows, dlog_fgate, dg2, 0);
-    if (e) return e;
+    if (dtype == GLA_BF16 && out_dtype == GLA_BF16) {
+        // the second pass takes the other half's value-side rows where they lie and adds what the first left, rounding once
+        // (a training step of B4 T2048 H8, with exchanged copies and kernels for the sums: 1131 -> 963 us)
+        const int h2 = (int)(2 * H);
+        e = gla::launch_recurrent_stream_dq128(st, (int)B, sg, h2, reverse, hidden_dtype, h0_cross, log_fgate, value, key, query,
+                                               dhT_cross, dout, dquery, (float *)dg2, 2, (const float *)dq1);
+        if (e) return e;
+        e = gla::launch_recurrent_stream_rev128(st, (int)B, sg, h2, reverse, hidden_dtype, log_fgate, value, key, query, dhT_cross,
+                                                dout, dh0_cross, (float *)dg2, dvalue, dkey, 2, (const float *)dv1,
+                                                (const float *)dk1, dlog_fgate);
+        if (e) return e;
+    } else {
+        e = gla::launch_swap_halves(st, dtype, rows, v_sw, value);
+        if (e) return e;
+        e = gla::launch_swap_halves(st, out_dtype, rows, do_sw, dout);
+        if (e) return e;
+        e = recurrent_bwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, out_dtype, reverse, h0_cross, log_fgate,
+                              v_sw, key, query, hidden_final, dhT_cross, do_sw, dh0_cross, (float *)dg2, dv2, dk2, dq2, 1);
+        if (e) return e;
+        e = gla::launch_sum_rows(st, dtype, rows, dquery, (const float *)dq1, (const float *)dq2, 0);
+        if (e) return e;
+        e = gla::launch_sum_rows(st, dtype, rows, dkey, (const float *)dk1, (const float *)dk2, 0);
+        if (e) return e;
+        e = gla::launch_sum_rows(st, dtype, rows, dvalue, (const float *)dv1, (const float *)dv2, 1);
+        if (e) return e;
+        e = gla::launch_add_rows(st, GLA_F32, rows, dlog_fgate, dg2, 0);
+        if (e) return e;
+    }
     return gla::launch_hidden_blocks(st, hidden_dtype, states * H, dhidden_init, dh0_same, dh0_cross, 0);
 }
 

@@ -38,7 +38,8 @@ template <typename TO, int C, int D, bool STATE = false>
 __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const __bf16 *__restrict__ v,
     const __bf16 *__restrict__ k, const __bf16 *__restrict__ q, void *__restrict__ hT,
-    TO *__restrict__ out, Segments sg, int H, int reverse, int hdt, int g_shift, float *__restrict__ gate_sums)
+    TO *__restrict__ out, Segments sg, int H, int reverse, int hdt, int g_shift, float *__restrict__ gate_sums,
+    int other_half)
 {
     typedef __bf16 T;
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4, NT = D / 16;
@@ -67,6 +68,7 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
     const int64_t seq = (seg.row0 * H + h) * D;      // element offset of (b, t = 0, h)
     const int64_t rowstride = (int64_t)H * D;
     const int64_t bh = (int64_t)seg.index * H + h;
+    if constexpr (STATE) v += ((h ^ other_half) - h) * D;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const int ptl = plain_tr_lane<T>(LS);
     const int wrow = 16 * w * LS + L.nat;          // this lane's row of a [token][feature] tile
@@ -315,7 +317,7 @@ __global__ __launch_bounds__(C * 4, STATE ? 2 : 1) void recurrent_stream_fwd_ker
 template <typename TO, int C, int D, bool STATE = false>
 static int launch_one(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
                       const void *v, const void *k, const void *q, void *hT, void *out, int g_shift = 0,
-                      float *gate_sums = nullptr)
+                      float *gate_sums = nullptr, int other_half = 0)
 {
     typedef __bf16 T;
     constexpr int LS = TileGeom<T, D>::kStride;
@@ -327,7 +329,7 @@ static int launch_one(hipStream_t st, int B, Segments sg, int H, int reverse, in
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, hT, (TO *)out,
-                       sg, H, reverse, hdt, g_shift, gate_sums);
+                       sg, H, reverse, hdt, g_shift, gate_sums, other_half);
     return launch_status();
 }
 
@@ -343,15 +345,15 @@ int launch_recurrent_stream_fwd(hipStream_t st, int B, Segments sg, int H, int D
 
 int launch_recurrent_stream_state(hipStream_t st, int B, Segments sg, int H, int D, int reverse, int hdt, const void *h0,
                                  const float *g, const void *v, const void *k, const void *q, void *hT, int g_shift,
-                                 float *gate_sums)
+                                 float *gate_sums, int other_half)
 {
     if (g_shift < -1 || g_shift > 1 || (g_shift && gate_sums)) return GLA_ERR_SHAPE;
     if (D == 64)
         return launch_one<__bf16, 128, 64, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, nullptr, g_shift,
-                                                 gate_sums);
+                                                 gate_sums, other_half);
     if (D == 128)
         return launch_one<__bf16, 64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, nullptr, g_shift,
-                                                 gate_sums);
+                                                 gate_sums, other_half);
     return GLA_ERR_UNSUPPORTED;
 }
 

@@ -18,15 +18,17 @@ namespace gla {
 // ---------------------------------------------------------------------------------------------------
 // sweep 1: dq and q*dq, the state S in accumulator registers
 // ---------------------------------------------------------------------------------------------------
-// WIDE: dq is a float array (head dimension 256 adds two such runs and rounds once, gla_split.hip)
-template <int C, int D, bool WIDE>
+// WIDE: the passes of head dimension 256 (gla_split.hip).  1: dq is a float array; 2: the value-side rows of the other half, and
+// dq1, what the first pass left, is added before the one rounding.
+template <int C, int D, int WIDE>
 __global__ __launch_bounds__(C * 8) void recurrent_stream_dq128_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k,
     const BT *__restrict__ q, const void *__restrict__ dhT, const BT *__restrict__ dout,
-    std::conditional_t<WIDE, float, BT> *__restrict__ dq, float *__restrict__ qdq, Segments sg, int H, int reverse, int hdt)
+    std::conditional_t<WIDE == 1, float, BT> *__restrict__ dq, float *__restrict__ qdq,
+    const float *__restrict__ dq1, Segments sg, int H, int reverse, int hdt)
 {
     typedef BT T;
-    typedef std::conditional_t<WIDE, float, BT> TG;
+    typedef std::conditional_t<WIDE == 1, float, BT> TG;
     constexpr int NB = C / 16, NW = 2 * NB, KS = D / 32, NT = D / 16;
     constexpr int DH = D / 2, KH = DH / 32;                          // a wave's key features, in slices of 32
     constexpr int RT = NT / NB, NTW = NT / 2;                        // its state tiles: RT value tiles x NTW key tiles
@@ -55,6 +57,11 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_dq128_kernel(
     const int h = blockIdx.x;
     const int64_t seq = (seg.row0 * H + h) * D;
     const int64_t rowstride = (int64_t)H * D;
+    if constexpr (WIDE == 2) {
+        const int other = ((h ^ 1) - h) * D;
+        v += other;
+        dout += other;
+    }
     const int64_t bh = (int64_t)seg.index * H + h;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
@@ -305,6 +312,11 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_dq128_kernel(
                 o[e] = el * acc[e >> 2][e & 3] + es * gq[e >> 2][e & 3] + dqo[e];
                 prod.v[e] = a[e] * o[e];
             }
+            if constexpr (WIDE == 2) {
+                const f32x8 t = ld8(dq1 + row + 32 * ks);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] += t.v[e];
+            }
             if (valid) {
                 st8(dq + row + 32 * ks, pack8<TG>(o));
                 st8(qdq + row + 32 * ks, prod);
@@ -365,10 +377,10 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_dq128_kernel(
     }
 }
 
-template <int C, int D, bool WIDE>
+template <int C, int D, int WIDE>
 static int launch_dq128(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
                         const void *v, const void *k, const void *q, const void *dhT, const void *dout, void *dq,
-                        float *qdq)
+                        float *qdq, const float *dq1)
 {
     typedef BT T;
     constexpr int LS = TileGeom<T, D>::kStride;
@@ -380,16 +392,16 @@ static int launch_dq128(hipStream_t st, int B, Segments sg, int H, int reverse, 
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 8);
     hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, dhT, (const T *)dout,
-                       (std::conditional_t<WIDE, float, T> *)dq, qdq, sg, H, reverse, hdt);
+                       (std::conditional_t<WIDE == 1, float, T> *)dq, qdq, dq1, sg, H, reverse, hdt);
     return launch_status();
 }
 
 int launch_recurrent_stream_dq128(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0,
                                   const float *g, const void *v, const void *k, const void *q, const void *dhT,
-                                  const void *dout, void *dq, float *qdq, int wide)
+                                  const void *dout, void *dq, float *qdq, int wide, const float *dq1)
 {
-    return wide ? launch_dq128<64, 128, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq)
-                : launch_dq128<64, 128, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq);
+    auto run = wide == 2 ? launch_dq128<64, 128, 2> : wide ? launch_dq128<64, 128, 1> : launch_dq128<64, 128, 0>;
+    return run(st, B, sg, H, reverse, hdt, h0, g, v, k, q, dhT, dout, dq, qdq, dq1);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -399,15 +411,15 @@ int launch_recurrent_stream_dq128(hipStream_t st, int B, Segments sg, int H, int
 // per block.  So K~ never leaves the wave's registers, and a block has two barriers.  Both waves of a sub-block read its value
 // rows from memory (the second time from cache), which no other wave needs.
 // ---------------------------------------------------------------------------------------------------
-template <int C, int D, bool WIDE>
+template <int C, int D, int WIDE>
 __global__ __launch_bounds__(C * 8) void recurrent_stream_rev128_kernel(
     const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k, const BT *__restrict__ q,
     const void *__restrict__ dhT, const BT *__restrict__ dout, void *__restrict__ dh0, float *__restrict__ dg,
-    std::conditional_t<WIDE, float, BT> *__restrict__ dv, std::conditional_t<WIDE, float, BT> *__restrict__ dk, Segments sg,
-    int H, int reverse, int hdt)
+    std::conditional_t<WIDE == 1, float, BT> *__restrict__ dv, std::conditional_t<WIDE == 1, float, BT> *__restrict__ dk,
+    const float *__restrict__ dv1, const float *__restrict__ dk1, float *__restrict__ dg1, Segments sg, int H, int reverse, int hdt)
 {
     typedef BT T;
-    typedef std::conditional_t<WIDE, float, BT> TG;
+    typedef std::conditional_t<WIDE == 1, float, BT> TG;
     constexpr int NB = C / 16, NW = 2 * NB, KS = D / 32, NT = D / 16;
     constexpr int DH = D / 2, KH = DH / 32;                          // a wave's features, in slices of 32
     constexpr int RT = NT / NB, NTW = NT / 2;                        // its state tiles: RT key tiles x NTW value tiles
@@ -439,6 +451,13 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev128_kernel(
     const int h = blockIdx.x;
     const int64_t seq = (seg.row0 * H + h) * D;
     const int64_t rowstride = (int64_t)H * D;
+    if constexpr (WIDE == 2) {           // (see sweep 1; the gates' gradient is added to dg1, `dg` holds sweep 1's q*dq of this pass)
+        const int other = ((h ^ 1) - h) * D;
+        v += other;
+        dout += other;
+        dv += other;
+        dv1 += other;
+    }
     const int64_t bh = (int64_t)seg.index * H + h;
     TrLane<T> L = make_tr_lane<T>(LS);
     const TrLane<T> Lx = make_tr_lane<T>(XS);
@@ -756,6 +775,11 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev128_kernel(
                 // q*dq - k*dk of the row, then its reverse running sum inside the sub-block
                 qdq[ks].v[e] = suffix_sum_rows((valid ? qdq[ks].v[e] : 0.f) - kk[e] * o[e]);
             }
+            if constexpr (WIDE == 2) {
+                const f32x8 t = ld8(dk1 + row + 32 * ks);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] += t.v[e];
+            }
             if (valid) st8(dk + row + 32 * ks, pack8<TG>(o));
             if (r == 0) st8(dltab + J0 * D + f + c8, qdq[ks]);
         }
@@ -829,6 +853,11 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev128_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[4 * tt + e] = own[2 * ks + tt][e] + t[e];
             }
+            if constexpr (WIDE == 2) {
+                const f32x8 t = ld8(dv1 + row + 32 * ks);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] += t.v[e];
+            }
             if (valid) st8(dv + row + 32 * ks, pack8<TG>(o));
             f32x8 tot = ld8(runtab + (n & 1) * D + f);
 #pragma unroll
@@ -843,7 +872,14 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev128_kernel(
                 }
             }
             if (J0 == 0 && r == 0) st8(runtab + ((n & 1) ^ 1) * D + f, tot);
-            if (valid) st8(dg + row + 32 * ks, qdq[ks]);
+            if constexpr (WIDE == 2) {
+                const f32x8 t = ld8(dg1 + row + 32 * ks);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qdq[ks].v[e] += t.v[e];
+                if (valid) st8(dg1 + row + 32 * ks, qdq[ks]);
+            } else if (valid) {
+                st8(dg + row + 32 * ks, qdq[ks]);
+            }
         }
         publish();
     }
@@ -858,13 +894,13 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev128_kernel(
         }
 }
 
-template <int C, int D, bool WIDE>
+template <int C, int D, int WIDE>
 static int launch_rev128(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const float *g, const void *v,
                          const void *k, const void *q, const void *dhT, const void *dout, void *dh0, float *dg, void *dv,
-                         void *dk)
+                         void *dk, const float *dv1, const float *dk1, float *dg1)
 {
     typedef BT T;
-    typedef std::conditional_t<WIDE, float, T> TG;
+    typedef std::conditional_t<WIDE == 1, float, T> TG;
     constexpr int LS = TileGeom<T, D>::kStride, NB = C / 16;
     const size_t lds = (size_t)(3 * C + 2 * D) * LS * sizeof(T) + (size_t)2 * NB * (D / 32) * 64 * sizeof(f32x4) +
                        (size_t)(2 * NB + 2) * D * sizeof(float);
@@ -873,16 +909,17 @@ static int launch_rev128(hipStream_t st, int B, Segments sg, int H, int reverse,
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 8);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q, dhT, (const T *)dout, dh0, dg,
-                       (TG *)dv, (TG *)dk, sg, H, reverse, hdt);
+                       (TG *)dv, (TG *)dk, dv1, dk1, dg1, sg, H, reverse, hdt);
     return launch_status();
 }
 
 int launch_recurrent_stream_rev128(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const float *g,
                                    const void *v, const void *k, const void *q, const void *dhT, const void *dout, void *dh0,
-                                   float *dg, void *dv, void *dk, int wide)
+                                   float *dg, void *dv, void *dk, int wide, const float *dv1,
+                                   const float *dk1, float *dg1)
 {
-    return wide ? launch_rev128<64, 128, true>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk)
-                : launch_rev128<64, 128, false>(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk);
+    auto run = wide == 2 ? launch_rev128<64, 128, 2> : wide ? launch_rev128<64, 128, 1> : launch_rev128<64, 128, 0>;
+    return run(st, B, sg, H, reverse, hdt, g, v, k, q, dhT, dout, dh0, dg, dv, dk, dv1, dk1, dg1);
 }
 
 }  // namespace gla

@@ -16,11 +16,13 @@
 
 namespace gla {
 
-template <typename TO, int C, int D>
+// SECOND: the second pass of head dimension 256 (gla_split.hip): head h takes the value rows of head h ^ 1, and `out1`, what the
+// first pass left there in fp32, is added before the one rounding.
+template <typename TO, int C, int D, bool SECOND>
 __global__ __launch_bounds__(C * 8) void recurrent_stream_fwd2_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const __bf16 *__restrict__ v,
     const __bf16 *__restrict__ k, const __bf16 *__restrict__ q, void *__restrict__ hT,
-    TO *__restrict__ out, Segments sg, int H, int reverse, int hdt)
+    TO *__restrict__ out, const float *__restrict__ out1, Segments sg, int H, int reverse, int hdt)
 {
     typedef __bf16 T;
     constexpr int NB = C / 16, NW = 2 * NB, KS = D / 32, NT = D / 16;
@@ -49,6 +51,12 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_fwd2_kernel(
     const int h = blockIdx.x;
     const int64_t seq = (seg.row0 * H + h) * D;      // element offset of (b, t = 0, h)
     const int64_t rowstride = (int64_t)H * D;
+    if constexpr (SECOND) {
+        const int other = ((h ^ 1) - h) * D;
+        v += other;
+        out += other;
+        out1 += other;
+    }
     const int64_t bh = (int64_t)seg.index * H + h;
     const TrLane<T> L = make_tr_lane<T>(LS);
     const int ptl = plain_tr_lane<T>(LS);
@@ -232,6 +240,11 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_fwd2_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[4 * tt + e] = own[ks][tt][e] + other[e];
             }
+            if constexpr (SECOND) {
+                const f32x8 t = ld8(out1 + row + 32 * ks + 8 * c);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] += t.v[e];
+            }
             if (valid) st8(out + row + 32 * ks + 8 * c, pack8<TO>(o));
         }
         publish_state();
@@ -247,25 +260,34 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_fwd2_kernel(
         }
 }
 
-template <typename TO>
-int launch_recurrent_stream_fwd2(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0,
-                                 const float *g, const void *v, const void *k, const void *q, void *hT, void *out)
+template <typename TO, bool SECOND>
+static int launch_fwd2(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
+                       const void *v, const void *k, const void *q, void *hT, void *out, const float *out1)
 {
     typedef __bf16 T;
     constexpr int C = 64, D = 128, LS = TileGeom<T, D>::kStride;
     const size_t lds = (size_t)(3 * C + 2 * D) * LS * sizeof(T) + (size_t)(C / 16) * D * sizeof(float) +
                        (size_t)(C / 8) * (D / 32) * 64 * sizeof(f32x4);
-    auto kern = recurrent_stream_fwd2_kernel<TO, C, D>;
+    auto kern = recurrent_stream_fwd2_kernel<TO, C, D, SECOND>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 8);
-    hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, hT, (TO *)out, sg, H,
+    hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, hT, (TO *)out, out1, sg, H,
                        reverse, hdt);
     return launch_status();
 }
+
+template <typename TO>
+int launch_recurrent_stream_fwd2(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0,
+                                 const float *g, const void *v, const void *k, const void *q, void *hT, void *out,
+                                 const float *out1)
+{
+    return out1 ? launch_fwd2<TO, true>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, out, out1)
+                : launch_fwd2<TO, false>(st, B, sg, H, reverse, hdt, h0, g, v, k, q, hT, out, nullptr);
+}
 template int launch_recurrent_stream_fwd2<__bf16>(hipStream_t, int, Segments, int, int, int, const void *, const float *,
-                                                  const void *, const void *, const void *, void *, void *);
+                                                  const void *, const void *, const void *, void *, void *, const float *);
 template int launch_recurrent_stream_fwd2<float>(hipStream_t, int, Segments, int, int, int, const void *, const float *,
-                                                 const void *, const void *, const void *, void *, void *);
+                                                 const void *, const void *, const void *, void *, void *, const float *);
 
 }  // namespace gla

@@ -7,10 +7,11 @@
 // A [B,T,H,256] array read as [B,T,2H,128] has the halves of head h as heads 2h and 2h+1, so the two problems
 // with a == b are ONE run of the 128-feature kernels on the arrays as they lie, and the two with a != b are a
 // second run on q, k, g as they lie and the value-side arrays with the halves of every row exchanged.  For bf16 data the
-// first run of chunk_gla leaves out, dq, dk and dv in fp32, and the second takes the other half's rows where they lie and adds
-// what the first left, rounding once, as one kernel over all 256 features would (WIDE in gla_chunk_fwd.hip and
-// gla_chunk_bwd.hip).  This file holds the small kernels around the runs: exchanging halves and adding the two runs' results
-// (fp32 data and recurrent_gla), and cutting the [256,256] states into their four [128,128] blocks and back.
+// first run leaves out, dq, dk and dv in fp32, and the second takes the other half's rows where they lie and adds what the
+// first left, rounding once, as one kernel over all 256 features would (WIDE in gla_chunk_fwd.hip, gla_chunk_bwd.hip and
+// gla_recurrent_stream_bwd128.hip, SECOND in gla_recurrent_stream_fwd2.hip).  This file holds the small kernels around the
+// runs: exchanging halves and adding the two runs' results (fp32 data, recurrent_gla with an fp32 dout or few steps), and
+// cutting the [256,256] states into their four [128,128] blocks and back.
 #include "gla_split.hpp"
 
 namespace gla {
