@@ -41,8 +41,8 @@ __global__ __launch_bounds__(C * 4) void chunk_grad_kernel(
     const T *__restrict__ q, const T *__restrict__ dout, const T *__restrict__ statesN,
     const T *__restrict__ dstatesT, const T *__restrict__ dstatesN, float *__restrict__ dg,
     std::conditional_t<WIDE == 1, float, T> *__restrict__ dv, std::conditional_t<WIDE == 1, float, T> *__restrict__ dk,
-    std::conditional_t<WIDE == 1, float, T> *__restrict__ dq, const float *__restrict__ dv1,
-    const float *__restrict__ dk1, const float *__restrict__ dq1, int T_len, int H)
+    std::conditional_t<WIDE == 1, float, T> *__restrict__ dq, int T_len, int H,
+    const float *__restrict__ dv1, const float *__restrict__ dk1, const float *__restrict__ dq1)
 {
     typedef std::conditional_t<WIDE == 1, float, T> TG;      // element type of dv, dk, dq
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4;
@@ -726,7 +726,7 @@ int launch_chunk_grad(hipStream_t st, int B, int T_len, int H, const float *g, c
     dim3 grid((T_len + C - 1) / C * H, B), block(C * 4);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q,
                        (const T *)dout, (const T *)statesN, (const T *)dstatesT, (const T *)dstatesN, dg,
-                       (TG *)dv, (TG *)dk, (TG *)dq, dv1, dk1, dq1, T_len, H);
+                       (TG *)dv, (TG *)dk, (TG *)dq, T_len, H, dv1, dk1, dq1);
     return launch_status();
 }
 

@@ -25,7 +25,7 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_dq128_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k,
     const BT *__restrict__ q, const void *__restrict__ dhT, const BT *__restrict__ dout,
     std::conditional_t<WIDE == 1, float, BT> *__restrict__ dq, float *__restrict__ qdq,
-    const float *__restrict__ dq1, Segments sg, int H, int reverse, int hdt)
+    Segments sg, int H, int reverse, int hdt, const float *__restrict__ dq1)
 {
     typedef BT T;
     typedef std::conditional_t<WIDE == 1, float, BT> TG;
@@ -392,7 +392,7 @@ static int launch_dq128(hipStream_t st, int B, Segments sg, int H, int reverse, 
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 8);
     hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, dhT, (const T *)dout,
-                       (std::conditional_t<WIDE == 1, float, T> *)dq, qdq, dq1, sg, H, reverse, hdt);
+                       (std::conditional_t<WIDE == 1, float, T> *)dq, qdq, sg, H, reverse, hdt, dq1);
     return launch_status();
 }
 
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_rev128_kernel(
     const float *__restrict__ g, const BT *__restrict__ v, const BT *__restrict__ k, const BT *__restrict__ q,
     const void *__restrict__ dhT, const BT *__restrict__ dout, void *__restrict__ dh0, float *__restrict__ dg,
     std::conditional_t<WIDE == 1, float, BT> *__restrict__ dv, std::conditional_t<WIDE == 1, float, BT> *__restrict__ dk,
-    const float *__restrict__ dv1, const float *__restrict__ dk1, float *__restrict__ dg1, Segments sg, int H, int reverse, int hdt)
+    Segments sg, int H, int reverse, int hdt, const float *__restrict__ dv1, const float *__restrict__ dk1, float *__restrict__ dg1)
 {
     typedef BT T;
     typedef std::conditional_t<WIDE == 1, float, BT> TG;
@@ -909,7 +909,7 @@ static int launch_rev128(hipStream_t st, int B, Segments sg, int H, int reverse,
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 8);
     hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)v, (const T *)k, (const T *)q, dhT, (const T *)dout, dh0, dg,
-                       (TG *)dv, (TG *)dk, dv1, dk1, dg1, sg, H, reverse, hdt);
+                       (TG *)dv, (TG *)dk, sg, H, reverse, hdt, dv1, dk1, dg1);
     return launch_status();
 }
 

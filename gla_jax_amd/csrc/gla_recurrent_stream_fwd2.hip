@@ -22,7 +22,7 @@ template <typename TO, int C, int D, bool SECOND>
 __global__ __launch_bounds__(C * 8) void recurrent_stream_fwd2_kernel(
     const void *__restrict__ h0, const float *__restrict__ g, const __bf16 *__restrict__ v,
     const __bf16 *__restrict__ k, const __bf16 *__restrict__ q, void *__restrict__ hT,
-    TO *__restrict__ out, const float *__restrict__ out1, Segments sg, int H, int reverse, int hdt)
+    TO *__restrict__ out, Segments sg, int H, int reverse, int hdt, const float *__restrict__ out1)
 {
     typedef __bf16 T;
     constexpr int NB = C / 16, NW = 2 * NB, KS = D / 32, NT = D / 16;
@@ -272,8 +272,8 @@ static int launch_fwd2(hipStream_t st, int B, Segments sg, int H, int reverse, i
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 8);
-    hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, hT, (TO *)out, out1, sg, H,
-                       reverse, hdt);
+    hipLaunchKernelGGL(kern, grid, block, lds, st, h0, g, (const T *)v, (const T *)k, (const T *)q, hT, (TO *)out, sg, H,
+                       reverse, hdt, out1);
     return launch_status();
 }
 
