@@ -19,7 +19,7 @@ namespace gla {
 // SECOND: the second pass of head dimension 256 (gla_split.hip): head h takes the value rows of head h ^ 1, and `out1`, what the
 // first pass left there in fp32, is added before the one rounding.
 template <typename TO, int C, int D, bool SECOND>
-__global__ __launch_bounds__(C * 8) void recurrent_stream_fwd2_kernel(
+__device__ __forceinline__ void recurrent_fwd2(
     const void *__restrict__ h0, const float *__restrict__ g, const __bf16 *__restrict__ v,
     const __bf16 *__restrict__ k, const __bf16 *__restrict__ q, void *__restrict__ hT,
     TO *__restrict__ out, Segments sg, int H, int reverse, int hdt, const float *__restrict__ out1)
@@ -260,6 +260,25 @@ __global__ __launch_bounds__(C * 8) void recurrent_stream_fwd2_kernel(
         }
 }
 
+namespace two_waves {
+template <typename TO, int C, int D>
+__global__ __launch_bounds__(C * 8) void recurrent_stream_fwd_kernel(
+    const void *__restrict__ h0, const float *__restrict__ g, const __bf16 *__restrict__ v, const __bf16 *__restrict__ k,
+    const __bf16 *__restrict__ q, void *__restrict__ hT, TO *__restrict__ out, Segments sg, int H, int reverse, int hdt,
+    const float *__restrict__)
+{
+    recurrent_fwd2<TO, C, D, false>(h0, g, v, k, q, hT, out, sg, H, reverse, hdt, nullptr);
+}
+template <typename TO, int C, int D>
+__global__ __launch_bounds__(C * 8) void recurrent_stream_second_kernel(
+    const void *__restrict__ h0, const float *__restrict__ g, const __bf16 *__restrict__ v, const __bf16 *__restrict__ k,
+    const __bf16 *__restrict__ q, void *__restrict__ hT, TO *__restrict__ out, Segments sg, int H, int reverse, int hdt,
+    const float *__restrict__ out1)
+{
+    recurrent_fwd2<TO, C, D, true>(h0, g, v, k, q, hT, out, sg, H, reverse, hdt, out1);
+}
+}  // namespace two_waves
+
 template <typename TO, bool SECOND>
 static int launch_fwd2(hipStream_t st, int B, Segments sg, int H, int reverse, int hdt, const void *h0, const float *g,
                        const void *v, const void *k, const void *q, void *hT, void *out, const float *out1)
@@ -268,7 +287,7 @@ static int launch_fwd2(hipStream_t st, int B, Segments sg, int H, int reverse, i
     constexpr int C = 64, D = 128, LS = TileGeom<T, D>::kStride;
     const size_t lds = (size_t)(3 * C + 2 * D) * LS * sizeof(T) + (size_t)(C / 16) * D * sizeof(float) +
                        (size_t)(C / 8) * (D / 32) * 64 * sizeof(f32x4);
-    auto kern = recurrent_stream_fwd2_kernel<TO, C, D, SECOND>;
+    auto kern = SECOND ? two_waves::recurrent_stream_second_kernel<TO, C, D> : two_waves::recurrent_stream_fwd_kernel<TO, C, D>;
     static LdsGrant grant;
     if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
     dim3 grid(H, sg.S, B), block(C * 8);
