@@ -206,8 +206,10 @@ template <int D, int DM> __device__ __forceinline__ void add_row_once(float (&o)
 // other token alone), and stores its results to a row that nobody reads.  Both are a scalar choice between two base
 // pointers: the kernels' instructions stay as they are (with the stores under a branch the gradient kernel lost 1 to 2 %
 // at full tiles, the branch being a wall to the scheduler).
-// (as aligned as the rows that they stand for: the kernels access them 16 bytes at a time)
-static __device__ __align__(16) float zero_row[128], spare_row[128];
+// Every such wave of a launch reads the one row and stores to the other, so each has whole 128-byte lines of its own.  Aligned to
+// 16 bytes only, wherever the linker put them, their pieces straddled lines and the two shared one (bf16, forward, us:
+// B32 T160 H16 D64 67 against 35, B32 T160 H16 D128 140 against 92, B8 T2080 H16 D64 121 against 77).
+static __device__ __align__(512) float zero_row[128], spare_row[128];
 template <typename P> __device__ __forceinline__ const P *rows_or_zeros(bool live, const P *rows)
 {
     return live ? rows : reinterpret_cast<const P *>(zero_row);

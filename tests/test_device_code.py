@@ -53,16 +53,22 @@ def test_the_scan_sees_a_mixed_sum():
 
 
 @pytest.fixture(scope="module")
-def listings(tmp_path_factory):
-    """The disassembly of the built library, one text per code object."""
+def objects(tmp_path_factory):
+    """The code objects of the built library."""
     _lib.load()
     if not os.path.exists(OBJDUMP):
         pytest.skip("needs ROCm's llvm-objdump")
     tmp_path = tmp_path_factory.mktemp("code")
     lib = shutil.copy(_lib.LIB_PATH, tmp_path / "lib.so")
     subprocess.run([OBJDUMP, "--offloading", str(lib)], cwd=tmp_path, check=True, capture_output=True)
-    objects = glob.glob(str(tmp_path / "*gfx950"))
-    assert objects
+    found = glob.glob(str(tmp_path / "*gfx950"))
+    assert found
+    return found
+
+
+@pytest.fixture(scope="module")
+def listings(objects):
+    """Their disassembly, one text each."""
     return [subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", o], check=True, capture_output=True, text=True).stdout for o in objects]
 
 
@@ -93,3 +99,17 @@ def test_recurrent_forward_moves_its_state_in_wide_accesses(listings):
     assert kernels == 6
     # (one gate sum per feature and sequence, in the two forms that leave nothing but states)
     assert [op for _, op in found] == ["global_store_dword"] * 2, found
+
+
+def test_shared_rows_of_empty_waves_lie_in_lines_of_their_own(objects):
+    """Waves past the end of a sequence all read one row of zeros and store to one spare row (gla_chunk_common.hpp): wherever the
+    linker puts the two, neither may share a 128-byte line with the other or with anything else."""
+    rows = []
+    for o in objects:
+        table = subprocess.run([OBJDUMP, "-t", o], check=True, capture_output=True, text=True).stdout
+        for line in table.splitlines():
+            if "zero_row" in line or "spare_row" in line:
+                address, *_, size, name = line.split()
+                rows.append((name, int(address, 16), int(size, 16)))
+    assert len(rows) >= 5 and any("spare_row" in name for name, *_ in rows)
+    assert not [row for row in rows if row[1] % 128 or row[2] % 128], rows
