@@ -380,8 +380,8 @@ static int check_recurrent(int64_t B, int64_t T, int64_t H, int64_t DK, int64_t 
 
 // ---- head dimension 256 as four problems of head dimension 128 (gla_split.hip) ---------------------------------
 // Two passes of the 128-feature kernels over 2H heads, the first one's results left in fp32 and added with one rounding by the
-// second, or, where the vector kernels run or dout is fp32, both left and added by kernels of their own (the workspace is sized
-// for that).
+// second, or, in the backward of fp32 data or of an fp32 dout, both left and added by kernels of their own (the backward's
+// workspace is sized for that, its size functions not being told the type of dout).
 // rows: one [B,T,H,256] array; hid: one [B,2H,128,128] array of states per segment (sized for fp32 states).
 namespace gla {
 struct SplitSizes {
@@ -393,8 +393,8 @@ struct SplitSizes {
     {
     }
     static size_t round_up256(size_t x) { return (x + 255) & ~(size_t)255; }
-    // forward: value rows with their halves exchanged, both passes' out, hidden_init and hidden_final in blocks
-    size_t fwd() const { return rows_e + 2 * rows_f32 + 4 * hid; }
+    // forward: the first pass's out, hidden_init and hidden_final in blocks
+    size_t fwd() const { return rows_f32 + 4 * hid; }
     // backward: value and dout rows exchanged, both passes' dq, dk, dv, the second pass's d(log_fgate), hidden_init,
     // dhidden_final and dhidden_init in blocks
     size_t bwd() const { return rows_e + rows_f32 + 7 * rows_f32 + 6 * hid; }
@@ -578,8 +578,8 @@ static int recurrent_fwd_inner(void *stream, int64_t B, gla::Segments sg, int64_
     const gla::SplitSizes z(rows, states, H, dtype);
     hipStream_t st = (hipStream_t)stream;
     unsigned char *ws = (unsigned char *)workspace;
-    unsigned char *v_sw = ws, *out1 = v_sw + z.rows_e, *out2 = out1 + z.rows_f32, *h0_same = out2 + z.rows_f32,
-                  *h0_cross = h0_same + z.hid, *hT_same = h0_cross + z.hid, *hT_cross = hT_same + z.hid;
+    unsigned char *out1 = ws, *h0_same = out1 + z.rows_f32, *h0_cross = h0_same + z.hid, *hT_same = h0_cross + z.hid,
+                  *hT_cross = hT_same + z.hid;
     int e = 0;
     if (hidden_init) {      // (a lean pass may start from zeros: no initial state given)
         e = gla::launch_hidden_blocks(st, hidden_dtype, states * H, const_cast<void *>(hidden_init), h0_same, h0_cross, 1);
@@ -600,19 +600,9 @@ static int recurrent_fwd_inner(void *stream, int64_t B, gla::Segments sg, int64_
     e = recurrent_fwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_same, log_fgate,
                           value, key, query, hT_same, out1);
     if (e) return e;
-    if (sg.L > gla::kFewSteps) {
-        auto run = out_dtype == GLA_F32 ? gla::launch_recurrent_stream_fwd2<float> : gla::launch_recurrent_stream_fwd2<__bf16>;
-        e = run(st, B, sg, 2 * H, reverse, hidden_dtype, h0_cross, log_fgate, value, key, query, hT_cross, out, (const float *)out1);
-        if (e) return e;
-    } else {        // the vector kernels: a copy with the halves of every row exchanged, and the sum behind
-        e = gla::launch_swap_halves(st, dtype, rows * H, v_sw, value);
-        if (e) return e;
-        e = recurrent_fwd_run(stream, B, sg, 2 * H, 128, 128, dtype, hidden_dtype, GLA_F32, reverse, h0_cross, log_fgate, v_sw,
-                              key, query, hT_cross, out2);
-        if (e) return e;
-        e = gla::launch_sum_rows(st, out_dtype, rows * H, out, (const float *)out1, (const float *)out2, 1);
-        if (e) return e;
-    }
+    auto run = out_dtype == GLA_F32 ? gla::launch_recurrent_stream_fwd2<float> : gla::launch_recurrent_stream_fwd2<__bf16>;
+    e = run(st, B, sg, 2 * H, reverse, hidden_dtype, h0_cross, log_fgate, value, key, query, hT_cross, out, (const float *)out1);
+    if (e) return e;
     return gla::launch_hidden_blocks(st, hidden_dtype, states * H, hidden_final, hT_same, hT_cross, 0);
 }
 

@@ -85,7 +85,7 @@ def test_chunk_plan_and_sizes():
     assert sub + 16 * rows + hid <= lib.gla_chunk_bwd_workspace_bytes(B, T, H, 256, 256, 128, _lib.GLA_BF16) <= (
         sub + 16 * rows + hid + 12 * 256)
     assert lib.gla_chunk_states_bytes(B, T, H, 512, 512, 128, _lib.GLA_BF16) == 0
-    # recurrent_gla: a workspace at head dimension 256 (both passes' results in fp32 and the exchanged rows) and, at
+    # recurrent_gla: a workspace at head dimension 256 (the first pass's results in fp32) and, at
     # every head dimension, where the sequences are few enough to run as S >= 4 segments of >= 128 steps side by
     # side (B*H*S <= 256 workgroups; S = 2 already for bf16 data at head dimensions 64 and more): the segments'
     # states in fp32, twice (backward: four times), and their gate sums
@@ -252,3 +252,14 @@ def test_canonical_arrays_pass_through_untouched():
     # every Function has a twin in the older style that shares its forward, context and backward
     for cls in (gla._ChunkGLA, gla._ChunkGLABwd, gla._RecurrentGLA, gla._RecurrentGLABwd):
         assert issubclass(cls._twin, torch.autograd.Function) and cls._twin.backward is cls.backward
+
+
+def test_recurrent_workspace_at_256_features():
+    """The forward on bf16 data keeps the first pass's `out` in fp32 and the states cut into blocks; the second pass reads the value
+    rows where they lie."""
+    lib = _lib.load()
+    r256 = lambda x: (x + 255) & ~255
+    for B, T, H in ((64, 65, 1), (8, 300, 16)):               # too many sequences for segments
+        rows, states = r256(B * T * H * 256 * 4), r256(B * 2 * H * 128 * 128 * 4)
+        assert lib.gla_recurrent_fwd_workspace_bytes(B, T, H, 256, 256, _lib.GLA_BF16) == rows + 4 * states
+    assert lib.gla_recurrent_fwd_workspace_bytes(64, 64, 1, 256, 256, _lib.GLA_BF16) == 256       # few steps: no passes
