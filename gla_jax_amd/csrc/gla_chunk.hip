@@ -295,16 +295,9 @@ static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         typedef decltype(t) E;
         constexpr int C_ = decltype(c)::value, D_ = decltype(d)::value, DM_ = decltype(dm)::value;
         int e = 0;
-        if ((stages & 1) && wide != 2)
+        if (stages & 1)
             e = launch_chunk_outer<E, C_, D_, DM_>(st, 0, (int)B, (int)T, (int)H, log_fgate, value, key, prodT, decay,
-                                                   pexp);
-        if ((stages & 1) && wide == 2) {
-            if constexpr (sizeof(E) == 2 && D_ == 128 && DM_ == 128)
-                e = launch_chunk_outer<E, C_, D_, DM_, true>(st, 0, (int)B, (int)T, (int)H, log_fgate, value, key, prodT,
-                                                             decay, pexp);
-            else
-                e = GLA_ERR_UNSUPPORTED;
-        }
+                                                   pexp, wide == 2);
         if (e) return e;
         if (stages & 2)
             e = launch_chunk_scan<E, D_, DM_>(st, (int)(B * H), N, 0, hidden_dtype, hidden_init, prodT, decay, pexp,
@@ -448,16 +441,9 @@ static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         typedef decltype(t) E;
         constexpr int C_ = decltype(c)::value, D_ = decltype(d)::value, DM_ = decltype(dm)::value;
         int e = 0;
-        if ((stages & 1) && wide != 2)
+        if (stages & 1)
             e = launch_chunk_outer<E, C_, D_, DM_>(st, 1, (int)B, (int)T, (int)H, log_fgate, dout, query, prodT, decay,
-                                                   pexp);
-        if ((stages & 1) && wide == 2) {
-            if constexpr (sizeof(E) == 2 && D_ == 128 && DM_ == 128)
-                e = launch_chunk_outer<E, C_, D_, DM_, true>(st, 1, (int)B, (int)T, (int)H, log_fgate, dout, query, prodT,
-                                                             decay, pexp);
-            else
-                e = GLA_ERR_UNSUPPORTED;
-        }
+                                                   pexp, wide == 2);
         if (e) return e;
         if (stages & 2)
             e = launch_chunk_scan<E, D_, DM_>(st, (int)(B * H), N, 1, hidden_dtype, dhidden_final, prodT, decay, pexp,

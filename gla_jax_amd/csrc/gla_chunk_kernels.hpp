@@ -35,11 +35,11 @@ namespace gla {
     M(float, 64, 128, 128)           \
     M(float, 32, 128, 128)
 
-// OTHER (built for bf16 at D = 128 only): head h takes the rows of x of head h ^ 1 (the second pass of head dimension 256)
-template <typename T, int C, int D, int DM, bool OTHER = false>
+template <typename T, int C, int D, int DM>
 // prodT: the per-chunk products in the library's own layout and type (gla_chunk_state.hip), pexp: their exponents
+// other_half != 0: head h takes the rows of x of head h ^ 1 (the second pass of head dimension 256)
 int launch_chunk_outer(hipStream_t st, int mode, int B, int T_len, int H, const float *g, const void *x,
-                       const void *y, void *prodT, float *decay, unsigned char *pexp);
+                       const void *y, void *prodT, float *decay, unsigned char *pexp, int other_half);
 
 template <typename T, int D, int DM>
 // hdt = gla_dtype of hin / hout (hidden_init and hidden_final, or their cotangents)

@@ -40,15 +40,13 @@ constexpr int kProdNotFinite = 255;      // the exponent byte of a group with a 
 
 // Two tiles and a table fit twice into a CU's LDS; the register budget is held to what lets two
 // workgroups share a CU, so that one loads while the other computes.
-// OTHER: head h takes the rows of x of head h ^ 1 (the second pass of head dimension 256, built for bf16 at D = 128 only).  As an
-// argument it was 15 instructions of every call, two of them ahead of the first loads.
-template <typename T, int C, int D, int DM, int MODE, bool OTHER>
+template <typename T, int C, int D, int DM, int MODE>
 __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C < 128 && D < 128 ? 8 : C / 32))) void chunk_outer_kernel(const float *__restrict__ g,
                                                             const T *__restrict__ x,
                                                             const T *__restrict__ y,
                                                             typename Prod<T>::type *__restrict__ prodT,
                                                             float *__restrict__ decay,
-                                                            unsigned char *__restrict__ pexp, int T_len, int H)
+                                                            unsigned char *__restrict__ pexp, int T_len, int H, int other_half)
 {
     constexpr int NB = C / 16, KS = D / 32, NV = D / 4, NT = D / 16;
     constexpr int LS = TileGeom<T, D>::kStride;
@@ -68,7 +66,7 @@ __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C
     const int64_t tok = (int64_t)b * T_len + (int64_t)n * C + 16 * w + r;
     const int64_t rowoff = live ? (tok * H + h) * DM : 0;     // DM features per row in memory (DM < D: see RowMap)
     g = rows_or_zeros(live, g);
-    x = rows_or_zeros(live, OTHER ? x + ((h ^ 1) - h) * DM : x);
+    x = rows_or_zeros(live, x + ((h ^ other_half) - h) * DM);
     y = rows_or_zeros(live, y);
 
     float p[NV];
@@ -324,26 +322,26 @@ __global__ __launch_bounds__(64) void chunk_scan_kernel(const void *__restrict__
     if (in_mem) store_hidden<4>(hout, hdt, (int64_t)bh * DM * DM + dk * DM + dv0, X);
 }
 
-template <typename T, int C, int D, int DM, bool OTHER>
+template <typename T, int C, int D, int DM>
 int launch_chunk_outer(hipStream_t st, int mode, int B, int T_len, int H, const float *g, const void *x,
-                       const void *y, void *prodT, float *decay, unsigned char *pexp)
+                       const void *y, void *prodT, float *decay, unsigned char *pexp, int other_half)
 {
     typedef typename Prod<T>::type P;
     constexpr int LS = TileGeom<T, D>::kStride;
     const size_t lds = (size_t)2 * C * LS * sizeof(T) + (size_t)(C / 16) * D * sizeof(float);
     dim3 grid((T_len + C - 1) / C * H, B), block(C * 4);
     if (mode == 0) {
-        auto kern = chunk_outer_kernel<T, C, D, DM, 0, OTHER>;
+        auto kern = chunk_outer_kernel<T, C, D, DM, 0>;
         static LdsGrant grant;
         if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
         hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)x, (const T *)y, (P *)prodT, decay, pexp, T_len,
-                           H);
+                           H, other_half);
     } else {
-        auto kern = chunk_outer_kernel<T, C, D, DM, 1, OTHER>;
+        auto kern = chunk_outer_kernel<T, C, D, DM, 1>;
         static LdsGrant grant;
         if (int e = allow_lds(grant, (const void *)kern, lds)) return e;
         hipLaunchKernelGGL(kern, grid, block, lds, st, g, (const T *)x, (const T *)y, (P *)prodT, decay, pexp, T_len,
-                           H);
+                           H, other_half);
     }
     return launch_status();
 }
@@ -366,17 +364,13 @@ int launch_chunk_scan(hipStream_t st, int BH, int N, int reverse, int hdt, const
     return launch_status();
 }
 
-#define GLA_INST_OUTER_AS(T, C, D, DM, OTHER)                                                         \
-    template int launch_chunk_outer<T, C, D, DM, OTHER>(hipStream_t, int, int, int, int, const float *, const void *, \
-                                                        const void *, void *, float *, unsigned char *);
-#define GLA_INST_OUTER(T, C, D, DM) GLA_INST_OUTER_AS(T, C, D, DM, false)
+#define GLA_INST_OUTER(T, C, D, DM)                                                                   \
+    template int launch_chunk_outer<T, C, D, DM>(hipStream_t, int, int, int, int, const float *, const void *, \
+                                                 const void *, void *, float *, unsigned char *, int);
 #define GLA_INST_SCAN(T, D, DM)                                                                       \
     template int launch_chunk_scan<T, D, DM>(hipStream_t, int, int, int, int, const void *, const void *, \
                                              const float *, const unsigned char *, void *, void *, void *, int, int);
 GLA_FOR_EACH_CHUNK_CONFIG(GLA_INST_OUTER)
-GLA_INST_OUTER_AS(__bf16, 128, 128, 128, true)
-GLA_INST_OUTER_AS(__bf16, 64, 128, 128, true)
-GLA_INST_OUTER_AS(__bf16, 32, 128, 128, true)
 GLA_INST_SCAN(__bf16, 32, 16)
 GLA_INST_SCAN(__bf16, 32, 32)
 GLA_INST_SCAN(__bf16, 64, 64)

@@ -115,24 +115,3 @@ def test_shared_rows_of_empty_waves_lie_in_lines_of_their_own(objects):
                 rows.append((name, int(address, 16), int(size, 16)))
     assert len(rows) >= 5 and any("spare_row" in name for name, *_ in rows)
     assert not [row for row in rows if row[1] % 128 or row[2] % 128], rows
-
-
-def test_only_the_other_halfs_pass_pays_for_the_other_half(listings):
-    """chunk_outer_kernel: the second pass of head dimension 256 takes the rows of the neighbouring head; what that costs ahead of
-    the first load is in a form of its own, and in no other."""
-    ahead = {}
-    for listing in listings:
-        kernel = ""
-        for line in listing.splitlines():
-            if line.endswith(">:"):
-                kernel = line.split("<")[1].split(">")[0]
-                kernel = kernel if "chunk_outer_kernel" in kernel else ""
-                count = 0
-            elif kernel and line.split():
-                count += 1
-                if line.split()[0].startswith(("global_load", "buffer_load")):
-                    ahead[kernel], kernel = count, ""
-    other = [k for k in ahead if "Lb1E" in k]
-    assert len(other) == 6                                    # bf16, 128 features, three tiles, forward and backward
-    for k in other:
-        assert ahead[k.replace("Lb1E", "Lb0E")] < ahead[k], k
