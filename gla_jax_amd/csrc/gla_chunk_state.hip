@@ -40,6 +40,10 @@ constexpr int kProdNotFinite = 255;      // the exponent byte of a group with a 
 
 // Two tiles and a table fit twice into a CU's LDS; the register budget is held to what lets two
 // workgroups share a CU, so that one loads while the other computes.
+// other_half != 0: head h takes the rows of x of head h ^ 1 (the second pass of head dimension 256).  An argument that every call
+// has, 15 instructions of it; as a form of its own it left the others no faster where they are short (B1 T256 H4 D128 9.6 to 9.9 us
+// either way) and slower where they are long (forward + backward of B1 T32768 H8 D128 603.5 -> 606 us, forward of B1 T8192 H16 95.2
+// -> 95.5).
 template <typename T, int C, int D, int DM, int MODE>
 __global__ __launch_bounds__(C * 4) __attribute__((amdgpu_waves_per_eu(C / 32, C < 128 && D < 128 ? 8 : C / 32))) void chunk_outer_kernel(const float *__restrict__ g,
                                                             const T *__restrict__ x,
