@@ -23,10 +23,12 @@ struct ChunkPlan {
     size_t rows_f32 = 0;                      // ... of floats
     size_t hid = 0;                           // one [B,2H,128,128] array of states (sized for fp32 states)
     size_t beside = 0;                        // what lies beside a pass's own workspace: a pass is planned with it again
-    bool wide = false;                        // bf16 data: both passes leave their results in fp32, summed and rounded once
-    // forward: value rows with their halves exchanged, the second pass's out (fp32 data) or both passes' (bf16 data),
-    // hidden_init and hidden_final in blocks; backward: value and dout rows exchanged, the second pass's dq, dk, dv
-    // (or both passes'), its d(log_fgate), the states' cotangents in blocks
+    bool wide = false;                        // bf16 data: the first pass's results are fp32, the second adds them and rounds once
+    // forward: value rows with their halves exchanged, the second pass's out, hidden_init and hidden_final in blocks; backward:
+    // value and dout rows exchanged, the second pass's dq, dk, dv and d(log_fgate), the states' cotangents in blocks.
+    // bf16 data: both passes' out, dq, dk, dv.  Its second pass reads and adds in place, so the exchanged rows and the second
+    // arrays lie idle (ten of a backward's sixteen arrays of bf16 rows); they are still in the sizes that callers ask for, of
+    // which the forward's decides the tile and what the static array takes.
     size_t fwd_bytes() const { return prod + decay + states + (split ? rows + (wide ? 2 : 1) * rows_f32 + 4 * hid : 0); }
     size_t bwd_bytes() const
     {
@@ -254,8 +256,7 @@ static int chunk_fwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         if (p.wide) {
             // bf16 data: the second pass's kernels take the other half's value rows where they lie and add what the first left
             // in fp32, so that `out` is rounded once (B2 T4096 H6, with an exchanged copy
-            // and a kernel for the sum: 195 -> 166 us).  The workspace's size, which a caller asks for and which decides what the static
-            // array takes, is still the one with the copies.
+            // and a kernel for the sum: 195 -> 166 us).  The workspace is still the size with the copies, see ChunkPlan.
             e = chunk_fwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, h0_same, log_fgate, value, key,
                               query, hT_same, out1_ws, states, ws, sub, 1, p.beside);
             if (e) return e;
@@ -398,8 +399,8 @@ static int chunk_bwd_run(void *stream, int stages, int64_t B, int64_t T, int64_t
         if (e) return e;
         const unsigned char *states2 = (const unsigned char *)states + p.resid;
         if (p.wide) {
-            // as in the forward (a training step of B2 T4096 H6: 637 -> 535 us; the second pass's gradient kernel 162 against
-            // 120 us, but two copies of 12, three sums of 25 and one of 30 less)
+            // as in the forward (a training step of B2 T4096 H6: 637 -> 535 us; the second pass's gradient kernel, which reads four
+            // fp32 rows more and spills six registers, 162 against 120 us, but two copies of 12, three sums of 25 and one of 30 less)
             e = chunk_bwd_run(stream, 7, B, T, 2 * H, 128, 128, chunk_size, dtype, hidden_dtype, log_fgate, value, key, query,
                               states, dhT_same, dout, dh0_same, dlog_fgate, dv1_ws, dk1_ws, dq1_ws, ws, sub, 1, p.beside);
             if (e) return e;

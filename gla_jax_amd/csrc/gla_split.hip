@@ -10,7 +10,7 @@
 // first run leaves out, dq, dk and dv in fp32, and the second takes the other half's rows where they lie and adds what the
 // first left, rounding once, as one kernel over all 256 features would (WIDE in gla_chunk_fwd.hip, gla_chunk_bwd.hip and
 // gla_recurrent_stream_bwd128.hip, SECOND in gla_recurrent_stream_fwd2.hip).  This file holds the small kernels around the
-// runs: exchanging halves and adding the two runs' results (fp32 data, recurrent_gla with an fp32 dout or few steps), and
+// runs: exchanging halves and adding the two runs' results (fp32 data, and the backward of recurrent_gla with an fp32 dout), and
 // cutting the [256,256] states into their four [128,128] blocks and back.
 #include "gla_split.hpp"
 
