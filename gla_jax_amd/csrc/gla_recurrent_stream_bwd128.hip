@@ -8,7 +8,8 @@
 //
 // B4 T4096 H16 D128 (256 workgroups of 1024 steps): sweep 1 225 -> 152 us, 652 MB by counter (its rows are 604) at 4.3 TB/s, against
 // 4.9 of a large copy; sweep 2 320 -> 244 us, 984 MB by counter at 4.1 TB/s: its rows and states are 839, the rest the value rows that
-// both waves read and spilled registers, about ten a lane and block.  With one wave per sub-block it was one wave per SIMD with more than 400 registers.
+// both waves read and spilled registers, about ten a lane and block.  With one wave per sub-block it was one wave per SIMD with more than
+// 400 registers.
 // What sweep 2 waits for is the sum of its parts: a 64-step block is 32 000 cycles, of them (counted) 12 000 of vector arithmetic, 6 000
 // of matrix instructions and 9 000 of LDS traffic per SIMD or CU, which two waves between two barriers overlap little.
 #include "gla_recurrent_stream_bwd.hpp"
